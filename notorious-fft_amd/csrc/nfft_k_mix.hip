@@ -1,0 +1,265 @@
+// nfft_k_mix.hip -- schedules and launchers of the one-pass mixed-radix lines.
+#include "nfft_internal.h"
+
+#include <algorithm>
+#include <cmath>
+#include <mutex>
+#include <map>
+
+namespace nfft {
+
+// instantiated in nfft_k_mix_f32.hip / nfft_k_mix_f64.hip
+extern template __global__ void k_mix_line<float, false>(MixArgs);
+extern template __global__ void k_mix_line<float, true>(MixArgs);
+extern template __global__ void k_mix_line<double, false>(MixArgs);
+extern template __global__ void k_mix_line<double, true>(MixArgs);
+
+namespace {
+
+constexpr int kRadices[] = {32, 30, 28, 27, 25, 24, 21, 20, 18, 16, 15, 14, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+
+// VALU instructions per point of a radix-r butterfly (two-level radices: both
+// levels and the inner twiddles)
+double dft_ops(int r)
+{
+    switch (r) {
+    case 2: return 2;
+    case 3: return 4.7;
+    case 4: return 4;
+    case 5: return 7.2;
+    case 7: return 9.4;
+    case 8: return 6.5;
+    case 16: return 10.5;
+    }
+    static const int two[][2] = {{2, 3}, {3, 3}, {2, 5}, {4, 3}, {3, 5}, {4, 5}, {5, 5}, {2, 7}, {2, 9},
+                                 {3, 7}, {3, 8}, {3, 9}, {4, 7}, {5, 6}, {4, 8}};
+    for (auto &t : two)
+        if (t[0] * t[1] == r) return dft_ops(t[0]) + dft_ops(t[1]) + 4.0 * (t[0] - 1) * (t[1] - 1) / r;
+    return 20;
+}
+
+int gcd_int(int a, int b) { return b ? gcd_int(b, a % b) : a; }
+
+float rcp_up_host(int d) { return (1.0f / (float)d) * 1.00000095367431640625f; }
+
+// Fill the steps of radices r[0..ns) (execution order) for G lines; false if
+// the lines do not fit the LDS.  Returns in *conflict the expected extra LDS
+// cycles factor of the first stage's writes.
+bool fill(MixPlan &p, int prec, int L, const int *r, int ns, bool blue, int G, double *conflict)
+{
+    const size_t cb = prec == 0 ? 8 : 16;
+    const int banks = prec == 0 ? 32 : 16;  // elements per LDS row of banks
+    p.L = L;
+    p.stages = ns;
+    p.steps = blue ? 2 * ns - 1 : ns;
+    p.G = G;
+    *conflict = 1.0;
+    for (int pads = 2; pads >= 0; pads--) {
+        long long lp = p.steps > 1 ? L : 0;
+        int Ns = 1;
+        for (int s = 0; s < p.steps; s++) {
+            MixStep &t = p.st[s];
+            const bool mid = blue && s == ns - 1;
+            t.radix = s < ns ? r[s] : r[2 * (ns - 1) - s];
+            t.ns = Ns;
+            t.nb = L / t.radix;
+            t.q = t.nb / Ns;
+            t.inb = rcp_up_host(t.nb);
+            t.ins = rcp_up_host(Ns);
+            const int so = mid ? 1 : Ns, U = so * t.radix;
+            t.pad = 0;
+            if (s + 1 < p.steps) {
+                if (so == 1) {
+                    if (pads >= 1 && U % 2 == 0) t.pad = 1;
+                    if (t.pad == 0) *conflict = std::max(*conflict, (double)gcd_int(U, banks) / 2);
+                } else if (pads >= 2) {
+                    const int w = ((so - U) % banks + banks) % banks;
+                    if ((long long)(L / U) * w <= L / 16) t.pad = w;
+                }
+                lp = std::max(lp, (long long)(L / U) * (U + t.pad));
+            }
+            Ns = mid ? t.radix : Ns * t.radix;
+        }
+        p.lp = (int)lp;
+        if ((size_t)lp * G * cb <= kMixLds) return true;
+        *conflict = 1.0;
+    }
+    return false;
+}
+
+// Estimated cost per line: instructions issued per wave and stage, scaled by
+// how many waves a CU keeps to hide latencies with.
+double cost_of(const MixPlan &p, int prec, double conflict)
+{
+    const size_t cb = prec == 0 ? 8 : 16;
+    const size_t lds = std::max<size_t>((size_t)p.lp * p.G * cb, 1024);
+    const int wv = p.nth / 64, vgpr_waves = prec == 0 ? 16 : 8;
+    const int wg = std::max(1, std::min((int)(kMixLds / lds), vgpr_waves / wv));
+    double c = 0;
+    for (int s = 0; s < p.steps; s++) {
+        const int total = p.G * p.st[s].nb, R = p.st[s].radix;
+        const bool mid = p.steps > p.stages && s == p.stages - 1;
+        double waves = 0;
+        for (int i = 0; i * p.nth < total; i++) waves += std::min(wv, (total - i * p.nth + 63) / 64);
+        // a whole round of the workgroup takes as long as its busiest SIMD
+        double simd = 0;
+        for (int i = 0; i * p.nth < total; i++) simd += (std::min(wv, (total - i * p.nth + 63) / 64) + 3) / 4;
+        const double per = R * (dft_ops(R) * (mid ? 2 : 1) + 16 + (s == 0 && R > 1 ? 4 * (conflict - 1) : 0)) + 50;
+        c += (wg > 1 ? waves / 4 * 0.7 + simd * 0.3 : simd) * per + 60;
+    }
+    return c / p.G * (1.0 + 6.0 / (wg * wv));
+}
+
+struct Search {
+    int prec, L;
+    bool blue;
+    double best = 1e300;
+    MixPlan plan;
+    int r[kMixMaxStages];
+
+    void consider(int ns)
+    {
+        const int tmax = prec == 0 ? mix_threads<float>() : mix_threads<double>();
+        const int gmax = L >= 4096 ? 1 : std::min(256, 8192 / L);
+        // an odd radix first, if there is one: its writes need no padding
+        int ord[kMixMaxStages];
+        std::copy(r, r + ns, ord);
+        for (int i = 0; i < ns; i++)
+            if (ord[i] % 2) {
+                std::rotate(ord, ord + i, ord + i + 1);
+                break;
+            }
+        for (int G = 1; G <= gmax; G = G < 8 ? G + 1 : G + G / 4) {
+            MixPlan p;
+            double conflict;
+            if (!fill(p, prec, L, ord, ns, blue, G, &conflict)) break;
+            for (int nth = 64; nth <= tmax; nth += 64) {
+                bool ok = true;
+                int most = 0;
+                for (int s = 0; s < ns && ok; s++) {
+                    const int total = G * (L / ord[s]);
+                    ok = total <= nth * mix_reps(ord[s]);
+                    most = std::max(most, total);
+                }
+                if (!ok) continue;
+                if (nth - 64 >= most) break;  // only idle waves beyond
+                p.nth = nth;
+                const double c = cost_of(p, prec, conflict);
+                if (c < best) {
+                    best = c;
+                    plan = p;
+                }
+            }
+        }
+    }
+    // every multiset of radices, in falling order, of at most `stages` stages
+    void split(int left, int depth, int maxr, int stages)
+    {
+        if (left == 1) {
+            if (depth) consider(depth);
+            return;
+        }
+        if (depth == stages) return;
+        for (int q : kRadices)
+            if (q <= maxr && left % q == 0 && std::pow((double)q, stages - depth) >= left) {
+                r[depth] = q;
+                split(left / q, depth + 1, q, stages);
+            }
+    }
+};
+
+struct Found {
+    double cost;
+    MixPlan plan;
+};
+std::mutex g_mix_mu;
+std::map<long long, Found> g_mix_plans;  // by length, precision and form: schedules are searched once per process
+
+const Found &find(int prec, int L, bool blue)
+{
+    const long long key = ((long long)L << 2) | (prec << 1) | (blue ? 1 : 0);
+    std::lock_guard<std::mutex> lk(g_mix_mu);
+    auto it = g_mix_plans.find(key);
+    if (it == g_mix_plans.end()) {
+        Search se;
+        se.prec = prec;
+        se.L = L;
+        se.blue = blue;
+        // the fewest stages possible and one more
+        for (int stages = 1, found = 0; stages <= kMixMaxStages && found < 2; stages++) {
+            se.split(L, 0, 32, stages);
+            if (se.best < 1e299) found++;
+        }
+        it = g_mix_plans.emplace(key, Found{se.best, se.plan}).first;
+    }
+    return it->second;
+}
+
+}  // namespace
+
+int mix_max(int prec) { return (int)(kMixLds / (prec == F32 ? 8 : 16)); }
+
+bool mix_plan(int prec, long long n, MixPlan *p)
+{
+    if (n < 2 || n > mix_max(prec)) return false;
+    const Found &f = find(prec, (int)n, false);
+    if (f.cost >= 1e299) return false;
+    *p = f.plan;
+    return true;
+}
+
+bool mix_blue_plan(int prec, long long n, MixPlan *p)
+{
+    // 7-smooth lengths from 2n - 1 up to a quarter more: the cheapest
+    const long long lo = 2 * n - 1, hi = std::min<long long>(mix_max(prec), lo + std::max<long long>(lo / 4, 4));
+    double best = 1e300;
+    for (long long m = lo; m <= hi; m++) {
+        long long v = m;
+        for (int q : {2, 3, 5, 7})
+            while (v % q == 0) v /= q;
+        if (v != 1) continue;
+        const Found &f = find(prec, (int)m, true);
+        if (f.cost < best) {
+            best = f.cost;
+            *p = f.plan;
+        }
+    }
+    return best < 1e299;
+}
+
+template <typename T, bool BLUE> static hipError_t mix_go(const MixArgs &a0, hipStream_t s)
+{
+    static const bool attr = [] {  // once per instantiation and process
+        (void)hipFuncSetAttribute((const void *)k_mix_line<T, BLUE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)kMixLds);
+        (void)hipGetLastError();
+        return true;
+    }();
+    (void)attr;
+    if (a0.nlines < 1) return hipSuccess;
+    MixArgs a = a0;
+    // lines of a workgroup are addressed by 32-bit byte offsets
+    const long long far = std::max(a.in_dist, a.out_dist);
+    if ((far * (a.pl.G - 1) + a.pl.L) * (long long)sizeof(Cx<T>) >= (1LL << 32)) a.pl.G = 1;
+    const long long grid = (a.nlines + a.pl.G - 1) / a.pl.G;
+    const size_t lds = (size_t)a.pl.G * a.pl.lp * sizeof(Cx<T>);
+    if (grid > 0x7fffffffLL || lds > kMixLds || a.pl.nth < 64 || a.pl.nth > mix_threads<T>()) return hipErrorInvalidValue;
+    for (int i = 0; i < a.pl.steps; i++)  // every butterfly has its place in a thread
+        if (a.pl.G * a.pl.st[i].nb > a.pl.nth * mix_reps(a.pl.st[i].radix)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_mix_line<T, BLUE>), dim3((unsigned)grid), dim3(a.pl.nth), lds, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_mix(int prec, const MixArgs &a, hipStream_t s)
+{
+    const bool blue = a.pl.steps > a.pl.stages || a.chirp;
+    const int slot = prof_on() ? prof_begin(s) : -1;
+    const hipError_t e = prec == F32 ? (blue ? mix_go<float, true>(a, s) : mix_go<float, false>(a, s))
+                                     : (blue ? mix_go<double, true>(a, s) : mix_go<double, false>(a, s));
+    if (slot >= 0)
+        prof_end(slot, s, blue ? "k_mix_line(bluestein)" : "k_mix_line", prec, a.pl.L,
+                 2.0 * (double)a.nlines * (blue ? a.n : a.pl.L) * (prec == F32 ? 8.0 : 16.0));
+    return e;
+}
+
+}  // namespace nfft

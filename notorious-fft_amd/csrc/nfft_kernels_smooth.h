@@ -12,8 +12,8 @@
 // Each stage dispatches once (uniformly) on its radix to a compile-time
 // butterfly, so the per-thread values stay in registers.
 //
-// Used for whole lines (k_smooth_line, several lines per workgroup) and as
-// the column / row passes of a four-step for lengths above the LDS limit.
+// Used as the column / row passes of a four-step for lengths beyond the
+// one-pass lines of nfft_kernels_mix.h, and by the ragged kernel.
 #pragma once
 #include "nfft_kernels.h"
 #include "nfft_kernels_persist.h"  // coh_ld / coh_st
@@ -21,11 +21,10 @@
 namespace nfft {
 
 constexpr int kSmoothMaxStages = 24;
-// Largest radix of the standalone mixed-radix kernels (k_smooth_line,
-// k_smooth_col, k_smooth_rowT): 10 in FP32 (N = 100 as 10 x 10: 0.78 -> 0.70
-// ms per 2^27 points, N = 10^4 1.85 -> 1.61 ms), 8 in FP64, where the radix-10
-// butterfly's registers (92 -> 118 VGPRs) cost more occupancy than the stages
-// it saves (N = 100 1.21 -> 1.26 ms).
+// Largest radix of the standalone mixed-radix kernels (k_smooth_col,
+// k_smooth_rowT): 10 in FP32 (N = 10^4 as 100 x 100, 2^27 points: 1.85 -> 1.61
+// ms), 8 in FP64, where the radix-10 butterfly's registers (92 -> 118 VGPRs)
+// cost more occupancy than the stages it saves (2.76 -> 2.82 ms).
 template <typename T> __host__ __device__ constexpr int smooth_radix() { return sizeof(T) == 4 ? 10 : 8; }
 
 // Stage schedule of a 7-smooth length (radices in execution order).
@@ -142,6 +141,110 @@ template <> struct RootTab<25> {
     static constexpr double s[25] = {0.0, 0.2486898871648548, 0.48175367410171527, 0.6845471059286887, 0.8443279255020151, 0.9510565162951535, 0.9980267284282716, 0.9822872507286887, 0.9048270524660196, 0.7705132427757893, 0.5877852522924731, 0.368124552684678, 0.12533323356430426, -0.12533323356430426, -0.368124552684678, -0.5877852522924731, -0.7705132427757893, -0.9048270524660196, -0.9822872507286887, -0.9980267284282716, -0.9510565162951535, -0.8443279255020151, -0.6845471059286887, -0.48175367410171527, -0.2486898871648548};
 };
 
+template <> struct RootTab<14> {
+    static constexpr double c[14] = {1.0, 0.9009688679024191, 0.6234898018587335, 0.2225209339563144,
+        -0.2225209339563144, -0.6234898018587335, -0.9009688679024191, -1.0, -0.9009688679024191,
+        -0.6234898018587335, -0.2225209339563144, 0.2225209339563144, 0.6234898018587335, 0.9009688679024191};
+    static constexpr double s[14] = {0.0, 0.4338837391175581, 0.7818314824680298, 0.9749279121818236,
+        0.9749279121818236, 0.7818314824680298, 0.4338837391175581, 0.0, -0.4338837391175581,
+        -0.7818314824680298, -0.9749279121818236, -0.9749279121818236, -0.7818314824680298,
+        -0.4338837391175581};
+};
+template <> struct RootTab<18> {
+    static constexpr double c[18] = {1.0, 0.9396926207859084, 0.766044443118978, 0.5, 0.17364817766693036,
+        -0.17364817766693036, -0.5, -0.766044443118978, -0.9396926207859084, -1.0, -0.9396926207859084,
+        -0.766044443118978, -0.5, -0.17364817766693036, 0.17364817766693036, 0.5, 0.766044443118978,
+        0.9396926207859084};
+    static constexpr double s[18] = {0.0, 0.3420201433256687, 0.6427876096865394, 0.8660254037844386,
+        0.984807753012208, 0.984807753012208, 0.8660254037844386, 0.6427876096865394, 0.3420201433256687, 0.0,
+        -0.3420201433256687, -0.6427876096865394, -0.8660254037844386, -0.984807753012208, -0.984807753012208,
+        -0.8660254037844386, -0.6427876096865394, -0.3420201433256687};
+};
+template <> struct RootTab<21> {
+    static constexpr double c[21] = {1.0, 0.9555728057861407, 0.8262387743159949, 0.6234898018587335,
+        0.36534102436639504, 0.07473009358642425, -0.2225209339563144, -0.5, -0.7330518718298263,
+        -0.9009688679024191, -0.9888308262251285, -0.9888308262251285, -0.9009688679024191,
+        -0.7330518718298263, -0.5, -0.2225209339563144, 0.07473009358642425, 0.36534102436639504,
+        0.6234898018587335, 0.8262387743159949, 0.9555728057861407};
+    static constexpr double s[21] = {0.0, 0.2947551744109042, 0.5633200580636221, 0.7818314824680298,
+        0.9308737486442042, 0.9972037971811801, 0.9749279121818236, 0.8660254037844386, 0.6801727377709194,
+        0.4338837391175581, 0.14904226617617444, -0.14904226617617444, -0.4338837391175581,
+        -0.6801727377709194, -0.8660254037844386, -0.9749279121818236, -0.9972037971811801,
+        -0.9308737486442042, -0.7818314824680298, -0.5633200580636221, -0.2947551744109042};
+};
+template <> struct RootTab<24> {
+    static constexpr double c[24] = {1.0, 0.9659258262890683, 0.8660254037844386, 0.7071067811865476, 0.5,
+        0.25881904510252074, 0.0, -0.25881904510252074, -0.5, -0.7071067811865476, -0.8660254037844386,
+        -0.9659258262890683, -1.0, -0.9659258262890683, -0.8660254037844386, -0.7071067811865476, -0.5,
+        -0.25881904510252074, 0.0, 0.25881904510252074, 0.5, 0.7071067811865476, 0.8660254037844386,
+        0.9659258262890683};
+    static constexpr double s[24] = {0.0, 0.25881904510252074, 0.5, 0.7071067811865476, 0.8660254037844386,
+        0.9659258262890683, 1.0, 0.9659258262890683, 0.8660254037844386, 0.7071067811865476, 0.5,
+        0.25881904510252074, 0.0, -0.25881904510252074, -0.5, -0.7071067811865476, -0.8660254037844386,
+        -0.9659258262890683, -1.0, -0.9659258262890683, -0.8660254037844386, -0.7071067811865476, -0.5,
+        -0.25881904510252074};
+};
+template <> struct RootTab<27> {
+    static constexpr double c[27] = {1.0, 0.9730448705798238, 0.8936326403234123, 0.766044443118978,
+        0.5971585917027862, 0.39607976603915684, 0.17364817766693036, -0.05814482891047583,
+        -0.28680323271109026, -0.5, -0.6862416378687336, -0.8354878114129364, -0.9396926207859084,
+        -0.993238357741943, -0.993238357741943, -0.9396926207859084, -0.8354878114129364, -0.6862416378687336,
+        -0.5, -0.28680323271109026, -0.05814482891047583, 0.17364817766693036, 0.39607976603915684,
+        0.5971585917027862, 0.766044443118978, 0.8936326403234123, 0.9730448705798238};
+    static constexpr double s[27] = {0.0, 0.23061587074244017, 0.44879918020046217, 0.6427876096865394,
+        0.8021231927550437, 0.918216106880274, 0.984807753012208, 0.9983081582712682, 0.9579895123154889,
+        0.8660254037844386, 0.7273736415730487, 0.549508978070806, 0.3420201433256687, 0.11609291412523023,
+        -0.11609291412523023, -0.3420201433256687, -0.549508978070806, -0.7273736415730487,
+        -0.8660254037844386, -0.9579895123154889, -0.9983081582712682, -0.984807753012208, -0.918216106880274,
+        -0.8021231927550437, -0.6427876096865394, -0.44879918020046217, -0.23061587074244017};
+};
+template <> struct RootTab<28> {
+    static constexpr double c[28] = {1.0, 0.9749279121818236, 0.9009688679024191, 0.7818314824680298,
+        0.6234898018587335, 0.4338837391175581, 0.2225209339563144, 0.0, -0.2225209339563144,
+        -0.4338837391175581, -0.6234898018587335, -0.7818314824680298, -0.9009688679024191,
+        -0.9749279121818236, -1.0, -0.9749279121818236, -0.9009688679024191, -0.7818314824680298,
+        -0.6234898018587335, -0.4338837391175581, -0.2225209339563144, 0.0, 0.2225209339563144,
+        0.4338837391175581, 0.6234898018587335, 0.7818314824680298, 0.9009688679024191, 0.9749279121818236};
+    static constexpr double s[28] = {0.0, 0.2225209339563144, 0.4338837391175581, 0.6234898018587335,
+        0.7818314824680298, 0.9009688679024191, 0.9749279121818236, 1.0, 0.9749279121818236,
+        0.9009688679024191, 0.7818314824680298, 0.6234898018587335, 0.4338837391175581, 0.2225209339563144,
+        0.0, -0.2225209339563144, -0.4338837391175581, -0.6234898018587335, -0.7818314824680298,
+        -0.9009688679024191, -0.9749279121818236, -1.0, -0.9749279121818236, -0.9009688679024191,
+        -0.7818314824680298, -0.6234898018587335, -0.4338837391175581, -0.2225209339563144};
+};
+template <> struct RootTab<30> {
+    static constexpr double c[30] = {1.0, 0.9781476007338057, 0.9135454576426009, 0.8090169943749475,
+        0.6691306063588582, 0.5, 0.30901699437494745, 0.10452846326765347, -0.10452846326765347,
+        -0.30901699437494745, -0.5, -0.6691306063588582, -0.8090169943749475, -0.9135454576426009,
+        -0.9781476007338057, -1.0, -0.9781476007338057, -0.9135454576426009, -0.8090169943749475,
+        -0.6691306063588582, -0.5, -0.30901699437494745, -0.10452846326765347, 0.10452846326765347,
+        0.30901699437494745, 0.5, 0.6691306063588582, 0.8090169943749475, 0.9135454576426009,
+        0.9781476007338057};
+    static constexpr double s[30] = {0.0, 0.20791169081775934, 0.4067366430758002, 0.5877852522924731,
+        0.7431448254773942, 0.8660254037844386, 0.9510565162951535, 0.9945218953682733, 0.9945218953682733,
+        0.9510565162951535, 0.8660254037844386, 0.7431448254773942, 0.5877852522924731, 0.4067366430758002,
+        0.20791169081775934, 0.0, -0.20791169081775934, -0.4067366430758002, -0.5877852522924731,
+        -0.7431448254773942, -0.8660254037844386, -0.9510565162951535, -0.9945218953682733,
+        -0.9945218953682733, -0.9510565162951535, -0.8660254037844386, -0.7431448254773942,
+        -0.5877852522924731, -0.4067366430758002, -0.20791169081775934};
+};
+template <> struct RootTab<32> {
+    static constexpr double c[32] = {1.0, 0.9807852804032304, 0.9238795325112867, 0.8314696123025452,
+        0.7071067811865476, 0.5555702330196022, 0.3826834323650898, 0.19509032201612828, 0.0,
+        -0.19509032201612828, -0.3826834323650898, -0.5555702330196022, -0.7071067811865476,
+        -0.8314696123025452, -0.9238795325112867, -0.9807852804032304, -1.0, -0.9807852804032304,
+        -0.9238795325112867, -0.8314696123025452, -0.7071067811865476, -0.5555702330196022,
+        -0.3826834323650898, -0.19509032201612828, 0.0, 0.19509032201612828, 0.3826834323650898,
+        0.5555702330196022, 0.7071067811865476, 0.8314696123025452, 0.9238795325112867, 0.9807852804032304};
+    static constexpr double s[32] = {0.0, 0.19509032201612828, 0.3826834323650898, 0.5555702330196022,
+        0.7071067811865476, 0.8314696123025452, 0.9238795325112867, 0.9807852804032304, 1.0,
+        0.9807852804032304, 0.9238795325112867, 0.8314696123025452, 0.7071067811865476, 0.5555702330196022,
+        0.3826834323650898, 0.19509032201612828, 0.0, -0.19509032201612828, -0.3826834323650898,
+        -0.5555702330196022, -0.7071067811865476, -0.8314696123025452, -0.9238795325112867,
+        -0.9807852804032304, -1.0, -0.9807852804032304, -0.9238795325112867, -0.8314696123025452,
+        -0.7071067811865476, -0.5555702330196022, -0.3826834323650898, -0.19509032201612828};
+};
+
 // a * e^{DIR 2 pi i E / P}, E and P compile-time.
 template <int DIR, int P, int E, typename C> __device__ __forceinline__ C twp(C a)
 {
@@ -188,7 +291,9 @@ template <int R1, int R2, int DIR, typename C> __device__ __forceinline__ void d
 }
 
 // Radices of the mixed-radix stages: 2, 3, 4, 5, 7, 8, 16, and the two-level
-// 6 = 2 x 3, 9 = 3 x 3, 10 = 2 x 5, 12 = 4 x 3, 15 = 3 x 5, 20 = 4 x 5, 25 = 5 x 5.
+// 6 = 2 x 3, 9 = 3 x 3, 10 = 2 x 5, 12 = 4 x 3, 15 = 3 x 5, 20 = 4 x 5, 25 = 5 x 5;
+// the in-place lines (nfft_kernels_mix.h) also use 14 = 2 x 7, 18 = 2 x 9,
+// 21 = 3 x 7, 24 = 3 x 8, 27 = 3 x 9, 28 = 4 x 7, 30 = 5 x 6 and 32 = 4 x 8.
 template <int R, int DIR, typename C> __device__ __forceinline__ void dft_any(C *v)
 {
     if constexpr (R == 3 || R == 5 || R == 7) dft_odd<R, DIR>(v);
@@ -199,6 +304,14 @@ template <int R, int DIR, typename C> __device__ __forceinline__ void dft_any(C 
     else if constexpr (R == 15) dft_two<3, 5, DIR>(v);
     else if constexpr (R == 20) dft_two<4, 5, DIR>(v);
     else if constexpr (R == 25) dft_two<5, 5, DIR>(v);
+    else if constexpr (R == 14) dft_two<2, 7, DIR>(v);
+    else if constexpr (R == 18) dft_two<2, 9, DIR>(v);
+    else if constexpr (R == 21) dft_two<3, 7, DIR>(v);
+    else if constexpr (R == 24) dft_two<3, 8, DIR>(v);
+    else if constexpr (R == 27) dft_two<3, 9, DIR>(v);
+    else if constexpr (R == 28) dft_two<4, 7, DIR>(v);
+    else if constexpr (R == 30) dft_two<5, 6, DIR>(v);
+    else if constexpr (R == 32) dft_two<4, 8, DIR>(v);
     else dftR<R, DIR>(v);
 }
 
@@ -282,62 +395,6 @@ __device__ __forceinline__ Cx<T> *smooth_lines(Cx<T> *a, Cx<T> *b, int G, const 
     }
     return src;
 }
-
-// ---------------------------------------------------------------------------
-// k_smooth_line: G lines of a 7-smooth length L per workgroup, contiguous
-// lines (line l at in + l * in_dist), out scaled by `scale`.
-// ---------------------------------------------------------------------------
-struct SmoothArgs {
-    const void *in;
-    void *out;
-    long long nlines;
-    long long in_dist, out_dist;
-    int G;            // lines per workgroup
-    SmoothPlan sp;
-    const void *tw;   // L entries e^{-2 pi i q / L}
-    double scale;
-};
-
-// TWL: the L twiddles are copied into LDS after the two line buffers (the
-// launcher gives up lines per workgroup for them, keeping the LDS size).
-template <typename T, int DIR, bool TWL = false> __global__ void __launch_bounds__(256) k_smooth_line(SmoothArgs a)
-{
-    using C = Cx<T>;
-    extern __shared__ char smem[];
-    C *A = (C *)smem;
-    const int L = a.sp.L, G = a.G;
-    C *B = A + G * L;
-    const long long l0 = (long long)blockIdx.x * G;
-    const int g_here = (int)((a.nlines - l0) < G ? (a.nlines - l0) : G);
-    const C *src = (const C *)a.in;
-    const C *twp = (const C *)a.tw;
-    if constexpr (TWL) {
-        C *tl = B + G * L;
-        for (int i = threadIdx.x; i < L; i += blockDim.x) tl[i] = twp[i];
-        twp = tl;
-    }
-    const float iL = rcp_up(L);
-    for (int idx = threadIdx.x; idx < G * L; idx += blockDim.x) {
-        const int g = fdiv(idx, iL), p = idx - __mul24(g, L);
-        A[idx] = g < g_here ? src[(l0 + g) * a.in_dist + p] : cmk<C>((T)0, (T)0);
-    }
-    __syncthreads();
-    const C *res = smooth_lines<T, DIR, smooth_radix<T>()>(A, B, G, a.sp, twp);
-    C *dst = (C *)a.out;
-    const T sc = (T)a.scale;
-    for (int idx = threadIdx.x; idx < G * L; idx += blockDim.x) {
-        const int g = fdiv(idx, iL), p = idx - __mul24(g, L);
-        if (g < g_here) {
-            C v = res[idx];
-            if (sc != (T)1) v = cscale(v, sc);
-            dst[(l0 + g) * a.out_dist + p] = v;
-        }
-    }
-}
-
-}  // namespace nfft
-
-namespace nfft {
 
 // ---------------------------------------------------------------------------
 // Mixed-radix four-step tiles for N = N1 x N2 (both 7-smooth): element n of

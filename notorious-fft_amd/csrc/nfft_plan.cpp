@@ -288,13 +288,12 @@ static int balanced_width(int len, int wmax)
     return (len + tiles - 1) / tiles;
 }
 
-// Measured on MI355X (2^28 FP32 / 2^27 FP64 elements): mixed-radix lines beat
-// Bluestein for every FP64 length and for FP32 up to 512 points; the
-// mixed-radix four-step wins for FP64 unless its tiles are a single column
-// or row wide, and for FP32 from 10^4 points with tiles >= 4 wide.
-static bool smooth_default(int prec, long long n, bool line, int wmin)
+// Measured on MI355X (2^28 FP32 / 2^27 FP64 elements), beyond the one-pass
+// lines (which win at every length they exist for): the mixed-radix four-step
+// wins for FP64 unless its tiles are a single column or row wide, and for
+// FP32 from 10^4 points with tiles >= 4 wide.
+static bool smooth_default(int prec, long long n, int wmin)
 {
-    if (line) return prec == F64 || n <= 512;
     return prec == F64 ? wmin >= 2 : (n >= 10000 && wmin >= 4);
 }
 
@@ -707,28 +706,28 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
     // when NFFT_TUNE=1, else the measured default rule
     const int smooth_env = env_int("NFFT_SMOOTH", 1);  // 0: never, 2: whenever possible
     if (smooth_env == 2 && smooth_mode == 2) smooth_mode = 1;
-    if (smooth_mode != 0 && smooth_env != 0 && !is_pow2(n)) {
+    if (smooth_mode != 0 && smooth_mode != 3 && smooth_env != 0 && !is_pow2(n)) {
         SmoothPlan p1{}, p2{};
-        const int mr = smooth_radix_of(prec);
-        const bool line = n <= smooth_line_max(prec) && smooth_factor(n, &p1, mr);
-        const bool four = !line && (smooth_split(n, smooth_line_max(prec), &p1, &p2, mr) ||
-                                    smooth_split(n, prec == F32 ? 8192 : 4096, &p1, &p2, mr));
-        if (line || four) {
+        const int mr = smooth_radix_of(prec), lm = smooth_line_max(prec);
+        // One pass, a line or a group of lines per workgroup, up to mix_max;
+        // NFFT_SMOOTH=2 takes the four-step from smooth_line_max on.
+        const bool mix = (smooth_env != 2 || n <= lm) && mix_plan(prec, n, &mx);
+        const bool four = !mix && (smooth_split(n, lm, &p1, &p2, mr) ||
+                                   smooth_split(n, prec == F32 ? 8192 : 4096, &p1, &p2, mr));
+        if (mix || four) {
             const int budget = smooth_tile_points(prec);
             const int w1 = four ? balanced_width(p2.L, budget / p1.L) : 0;
             const int w2 = four ? balanced_width(p1.L, budget / p2.L) : 0;
             int use = smooth_mode == 1 ? 1 : tuned_choice(prec, n);
             if (use < 0 && env_int("NFFT_TUNE", 0)) use = tune_smooth(n, prec);
-            if (use < 0) use = smooth_default(prec, n, line, std::min(w1, w2)) ? 1 : 0;
+            if (use < 0) use = mix || smooth_default(prec, n, std::min(w1, w2)) ? 1 : 0;
+            if (use == 1 && mix) {
+                algo = ALG_MIX;
+                tw_a = phase_table(prec, n, 1, 0, n);
+                return tw_a != nullptr;
+            }
             if (use == 1) {
                 sp = p1;
-                if (line) {
-                    algo = ALG_SMOOTH;
-                    L = n;
-                    sgroup = std::max(1, budget / n);
-                    tw_a = phase_table(prec, n, 1, 0, n);
-                    return tw_a != nullptr;
-                }
                 algo = ALG_SMOOTH4;
                 sp2 = p2;
                 n1 = p1.L;
@@ -748,7 +747,18 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
     const double2 *chirp64 = nullptr;
     chirp = chirp_table(prec, n, &chirp64);
     if (!chirp || !chirp64) return false;
-    if (m <= line_max(prec)) {
+    // Where the power-of-two M does not fit one workgroup, a 7-smooth M that
+    // does makes the transform one pass instead of three (2^26 points: FP32 N
+    // = 10007 2.27 -> 1.06 ms, FP64 N = 4097 4.12 -> 2.10 ms).  Where both
+    // fit, the power-of-two line is the faster (FP32 N = 1009 0.47 vs 0.76
+    // ms, FP64 0.86 vs 1.65).
+    const bool mixblue = smooth_mode != 3 && m > line_max(prec) && mix_blue_plan(prec, n, &mx);
+    if (mixblue) {
+        algo = ALG_MIXBLUE;
+        m = mx.L;
+        tw_a = phase_table(prec, m, 1, 0, m);
+        if (!tw_a) return false;
+    } else if (m <= line_max(prec)) {
         algo = ALG_BLUE1;
         L = m;
         tw_a = stage_table(prec, m);
@@ -759,7 +769,7 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
         m2 = 1 << lg2;
         m1 = m / m2;
     }
-    if (m > line_max(prec) && m1 > col_max(prec)) {
+    if (!mixblue && m > line_max(prec) && m1 > col_max(prec)) {
         // M beyond the three-pass form: chirp, FFT_M, x H, IFFT_M, chirp as
         // elementwise passes around an M-point engine
         if (m > kMaxLen) {
@@ -771,7 +781,7 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
         sub1 = std::make_shared<C2C>();
         if (!sub1->init(m, prec)) return false;
         scratch_per_line = m + sub1->scratch_per_line;
-    } else if (m > line_max(prec)) {
+    } else if (!mixblue && m > line_max(prec)) {
         algo = ALG_BLUE3;
         tw_a = stage_table(prec, m1);
         tw_b = stage_table(prec, m2);
@@ -780,7 +790,7 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
     }
     // filter spectrum H = FFT_m(h) / m, computed in FP64 by this engine
     C2C h64;
-    if (!h64.init(m, F64)) return false;
+    if (!h64.init(m, F64, mixblue ? 1 : 2)) return false;
     hipStream_t st = setup_stream();
     void *hbuf = nullptr, *Hbuf = nullptr, *sbuf = nullptr;
     bool ok = hip_ok(dev_malloc(&hbuf, (size_t)m * 16), "hipMalloc") &&
@@ -846,14 +856,16 @@ std::string C2C::describe() const
             snprintf(b, sizeof b, "four-step %dx%d", n1, n2);
         break;
     case ALG_BLUE1: snprintf(b, sizeof b, "bluestein N=%d M=%d single-pass", n, m); break;
-    case ALG_SMOOTH: {
-        int o = snprintf(b, sizeof b, "mixed-radix %d (", n);
-        for (int i = 0; i < sp.ns && o < (int)sizeof b - 8; i++)
-            o += snprintf(b + o, sizeof b - o, i ? "x%d" : "%d", sp.radix[i]);
-        snprintf(b + o, sizeof b - o, ")");
+    case ALG_SMOOTH4: snprintf(b, sizeof b, "mixed-radix four-step %dx%d", n1, n2); break;
+    case ALG_MIX:
+    case ALG_MIXBLUE: {
+        int o = algo == ALG_MIX ? snprintf(b, sizeof b, "mixed-radix %d (", n)
+                                : snprintf(b, sizeof b, "bluestein N=%d M=%d one pass (", n, m);
+        for (int i = 0; i < mx.stages && o < (int)sizeof b - 48; i++)
+            o += snprintf(b + o, sizeof b - o, i ? "x%d" : "%d", mx.st[i].radix);
+        snprintf(b + o, sizeof b - o, ", %d lines on %d threads)", mx.G, mx.nth);
         break;
     }
-    case ALG_SMOOTH4: snprintf(b, sizeof b, "mixed-radix four-step %dx%d", n1, n2); break;
     case ALG_BLUE3: snprintf(b, sizeof b, "bluestein N=%d M=%d (%dx%d)", n, m, m1, m2); break;
     case ALG_BIG:
         snprintf(b, sizeof b, "six-step %dx%d [%s | %s]", n1, n2, sub1 ? sub1->describe().c_str() : "?",
@@ -881,9 +893,14 @@ hipError_t C2C::run(const void *in, void *out, long long nlines, long long in_di
         BlueArgs a{in, out, nlines, in_dist, out_dist, n, tw_a, chirp, H, dir > 0 ? 1 : 0, scale};
         return launch_blue_line(prec, m, a, s);
     }
-    case ALG_SMOOTH: {
-        SmoothArgs a{in, out, nlines, in_dist, out_dist, sgroup, sp, tw_a, scale};
-        return launch_smooth_line(prec, dir, a, s);
+    case ALG_MIX:
+    case ALG_MIXBLUE: {
+        MixArgs a{in, out, nlines, in_dist, out_dist, mx, tw_a, dir > 0 ? 1 : 0, scale, n, nullptr, nullptr};
+        if (algo == ALG_MIXBLUE) {
+            a.chirp = chirp;
+            a.H = H;
+        }
+        return launch_mix(prec, a, s);
     }
     case ALG_SMOOTH4: {
         if (scratch_lines < 1 || !scratch) return hipErrorInvalidValue;

@@ -733,7 +733,7 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
             // for M <= line limit (natural) or M1 x M2 (permuted); the ragged
             // kernel needs natural order for M <= 4096 and the [k1][k2] order
             // for its own M1 x M2 split, so H is rebuilt here when they differ.
-            if (!e.init(n, prec, 0)) { ragged_free(r); return setup_fail(fails0); }
+            if (!e.init(n, prec, 3)) { ragged_free(r); return setup_fail(fails0); }
             t.chirp = e.chirp;
             size_kind[n] = m <= 4096 ? RG_BLUE1 : RG_BLUE3;
             if (m <= 4096) {

@@ -1,0 +1,68 @@
+"""One-pass mixed-radix lines (nfft_kernels_mix.h) against pocketfft: one to
+six stages, groups of lines with a ragged last group, the longest lines of
+each precision, and Bluestein over a 7-smooth M in one workgroup.
+
+Tolerance: each point passes about log2(N) levels of butterflies, with a
+handful of roundings (sums, one twiddle product of two rounded factors) per
+level; as a random walk that is below 4 eps sqrt(log2 N), doubled for the
+two transforms and three products of Bluestein."""
+import math
+
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+from gpu_util import pocket, rounded, run_plan
+
+pytestmark = pytest.mark.gpu
+
+EPS = {"f32": 2.0 ** -24, "f64": 2.0 ** -53}
+# single stage, two and three, odd ones, all radices of 7, up to the limit
+LINES = [3, 6, 7, 30, 35, 54, 100, 189, 640, 1029, 2401, 4374, 5000, 9216, 10206]
+LINES32 = LINES + [10290, 15625, 16807, 19683, 20000, 20412, 20480]
+LINES64 = LINES + [10240]
+
+
+@pytest.mark.parametrize("prec,n", [("f32", n) for n in LINES32] + [("f64", n) for n in LINES64])
+def test_lines(pkg, dev, prec, n):
+    plan = pkg.Plan("dft", prec, [n], 1)
+    desc = plan.describe()
+    plan.close()
+    assert desc.startswith("mixed-radix") and "lines on" in desc, desc
+    tol = 4 * EPS[prec] * math.sqrt(math.log2(n))
+    lines = int(desc.split(", ")[1].split()[0])  # per workgroup
+    for batch in (1, 2 * lines + 1):
+        x = rounded(ol.uniform(41, 2 * n * batch), prec)
+        for op, inplace in (("dft", False), ("dft", True), ("invdft", False)):
+            got = run_plan(pkg, dev, op, [n], x, batch, prec, inplace=inplace)
+            err = ol.rel_l2(got, pocket(op, [n], x, batch))
+            assert err < tol, (prec, n, batch, op, inplace, err, desc)
+
+
+@pytest.mark.parametrize("prec,n", [("f32", n) for n in (8209, 9973, 10007, 10169)] +
+                         [("f64", n) for n in (4099, 5003, 5101)])
+def test_bluestein_one_pass(pkg, dev, prec, n):
+    plan = pkg.Plan("dft", prec, [n], 1)
+    desc = plan.describe()
+    plan.close()
+    assert desc.startswith("bluestein") and "one pass" in desc, desc
+    tol = 2 * 4 * EPS[prec] * math.sqrt(math.log2(n))
+    for batch in (1, 3):
+        x = rounded(ol.uniform(42, 2 * n * batch), prec)
+        for op, inplace in (("dft", False), ("invdft", True)):
+            got = run_plan(pkg, dev, op, [n], x, batch, prec, inplace=inplace)
+            err = ol.rel_l2(got, pocket(op, [n], x, batch))
+            assert err < tol, (prec, n, batch, op, inplace, err, desc)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("dims", [[100, 48, 30], [5, 5000], [1000, 81]])
+def test_axes(pkg, dev, prec, dims):
+    """Contiguous and strided axes of an N-D transform through the same lines."""
+    p = int(np.prod(dims))
+    x = rounded(ol.uniform(43, 2 * p * 2), prec)
+    tol = 4 * EPS[prec] * math.sqrt(math.log2(p))
+    for op in ("dft", "invdft"):
+        got = run_plan(pkg, dev, op, dims, x, 2, prec)
+        err = ol.rel_l2(got, pocket(op, dims, x, 2))
+        assert err < tol, (prec, dims, op, err)
