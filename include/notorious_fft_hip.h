@@ -7,7 +7,7 @@
  *   - device-resident plans ("device-aux"): tables and scratch in HBM;
  *   - uniform batches of contiguous transforms on a caller stream;
  *   - an explicit normalisation flag;
- *   - ragged batches of mixed sizes (one persistent launch, graph-captured);
+ *   - ragged batches of mixed sizes (one graph launch);
  *   - vector-Jacobian products (adjoints) of every transform;
  *   - status codes with a thread-local message.
  * Library: libnotorious_fft_hip.so (both precisions; the precision is a plan
@@ -134,23 +134,21 @@ int nfft_plan_check(nfft_plan *plan, void *stream);
 
 /* Ragged batch: `count` 1D complex transforms of sizes[i] (1 <= N <= 65536,
  * any N), packed back to back (transform i starts at element
- * sizes[0] + ... + sizes[i-1]).  Execution is one persistent kernel launch
- * (after a one-node counter reset), recorded into a HIP graph on first use
- * for each (in, out, direction) and replayed afterwards.  Inverse transforms
+ * sizes[0] + ... + sizes[i-1]).  Execution is one HIP graph launch of a few
+ * kernels over the whole list, recorded on first use for each (in, out,
+ * direction) and replayed afterwards.  Inverse transforms
  * follow the reference's normalisation (1/N for non-power-of-two N only).
- * flags bit 0: autotune on a scratch batch -- first the tile size (column /
- * row groups per tile) and the pipeline lag of the long transforms over five
- * candidates, then the persistent grid (workgroups per CU); the choices are
- * appended to the file named by NFFT_TUNE_CACHE, if set, and read back (not
- * measured again) by later creates with the same size list. */
+ * flags bit 0: autotune on a scratch batch -- first the tile size (points per
+ * thread of a tile) and the scratch budget of the long transforms over five
+ * candidates, then a resident grid for their tiles (workgroups per CU); the
+ * choices are appended to the file named by NFFT_TUNE_CACHE, if set, and read
+ * back (not measured again) by later creates with the same size list. */
 int nfft_ragged_create(nfft_ragged **r, int prec, int count, const int *sizes, int flags);
 int nfft_ragged_execute(nfft_ragged *r, int inverse, const void *in, void *out, void *stream);
 int nfft_ragged_destroy(nfft_ragged *r);
 long long nfft_ragged_total(const nfft_ragged *r);
 
-/* Synchronises `stream` and reports whether an earlier execute of `r` hit a
- * device-side fault: the tiles of the long transforms wait for each other
- * with bounded waits that raise a flag instead of spinning forever. Returns
+/* Synchronises `stream` and reports whether the work on it completed:
  * NFFT_OK, or NFFT_E_HIP with the message set (outputs then undefined). */
 int nfft_ragged_check(nfft_ragged *r, void *stream);
 

@@ -167,11 +167,26 @@ hipError_t launch_smooth4(int prec, int dir, const Smooth4Args &a, hipStream_t s
 int smooth_line_max(int prec);
 inline int smooth_tile_points(int prec) { return prec == F32 ? 2048 : 1024; }
 
-// one-pass mixed-radix lines (nfft_k_mix.hip): the schedule of a 7-smooth
-// length n >= 2 (false: n has another factor, or is longer than mix_max), and
-// of a Bluestein transform of any length n over the 7-smooth M >= 2n - 1 that
-// is cheapest to transform (false: no such M in one workgroup)
+// Schedules of the mixed-radix lines and tiles (nfft_k_mix.hip).
+// How lanes map to the points of a workgroup's lines: neighbouring points
+// (contiguous lines), neighbouring lines (columns), or points on the first
+// step and lines on the last (rows stored transposed).
+enum MixLanes { MIX_LANES_POINTS = 0, MIX_LANES_LINES = 1, MIX_LANES_TRANSPOSE = 2 };
+// What a schedule may use: lines and threads per workgroup, LDS bytes.
+struct MixShape {
+    int g_min = 1, g_max = 1;
+    int nth_min = 64, nth_max = 1024;
+    MixLanes lanes = MIX_LANES_POINTS;
+    size_t lds_max = kMixLds;
+};
 int mix_max(int prec);
+// The cheapest schedule of length n within a shape (blue: a Bluestein line's,
+// forward and inverse); false if n has a factor above 7 or nothing fits.
+// cost: per line, in issue slots of a SIMD.
+bool mix_fit(int prec, long long n, bool blue, const MixShape &sh, MixPlan *p, double *cost = nullptr);
+// The same over the 7-smooth M >= 2n - 1 that is cheapest; sh.g_max in points.
+bool mix_blue_fit(int prec, long long n, MixShape sh, MixPlan *p);
+// one-pass lines of a batch: 7-smooth n >= 2, and Bluestein of any n
 bool mix_plan(int prec, long long n, MixPlan *p);
 bool mix_blue_plan(int prec, long long n, MixPlan *p);
 hipError_t launch_mix(int prec, const MixArgs &a, hipStream_t s);

@@ -5,6 +5,7 @@
 #include <cmath>
 #include <mutex>
 #include <map>
+#include <tuple>
 
 namespace nfft {
 
@@ -45,14 +46,17 @@ float rcp_up_host(int d) { return (1.0f / (float)d) * 1.00000095367431640625f; }
 // Fill the steps of radices r[0..ns) (execution order) for G lines; false if
 // the lines do not fit the LDS.  Returns in *conflict the expected extra LDS
 // cycles factor of the first stage's writes.
-bool fill(MixPlan &p, int prec, int L, const int *r, int ns, bool blue, int G, double *conflict)
+bool fill(MixPlan &p, int prec, int L, const int *r, int ns, bool blue, int G, MixLanes lanes, size_t lds_max,
+          double *conflict)
 {
     const size_t cb = prec == 0 ? 8 : 16;
     const int banks = prec == 0 ? 32 : 16;  // elements per LDS row of banks
     p.L = L;
     p.stages = ns;
     p.steps = blue ? 2 * ns - 1 : ns;
+    p.blue = blue ? 1 : 0;
     p.G = G;
+    p.inG = rcp_up_host(G);
     *conflict = 1.0;
     for (int pads = 2; pads >= 0; pads--) {
         long long lp = p.steps > 1 ? L : 0;
@@ -68,6 +72,7 @@ bool fill(MixPlan &p, int prec, int L, const int *r, int ns, bool blue, int G, d
             t.ins = rcp_up_host(Ns);
             const int so = mid ? 1 : Ns, U = so * t.radix;
             t.pad = 0;
+            t.gfast = lanes == MIX_LANES_LINES || (lanes == MIX_LANES_TRANSPOSE && s > 0 && s + 1 == p.steps) ? 1 : 0;
             if (s + 1 < p.steps) {
                 if (so == 1) {
                     if (pads >= 1 && U % 2 == 0) t.pad = 1;
@@ -80,8 +85,15 @@ bool fill(MixPlan &p, int prec, int L, const int *r, int ns, bool blue, int G, d
             }
             Ns = mid ? t.radix : Ns * t.radix;
         }
+        if (lanes != MIX_LANES_POINTS && lp > 0) {
+            // neighbouring lanes on neighbouring lines: line distance such that
+            // G lines and the butterflies beside them fall on different banks
+            int w = 1;
+            while (w < G && w < banks) w <<= 1;
+            lp += (((long long)(banks / w) - lp) % banks + banks) % banks;
+        }
         p.lp = (int)lp;
-        if ((size_t)lp * G * cb <= kMixLds) return true;
+        if ((size_t)lp * G * cb <= lds_max) return true;
         *conflict = 1.0;
     }
     return false;
@@ -98,7 +110,7 @@ double cost_of(const MixPlan &p, int prec, double conflict)
     double c = 0;
     for (int s = 0; s < p.steps; s++) {
         const int total = p.G * p.st[s].nb, R = p.st[s].radix;
-        const bool mid = p.steps > p.stages && s == p.stages - 1;
+        const bool mid = p.blue && s == p.stages - 1;
         double waves = 0;
         for (int i = 0; i * p.nth < total; i++) waves += std::min(wv, (total - i * p.nth + 63) / 64);
         // a whole round of the workgroup takes as long as its busiest SIMD
@@ -113,14 +125,14 @@ double cost_of(const MixPlan &p, int prec, double conflict)
 struct Search {
     int prec, L;
     bool blue;
+    MixShape shape;
     double best = 1e300;
     MixPlan plan;
     int r[kMixMaxStages];
 
     void consider(int ns)
     {
-        const int tmax = prec == 0 ? mix_threads<float>() : mix_threads<double>();
-        const int gmax = L >= 4096 ? 1 : std::min(256, 8192 / L);
+        const int tmax = std::min(shape.nth_max, prec == 0 ? mix_threads<float>() : mix_threads<double>());
         // an odd radix first, if there is one: its writes need no padding
         int ord[kMixMaxStages];
         std::copy(r, r + ns, ord);
@@ -129,11 +141,11 @@ struct Search {
                 std::rotate(ord, ord + i, ord + i + 1);
                 break;
             }
-        for (int G = 1; G <= gmax; G = G < 8 ? G + 1 : G + G / 4) {
+        for (int G = shape.g_min; G <= shape.g_max; G = G < 8 ? G + 1 : G + G / 4) {
             MixPlan p;
             double conflict;
-            if (!fill(p, prec, L, ord, ns, blue, G, &conflict)) break;
-            for (int nth = 64; nth <= tmax; nth += 64) {
+            if (!fill(p, prec, L, ord, ns, blue, G, shape.lanes, shape.lds_max, &conflict)) break;
+            for (int nth = shape.nth_min; nth <= tmax; nth += 64) {
                 bool ok = true;
                 int most = 0;
                 for (int s = 0; s < ns && ok; s++) {
@@ -142,7 +154,7 @@ struct Search {
                     most = std::max(most, total);
                 }
                 if (!ok) continue;
-                if (nth - 64 >= most) break;  // only idle waves beyond
+                if (nth > shape.nth_min && nth - 64 >= most) break;  // only idle waves beyond
                 p.nth = nth;
                 const double c = cost_of(p, prec, conflict);
                 if (c < best) {
@@ -172,12 +184,13 @@ struct Found {
     double cost;
     MixPlan plan;
 };
+typedef std::tuple<int, int, int, int, int, int, int, int, size_t> Key;
 std::mutex g_mix_mu;
-std::map<long long, Found> g_mix_plans;  // by length, precision and form: schedules are searched once per process
+std::map<Key, Found> g_mix_plans;  // schedules are searched once per process
 
-const Found &find(int prec, int L, bool blue)
+const Found &find(int prec, int L, bool blue, const MixShape &sh)
 {
-    const long long key = ((long long)L << 2) | (prec << 1) | (blue ? 1 : 0);
+    const Key key(L, prec, blue ? 1 : 0, sh.g_min, sh.g_max, sh.nth_min, sh.nth_max, (int)sh.lanes, sh.lds_max);
     std::lock_guard<std::mutex> lk(g_mix_mu);
     auto it = g_mix_plans.find(key);
     if (it == g_mix_plans.end()) {
@@ -185,6 +198,7 @@ const Found &find(int prec, int L, bool blue)
         se.prec = prec;
         se.L = L;
         se.blue = blue;
+        se.shape = sh;
         // the fewest stages possible and one more
         for (int stages = 1, found = 0; stages <= kMixMaxStages && found < 2; stages++) {
             se.split(L, 0, 32, stages);
@@ -195,36 +209,59 @@ const Found &find(int prec, int L, bool blue)
     return it->second;
 }
 
+MixShape line_shape(int L)
+{
+    MixShape sh;
+    sh.g_max = L >= 4096 ? 1 : std::min(256, 8192 / L);
+    return sh;
+}
+
+bool smooth7(long long v)
+{
+    for (int q : {2, 3, 5, 7})
+        while (v % q == 0) v /= q;
+    return v == 1;
+}
+
 }  // namespace
 
 int mix_max(int prec) { return (int)(kMixLds / (prec == F32 ? 8 : 16)); }
 
-bool mix_plan(int prec, long long n, MixPlan *p)
+bool mix_fit(int prec, long long n, bool blue, const MixShape &sh, MixPlan *p, double *cost)
 {
-    if (n < 2 || n > mix_max(prec)) return false;
-    const Found &f = find(prec, (int)n, false);
+    if (n < 2 || n > mix_max(prec) || !smooth7(n)) return false;
+    const Found &f = find(prec, (int)n, blue, sh);
     if (f.cost >= 1e299) return false;
     *p = f.plan;
+    if (cost) *cost = f.cost;
     return true;
+}
+
+bool mix_plan(int prec, long long n, MixPlan *p) { return mix_fit(prec, n, false, line_shape((int)n), p); }
+
+bool mix_blue_fit(int prec, long long n, MixShape sh, MixPlan *p)
+{
+    // 7-smooth lengths from 2n - 1 up to a quarter more: the cheapest
+    const long long lo = 2 * n - 1, hi = std::min<long long>(mix_max(prec), lo + std::max<long long>(lo / 4, 4));
+    const int points = sh.g_max;
+    double best = 1e300;
+    for (long long m = lo; m <= hi; m++) {
+        MixPlan q;
+        double c;
+        sh.g_max = std::max<long long>(1, points / m);
+        if (mix_fit(prec, m, true, sh, &q, &c) && c < best) {
+            best = c;
+            *p = q;
+        }
+    }
+    return best < 1e299;
 }
 
 bool mix_blue_plan(int prec, long long n, MixPlan *p)
 {
-    // 7-smooth lengths from 2n - 1 up to a quarter more: the cheapest
-    const long long lo = 2 * n - 1, hi = std::min<long long>(mix_max(prec), lo + std::max<long long>(lo / 4, 4));
-    double best = 1e300;
-    for (long long m = lo; m <= hi; m++) {
-        long long v = m;
-        for (int q : {2, 3, 5, 7})
-            while (v % q == 0) v /= q;
-        if (v != 1) continue;
-        const Found &f = find(prec, (int)m, true);
-        if (f.cost < best) {
-            best = f.cost;
-            *p = f.plan;
-        }
-    }
-    return best < 1e299;
+    MixShape sh;
+    sh.g_max = 2 * n - 1 >= 4096 ? 4096 : 8192;  // points per workgroup
+    return mix_blue_fit(prec, n, sh, p);
 }
 
 template <typename T, bool BLUE> static hipError_t mix_go(const MixArgs &a0, hipStream_t s)
@@ -252,7 +289,8 @@ template <typename T, bool BLUE> static hipError_t mix_go(const MixArgs &a0, hip
 
 hipError_t launch_mix(int prec, const MixArgs &a, hipStream_t s)
 {
-    const bool blue = a.pl.steps > a.pl.stages || a.chirp;
+    const bool blue = a.pl.blue != 0;
+    if (blue && (!a.chirp || !a.H)) return hipErrorInvalidValue;
     const int slot = prof_on() ? prof_begin(s) : -1;
     const hipError_t e = prec == F32 ? (blue ? mix_go<float, true>(a, s) : mix_go<float, false>(a, s))
                                      : (blue ? mix_go<double, true>(a, s) : mix_go<double, false>(a, s));

@@ -38,11 +38,14 @@ constexpr size_t kMixLds = 160 * 1024;
 struct MixStep {
     int radix, pad, nb, ns, q;
     float inb, ins;
+    int gfast;  // neighbouring lanes take neighbouring lines (else neighbouring butterflies)
 };
 struct MixPlan {
     int L = 0;
     int stages = 0, steps = 0;  // steps: stages, or 2 stages - 1 for Bluestein
+    int blue = 0;               // Bluestein: step stages - 1 is the middle one
     int G = 1;                  // lines per workgroup
+    float inG = 1.0f;           // its reciprocal for fdiv
     int nth = 0;                // threads per workgroup
     int lp = 0;                 // LDS points per line, padding included
     MixStep st[kMixMaxSteps];
@@ -53,6 +56,14 @@ struct MixPlan {
 // 1024-thread workgroup; FP64: 128 under the 256 of 512 threads).
 template <typename T> __host__ __device__ constexpr int mix_threads() { return sizeof(T) == 4 ? 1024 : 512; }
 __host__ __device__ constexpr int mix_reps(int R) { return 32 / R; }
+
+// Buffer view of `bytes` bytes: loads beyond them return zero, stores beyond
+// them are dropped, and kMixNone is beyond them.
+constexpr uint32_t kMixNone = 0xfffffff0u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mix_rsrc(const void *base, uint32_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, 0x00020000);
+}
 
 // w^t, t < R, applied to v: entry e of the table is e^{-2 pi i e / L}, w the
 // entry `e`.  Powers t = Q h + l from the entries of l and Q h.
@@ -75,15 +86,17 @@ __device__ __forceinline__ void mix_twiddle(Cx<T> (&v)[R], __amdgpu_buffer_rsrc_
     }
 }
 
-// One step of all the lines of a workgroup.  Every thread must call it.
-template <typename T, int R, bool BLUE, class IO>
-__device__ __forceinline__ void mix_step(const MixPlan &pl, int s, Cx<T> *lds, __amdgpu_buffer_rsrc_t tw, const IO &io)
+// One step of all the lines of a workgroup.  Every thread must call it.  PL:
+// MixPlan, in any address space (kernel arguments or constant memory).
+template <typename T, int R, bool BLUE, class PL, class IO>
+__device__ __forceinline__ void mix_step(const PL &pl, int s, Cx<T> *lds, __amdgpu_buffer_rsrc_t tw, const IO &io)
 {
     using C = Cx<T>;
     constexpr int B = mix_reps(R);
-    const MixStep st = pl.st[s];
+    const auto &ps = pl.st[s];
+    const MixStep st{ps.radix, ps.pad, ps.nb, ps.ns, ps.q, ps.inb, ps.ins, ps.gfast};
     const int total = pl.G * st.nb, nth = blockDim.x;
-    const bool first = s == 0, last = s + 1 == pl.steps, mid = BLUE && s + 1 == pl.stages;
+    const bool first = s == 0, last = s + 1 == pl.steps, mid = BLUE && pl.blue && s + 1 == pl.stages;
     const int up = st.ns + (first ? 0 : pl.st[s - 1].pad);  // padded input blocks
     const int rs = st.q * up;                               // LDS distance of points L / R apart
     const int so = mid ? 1 : st.ns;                         // output distance of a butterfly's points
@@ -97,7 +110,14 @@ __device__ __forceinline__ void mix_step(const MixPlan &pl, int s, Cx<T> *lds, _
             if (i > 0 && i * nth >= total) break;  // uniform
             int idx = threadIdx.x + i * nth;
             if (i > 0 && idx >= total) idx = total - 1;  // not stored
-            const int g = fdiv(idx, st.inb), j = idx - __mul24(g, st.nb);
+            int g, j;
+            if (st.gfast) {
+                j = fdiv(idx, pl.inG);
+                g = idx - __mul24(j, pl.G);
+            } else {
+                g = fdiv(idx, st.inb);
+                j = idx - __mul24(g, st.nb);
+            }
             gg[i] = g;
             int jq = j, k = 0;
             if (first) {
@@ -113,7 +133,7 @@ __device__ __forceinline__ void mix_step(const MixPlan &pl, int s, Cx<T> *lds, _
             dft_any<R, -1>(v[i]);
             if constexpr (BLUE) {
                 if (mid) {
-                    io.template middle<R>(v[i], j, st.ns);
+                    io.template middle<R>(v[i], g, j, st.ns);
                     dft_any<R, -1>(v[i]);
                     jq = j;
                     k = 0;
@@ -144,8 +164,8 @@ __device__ __forceinline__ void mix_step(const MixPlan &pl, int s, Cx<T> *lds, _
     X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(14) X(15) X(16) X(18) X(20) X(21) X(24) X(25) X(27)   \
     X(28) X(30) X(32)
 
-template <typename T, bool BLUE, class IO>
-__device__ __forceinline__ void mix_lines(const MixPlan &pl, Cx<T> *lds, const void *tw, const IO &io)
+template <typename T, bool BLUE, class PL, class IO>
+__device__ __forceinline__ void mix_lines(const PL &pl, Cx<T> *lds, const void *tw, const IO &io)
 {
     const auto rt = buf_rsrc(tw);
     for (int s = 0; s < pl.steps; s++) {
@@ -157,36 +177,33 @@ __device__ __forceinline__ void mix_lines(const MixPlan &pl, Cx<T> *lds, const v
     }
 }
 
-// Contiguous lines in global memory.  BLUE: n < L points per line, times the
-// chirp on both sides, the filter spectrum between the two transforms; the
-// inverse of the convolution is conj(FFT(conj(.))), folded into the products.
-template <typename T, bool BLUE> struct MixIoLine {
+// Lines in global memory, points contiguous.  BLUE: n < L points per line,
+// times the chirp on both sides, the filter spectrum between the two
+// transforms; the inverse of the convolution is conj(FFT(conj(.))), folded
+// into the products.  OFFS gives the byte offset of a line from the base of
+// `in` / `out`.
+template <typename T, bool BLUE, class OFFS> struct MixIoLine {
     using C = Cx<T>;
-    __amdgpu_buffer_rsrc_t in, out, chirp, H;
-    uint32_t idist, odist;  // bytes between lines
-    int glast;              // last line of this workgroup
-    int n;                  // BLUE: points per line
-    T sg, sc;               // sign of the imaginary parts (-1: inverse), output scale
+    __amdgpu_buffer_rsrc_t in, out, chirp, H;  // in, out, chirp end with their last point
+    OFFS offs;
+    int glast;  // last line of this workgroup
+    int n;      // BLUE: points per line
+    T sg, sc;   // sign of the imaginary parts (-1: inverse), output scale
 
     template <int R> __device__ __forceinline__ void load(C (&v)[R], int g, int j, int nb) const
     {
-        const uint32_t off = (uint32_t)min(g, glast) * idist;
+        const uint32_t off = offs.in(min(g, glast));
+        const uint32_t o = off + (uint32_t)j * (uint32_t)sizeof(C);
+        const uint32_t step = (uint32_t)nb * (uint32_t)sizeof(C);
         if constexpr (BLUE) {
 #pragma unroll
             for (int t = 0; t < R; t++) {
                 const int p = j + t * nb;
-                const uint32_t pb = p < n ? (uint32_t)p * (uint32_t)sizeof(C) : 0u;
-                if (t * nb < n) {  // uniform
-                    C x = buf_ld<C>(in, off + pb, 0);
-                    x.y *= sg;
-                    x = cmul(x, buf_ld<C>(chirp, pb, 0));
-                    v[t] = p < n ? x : cmk<C>((T)0, (T)0);
-                } else {
-                    v[t] = cmk<C>((T)0, (T)0);
-                }
+                C x = buf_ld<C>(in, p < n ? o + (uint32_t)t * step : kMixNone, 0);
+                x.y *= sg;
+                v[t] = cmul(x, buf_ld<C>(chirp, (uint32_t)p * (uint32_t)sizeof(C), 0));
             }
         } else {
-            const uint32_t o = off + (uint32_t)j * (uint32_t)sizeof(C), step = (uint32_t)nb * (uint32_t)sizeof(C);
 #pragma unroll
             for (int t = 0; t < R; t++) v[t] = buf_ld<C>(in, o, (uint32_t)t * step);
 #pragma unroll
@@ -194,7 +211,7 @@ template <typename T, bool BLUE> struct MixIoLine {
         }
     }
     // v (points j + t ns of the spectrum) -> conj(v H)
-    template <int R> __device__ __forceinline__ void middle(C (&v)[R], int j, int ns) const
+    template <int R> __device__ __forceinline__ void middle(C (&v)[R], int, int j, int ns) const
     {
 #pragma unroll
         for (int t = 0; t < R; t++)
@@ -204,22 +221,34 @@ template <typename T, bool BLUE> struct MixIoLine {
     template <int R> __device__ __forceinline__ void store(const C (&v)[R], int g, int k, int ns) const
     {
         if (g > glast) return;
-        const uint32_t o = (uint32_t)g * odist + (uint32_t)k * (uint32_t)sizeof(C);
+        const uint32_t o = offs.out(g) + (uint32_t)k * (uint32_t)sizeof(C);
         const uint32_t step = (uint32_t)ns * (uint32_t)sizeof(C);
         const T sy = sc * sg;
 #pragma unroll
         for (int t = 0; t < R; t++) {
             if constexpr (BLUE) {
                 const int p = k + t * ns;
-                if (p < n) {
-                    const C z = cmulc(buf_ld<C>(chirp, (uint32_t)p * (uint32_t)sizeof(C), 0), v[t]);
-                    buf_st<C>(out, o, (uint32_t)t * step, cmk<C>(z.x * sc, z.y * sy));
-                }
+                const C z = cmulc(buf_ld<C>(chirp, (uint32_t)p * (uint32_t)sizeof(C), 0), v[t]);
+                buf_st<C>(out, p < n ? o + (uint32_t)t * step : kMixNone, 0, cmk<C>(z.x * sc, z.y * sy));
             } else {
                 buf_st<C>(out, o, (uint32_t)t * step, cmk<C>(v[t].x * sc, v[t].y * sy));
             }
         }
     }
+};
+
+// lines at a fixed distance
+struct MixDist {
+    uint32_t idist, odist;  // bytes
+    __device__ __forceinline__ uint32_t in(int g) const { return (uint32_t)g * idist; }
+    __device__ __forceinline__ uint32_t out(int g) const { return (uint32_t)g * odist; }
+};
+// lines at offsets of their own, the first one the lowest
+template <typename C> struct MixOffs {
+    const long long *offs;  // elements
+    long long base;
+    __device__ __forceinline__ uint32_t in(int g) const { return (uint32_t)(offs[g] - base) * (uint32_t)sizeof(C); }
+    __device__ __forceinline__ uint32_t out(int g) const { return in(g); }
 };
 
 struct MixArgs {
@@ -248,18 +277,227 @@ template <typename T, bool BLUE> __global__ void __launch_bounds__(mix_threads<T
     extern __shared__ char smem[];
     const long long l0 = (long long)blockIdx.x * a.pl.G;
     const long long rem = a.nlines - l0;
-    MixIoLine<T, BLUE> io;
-    io.in = buf_rsrc((const C *)a.in + l0 * a.in_dist);
-    io.out = buf_rsrc((C *)a.out + l0 * a.out_dist);
-    io.idist = (uint32_t)a.in_dist * (uint32_t)sizeof(C);
-    io.odist = (uint32_t)a.out_dist * (uint32_t)sizeof(C);
-    io.glast = (int)(rem < a.pl.G ? rem : a.pl.G) - 1;
-    io.n = a.n;
-    io.sg = a.inverse ? (T)-1 : (T)1;
-    io.sc = (T)a.scale;
-    io.chirp = buf_rsrc(a.chirp);
-    io.H = buf_rsrc(a.H);
+    const int cnt = (int)(rem < a.pl.G ? rem : a.pl.G);
+    const MixDist d{(uint32_t)a.in_dist * (uint32_t)sizeof(C), (uint32_t)a.out_dist * (uint32_t)sizeof(C)};
+    const uint32_t len = (uint32_t)(BLUE ? a.n : a.pl.L) * (uint32_t)sizeof(C);
+    const MixIoLine<T, BLUE, MixDist> io{mix_rsrc((const C *)a.in + l0 * a.in_dist, (uint32_t)(cnt - 1) * d.idist + len),
+                                         mix_rsrc((C *)a.out + l0 * a.out_dist, (uint32_t)(cnt - 1) * d.odist + len),
+                                         mix_rsrc(a.chirp, len),
+                                         buf_rsrc(a.H),
+                                         d,
+                                         cnt - 1,
+                                         a.n,
+                                         a.inverse ? (T)-1 : (T)1,
+                                         (T)a.scale};
     mix_lines<T, BLUE>(a.pl, (C *)smem, a.tw, io);
+}
+
+// ---------------------------------------------------------------------------
+// Tiles: G lines of an array with any line and point strides, the passes of
+// transforms longer than one workgroup.
+//   N = N1 x N2 (both 7-smooth), element n1 N2 + n2:
+//     phase 1, columns [c0, c0 + G): FFT_N1, times w_N^{k1 c}, to scratch
+//     phase 2, rows of the scratch: FFT_N2, stored transposed (k1 + N1 k2)
+//   Bluestein over M = M1 x M2 >= 2N - 1 (both 7-smooth):
+//     phase 1, columns: times the chirp, FFT_M1, times w_M^{k1 c}
+//     phase 2, rows: FFT_M2, times the filter, conjugate, FFT_M2, times
+//              w_M^{k1 c}, in place: the conjugate of the inverse's first half
+//     phase 3, columns: FFT_M1, conjugate, times the chirp
+// ---------------------------------------------------------------------------
+enum { MIX_CHIRP_IN = 1, MIX_CHIRP_OUT = 2, MIX_TW = 4, MIX_HEAD = 8, MIX_TAIL = 16 };
+struct MixPhase {
+    MixPlan pl;
+    const void *tw;            // L entries e^{-2 pi i q / L}
+    Tw2 tw2;                   // MIX_TW: two-level table of the whole length
+    const void *chirp, *H;     // chirp entries below nv; filter in the layout of the rows
+    int ig, ip, og, op;        // element distances of lines and points, input and output
+    int lines;                 // lines of the phase (tiles of pl.G)
+    int nv;                    // Bluestein: points of the transform
+    int flags;                 // MIX_HEAD / MIX_TAIL: reads the input / writes the output of the transform
+};
+
+// Phases and items in constant memory: read through the scalar cache, and not
+// again after every store.
+typedef const MixPhase __attribute__((address_space(4))) MixPhaseK;
+
+// v[t] *= w^{e0 + t es} (w = e^{-2 pi i / N}): two table entries and chains
+// of FP64 products (FP32: two chains, which leaves the registers of radix 32
+// below 128; FP64: four, at most nine products deep).
+template <int R, typename C>
+__device__ __forceinline__ void mix_tw2(C (&v)[R], const Tw2 &tab, uint32_t e0, uint32_t es)
+{
+    constexpr int Q = sizeof(v[0].x) == 4 ? 2 : 4;
+    double2 st = tw2_get(tab, es), b[Q];
+    b[0] = tw2_get(tab, e0);
+    b[1] = dmul(b[0], st);
+    st = dmul(st, st);
+    if constexpr (Q == 4) {
+        b[2] = dmul(b[0], st);
+        b[3] = dmul(b[1], st);
+        st = dmul(st, st);
+    }
+#pragma unroll
+    for (int t = 0; t < R; t++) {
+        v[t] = ctw64<-1>(v[t], b[t % Q]);
+        if (t + Q < R) b[t % Q] = dmul(b[t % Q], st);
+    }
+}
+
+template <typename T> struct MixIoTile {
+    using C = Cx<T>;
+    MixPhaseK &ph;
+    __amdgpu_buffer_rsrc_t in, out, chirp, H;  // in / out / H at line c0 (chirped sides: at the transform)
+    int c0, glast;
+    T sg, sc;                                  // inverse: -1 and the scale of the result
+
+    template <int R> __device__ __forceinline__ void load(C (&v)[R], int g, int j, int nb) const
+    {
+        const int gc = min(g, glast), step = nb * ph.ip;
+        if (ph.flags & MIX_CHIRP_IN) {  // `in` and `chirp` end with point nv - 1
+            const uint32_t o = (uint32_t)((c0 + gc) * ph.ig + j * ph.ip) * (uint32_t)sizeof(C);
+#pragma unroll
+            for (int t = 0; t < R; t++) {
+                C x = buf_ld<C>(in, o + (uint32_t)(t * step) * (uint32_t)sizeof(C), 0);
+                x.y *= sg;
+                v[t] = cmul(x, buf_ld<C>(chirp, o + (uint32_t)(t * step) * (uint32_t)sizeof(C), 0));
+            }
+            return;
+        }
+        const uint32_t o = (uint32_t)(gc * ph.ig + j * ph.ip) * (uint32_t)sizeof(C);
+#pragma unroll
+        for (int t = 0; t < R; t++) v[t] = buf_ld<C>(in, o, (uint32_t)(t * step) * (uint32_t)sizeof(C));
+        if (ph.flags & MIX_HEAD) {
+#pragma unroll
+            for (int t = 0; t < R; t++) v[t].y *= sg;
+        }
+    }
+    template <int R> __device__ __forceinline__ void middle(C (&v)[R], int g, int j, int ns) const
+    {
+        const uint32_t o = (uint32_t)(min(g, glast) * ph.ig + j) * (uint32_t)sizeof(C);
+#pragma unroll
+        for (int t = 0; t < R; t++)
+            v[t] = cconj(cmul(v[t], buf_ld<C>(H, o, (uint32_t)(t * ns) * (uint32_t)sizeof(C))));
+    }
+    template <int R> __device__ __forceinline__ void store(C (&v)[R], int g, int k, int ns) const
+    {
+        if (g > glast) return;
+        if (ph.flags & MIX_TW) mix_tw2<R>(v, Tw2{ph.tw2.hi, ph.tw2.lo, ph.tw2.sh, ph.tw2.mask}, (uint32_t)(c0 + g) * (uint32_t)k, (uint32_t)(c0 + g) * (uint32_t)ns);
+        const int step = ns * ph.op;
+        if (ph.flags & MIX_CHIRP_OUT) {  // `out` and `chirp` end with point nv - 1
+            const uint32_t o = (uint32_t)((c0 + g) * ph.og + k * ph.op) * (uint32_t)sizeof(C);
+            const T sy = sc * sg;
+#pragma unroll
+            for (int t = 0; t < R; t++) {
+                const uint32_t ot = o + (uint32_t)(t * step) * (uint32_t)sizeof(C);
+                const C z = cmulc(buf_ld<C>(chirp, ot, 0), v[t]);
+                buf_st<C>(out, ot, 0, cmk<C>(z.x * sc, z.y * sy));
+            }
+            return;
+        }
+        const uint32_t o = (uint32_t)(g * ph.og + k * ph.op) * (uint32_t)sizeof(C);
+        if (ph.flags & MIX_TAIL) {
+            const T sy = sc * sg;
+#pragma unroll
+            for (int t = 0; t < R; t++) v[t] = cmk<C>(v[t].x * sc, v[t].y * sy);
+        }
+#pragma unroll
+        for (int t = 0; t < R; t++) buf_st<C>(out, o, (uint32_t)(t * step) * (uint32_t)sizeof(C), v[t]);
+    }
+};
+
+// Lines [c0, c0 + cnt) of phase `ph` of one transform (cnt <= ph.pl.G); src
+// and dst at the transform (or its scratch).
+template <typename T>
+__device__ __forceinline__ void mix_tile(MixPhaseK &ph, const Cx<T> *src, Cx<T> *dst, int c0, int cnt, int inverse,
+                                         T scale, Cx<T> *lds)
+{
+    using C = Cx<T>;
+    const uint32_t nb = (uint32_t)ph.nv * (uint32_t)sizeof(C);
+    MixIoTile<T> io{ph,
+                    ph.flags & MIX_CHIRP_IN ? mix_rsrc(src, nb) : buf_rsrc(src + (long long)c0 * ph.ig),
+                    ph.flags & MIX_CHIRP_OUT ? mix_rsrc(dst, nb) : buf_rsrc(dst + (long long)c0 * ph.og),
+                    mix_rsrc(ph.chirp, nb),
+                    buf_rsrc((const C *)ph.H + (long long)c0 * ph.ig),
+                    c0,
+                    cnt - 1,
+                    inverse ? (T)-1 : (T)1,
+                    scale};
+    mix_lines<T, true>(ph.pl, lds, ph.tw, io);
+}
+
+// ---------------------------------------------------------------------------
+// Ragged batches (nfft_ragged.hip): one launch per phase over a list of
+// items, an item a tile of one long transform, or a group of same-size short
+// transforms at any offsets.
+// ---------------------------------------------------------------------------
+struct RagItem {
+    int phase;           // index of its MixPhase
+    int c0, cnt;         // tiles: lines [c0, c0 + cnt); groups: cnt transforms
+    int first;           // groups: first entry of the offset list
+    long long src, dst;  // tiles: element offsets of the transform (or its scratch)
+    int n;               // transform length
+    int pow2;            // inverse not scaled
+    int in_place;        // tiles: written back to the scratch
+};
+typedef const RagItem __attribute__((address_space(4))) RagItemK;
+struct RagArgs {
+    const void *in;
+    void *out;
+    const MixPhase *phases;
+    const RagItem *items;
+    int nitems;
+    int inverse;
+    const long long *offs;  // groups: element offset of each transform
+    void *alt;              // tiles: scratch, the output of in-place items
+};
+
+template <typename T> __device__ __forceinline__ T rag_scale(const RagArgs &a, RagItemK &it)
+{
+    return a.inverse && !it.pow2 ? (T)1 / (T)it.n : (T)1;
+}
+
+// Groups of short transforms.
+template <typename T, bool BLUE> __global__ void __launch_bounds__(mix_threads<T>()) k_rag_group(RagArgs a)
+{
+    using C = Cx<T>;
+    extern __shared__ char smem[];
+    RagItemK &it = ((RagItemK *)a.items)[blockIdx.x];
+    MixPhaseK &ph = ((MixPhaseK *)a.phases)[it.phase];
+    const long long *offs = a.offs + it.first;
+    const long long base = offs[0];
+    const C *in = (const C *)a.in + base;
+    C *out = (C *)a.out + base;
+    if (ph.pl.steps == 0) {  // one-point transforms
+        for (int i = threadIdx.x; i < it.cnt; i += blockDim.x) out[offs[i] - base] = in[offs[i] - base];
+        return;
+    }
+    const uint32_t len = (uint32_t)it.n * (uint32_t)sizeof(C);
+    const uint32_t end = (uint32_t)(offs[it.cnt - 1] - base) * (uint32_t)sizeof(C) + len;
+    const MixIoLine<T, BLUE, MixOffs<C>> io{mix_rsrc(in, end), mix_rsrc(out, end), mix_rsrc(ph.chirp, len),
+                                            buf_rsrc(ph.H),    MixOffs<C>{offs, base}, it.cnt - 1,
+                                            it.n,              a.inverse ? (T)-1 : (T)1, rag_scale<T>(a, it)};
+    mix_lines<T, BLUE>(ph.pl, (C *)smem, ph.tw, io);
+}
+
+// Tiles of long transforms.
+constexpr int kTileThreads = 256;
+template <typename T> __global__ void __launch_bounds__(kTileThreads, (sizeof(T) == 4 ? 4 : 2)) k_rag_tile(RagArgs a)
+{
+    using C = Cx<T>;
+    extern __shared__ char smem[];
+    // kTileRun neighbouring items go to one XCD (workgroup b runs on XCD b mod
+    // 8): tiles whose edges share 128-byte lines then share an L2
+    constexpr int kTileRun = 16;
+    const int full = a.nitems / (8 * kTileRun) * (8 * kTileRun);
+    for (int b = blockIdx.x; b < a.nitems; b += gridDim.x) {
+        const int w = b % (8 * kTileRun);
+        const int i = b < full ? b - w + (w & 7) * kTileRun + (w >> 3) : b;
+        RagItemK &it = ((RagItemK *)a.items)[i];
+        MixPhaseK &ph = ((MixPhaseK *)a.phases)[it.phase];
+        mix_tile<T>(ph, (const C *)a.in + it.src, (C *)(it.in_place ? a.alt : a.out) + it.dst, it.c0, it.cnt, a.inverse, rag_scale<T>(a, it),
+                    (C *)smem);
+        __syncthreads();  // the next tile overwrites the buffer
+    }
 }
 
 }  // namespace nfft
