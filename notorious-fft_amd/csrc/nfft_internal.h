@@ -14,6 +14,7 @@
 #include "nfft_kernels_smooth.h"
 #include "nfft_kernels_mix.h"
 #include "nfft_kernels_rt.h"
+#include "nfft_kernels_tcol.h"
 
 namespace nfft {
 
@@ -108,6 +109,11 @@ hipError_t launch_r2c(int prec, int L, const RtArgs &a, hipStream_t s);
 hipError_t launch_c2r(int prec, int L, const RtArgs &a, hipStream_t s);
 hipError_t launch_t23(int prec, int L, int op, const RtArgs &a, hipStream_t s);
 hipError_t launch_t4(int prec, int L, int op, const RtArgs &a, hipStream_t s);
+// DCT / DST down columns of N points (nfft_kernels_tcol.h); with query, only
+// whether a kernel takes these arguments
+template <typename T> hipError_t tcol_impl(int N, int op, const TrigColArgs &a, hipStream_t s, bool query);
+extern template hipError_t tcol_impl<float>(int, int, const TrigColArgs &, hipStream_t, bool);
+extern template hipError_t tcol_impl<double>(int, int, const TrigColArgs &, hipStream_t, bool);
 
 // persistent four-step (nfft_k_persist.hip): shape `variant` (0 = default)
 // of a power-of-two length n; false if that length/variant is not built.

@@ -1449,6 +1449,27 @@ static double axis_inv_scale(int norm, int n)
     return is_pow2(n) ? 1.0 : 1.0 / n;  // reference behaviour
 }
 
+// The strided form of a trig axis of n points over rows of B reals in `outer`
+// arrays: every length that has a column kernel (up to 4096 points).  Longer
+// axes and arrays beyond 32-bit offsets are transposed (dist stays 0).  False
+// if a table cannot be made.
+static bool trig_col(TrigColArgs &c, int prec, int t4, int n, long long outer, long long B)
+{
+    TrigColArgs a{};
+    a.ncols = B / 2;
+    a.total = outer * a.ncols;
+    a.dist = (long long)n * a.ncols;
+    a.scale = a.w0 = 1.0;
+    if ((prec == F32 ? tcol_impl<float>(n, 0, a, nullptr, true) : tcol_impl<double>(n, 0, a, nullptr, true)) != hipSuccess)
+        return true;
+    a.tw = stage_table(prec, t4 ? n / 2 : n);
+    a.t1 = t4 ? phase_table(prec, n / 2, 1, 0, 2LL * n) : phase_table(prec, n, 1, 0, 4LL * n);
+    a.t2 = t4 ? phase_table(prec, n, 2, 1, 8LL * n) : a.t1;
+    if (!a.tw || !a.t1 || !a.t2) return false;
+    c = a;
+    return true;
+}
+
 bool nfft_plan::init(int kind_, int prec_, int d_, const int *dims_, long long batch_, int norm_)
 {
     kind = kind_;
@@ -1522,14 +1543,21 @@ bool nfft_plan::init(int kind_, int prec_, int d_, const int *dims_, long long b
         while (n_active > 1 && dims[n_active - 1] == 1) n_active--;
         dsc = std::string(t4 ? "dct4/dst4 " : "dct2/3 dst2/3 ") + std::to_string(P) +
               (d > 1 ? " separable" : (tax[0].single ? " single-pass" : " multi-pass"));
+        tcol.assign(d, TrigColArgs{});
+        for (int i = 0; i < n_active; i++) {
+            const long long B = prod(dims, i + 1, d);
+            if (B == 1) continue;
+            if (dims[i] > 1 && !trig_col(tcol[i], prec, t4, dims[i], batch * P / (dims[i] * B), B)) return false;
+            if (tcol[i].dist == 0) trig_full = batch * P;
+        }
         long long e_max = 0;
         for (int i = 0; i < n_active; i++) {
+            if (tcol[i].dist) continue;
             const long long lines_i = batch * P / dims[i];
             e_max = std::max(e_max, chunk_lines(lines_i, tax[i].scratch_per_line, rb) * tax[i].scratch_per_line);
         }
         // in reals: full-array transposes (2 copies) + the engine scratch (complex)
-        full = n_active > 1 || d > 1 ? 2 * batch * P : 0;
-        work_bytes = (size_t)full * rb + (size_t)e_max * cb;
+        work_bytes = (size_t)(2 * trig_full) * rb + (size_t)e_max * cb;
     }
     desc = dsc;
     if (work_bytes) {
@@ -1593,6 +1621,14 @@ static hipError_t dft_nd(const nfft_plan &p, const std::vector<C2C> &ax, const s
     return hipSuccess;
 }
 
+static hipError_t launch_tcol(int prec, int n, int top, const TrigColArgs &a, hipStream_t s)
+{
+    const int slot = prof_on() ? prof_begin(s) : -1;
+    const hipError_t e = prec == F32 ? tcol_impl<float>(n, top, a, s, false) : tcol_impl<double>(n, top, a, s, false);
+    if (slot >= 0) prof_end(slot, s, "k_trig_col", prec, n, 2.0 * (double)a.total * n * (double)cx_bytes(prec));
+    return e;
+}
+
 // trig transform along axis i of a row-major (outer, dims...) real array.
 static hipError_t trig_axis(const nfft_plan &p, int i, int op, const void *in, void *out, double w0, void *scr,
                             hipStream_t s)
@@ -1600,11 +1636,17 @@ static hipError_t trig_axis(const nfft_plan &p, int i, int op, const void *in, v
     const size_t rb = re_bytes(p.prec);
     const int n = p.dims[i];
     const long long A = p.batch * prod(p.dims, 0, i), B = prod(p.dims, i + 1, p.d);
-    const long long tot = A * n * B;
-    void *full0 = scr, *full1 = (char *)scr + (size_t)tot * rb;
-    void *eng = (char *)scr + (size_t)(p.d > 1 || p.n_active > 1 ? 2 * tot : 0) * rb;
-    const long long eng_elems =
-        (long long)((p.work_bytes - (size_t)(p.d > 1 || p.n_active > 1 ? 2 * tot : 0) * rb) / cx_bytes(p.prec));
+    const long long full = 2 * p.trig_full;
+    void *full0 = scr, *full1 = (char *)scr + (size_t)p.trig_full * rb;
+    void *eng = (char *)scr + (size_t)full * rb;
+    const long long eng_elems = (long long)((p.work_bytes - (size_t)full * rb) / cx_bytes(p.prec));
+    if (p.tcol[i].dist) {
+        TrigColArgs a = p.tcol[i];
+        a.in = in;
+        a.out = out;
+        a.w0 = w0;
+        return launch_tcol(p.prec, n, op - NFFT_OP_DCT2, a, s);
+    }
     if (B == 1) return p.tax[i].run(op, in, out, A, n, n, 1.0, w0, eng, eng_elems, s);
     hipError_t e = launch_transpose(in, full0, A, n, B, (int)rb, s);
     if (e != hipSuccess) return e;

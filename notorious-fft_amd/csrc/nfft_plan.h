@@ -60,6 +60,8 @@ struct nfft_plan {
     std::vector<nfft::C2C> ax;        // DFT axes (REALDFT: leading axes)
     nfft::R2C real;                   // REALDFT last axis
     std::vector<nfft::Trig> tax;      // trig axes
+    std::vector<nfft::TrigColArgs> tcol;  // their strided form (dist 0: none, the axis is transposed)
+    long long trig_full = 0;          // reals of one transposed copy (0: no axis is transposed)
     void *work = nullptr;
     size_t work_bytes = 0;
     std::string desc;
