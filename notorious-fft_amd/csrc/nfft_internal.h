@@ -15,6 +15,7 @@
 #include "nfft_kernels_mix.h"
 #include "nfft_kernels_rt.h"
 #include "nfft_kernels_tcol.h"
+#include "nfft_kernels_c2r.h"
 
 namespace nfft {
 
@@ -105,6 +106,10 @@ hipError_t launch_col(int prec, int L, int dir, int mode, const ColArgs &a, hipS
 hipError_t launch_rowT(int prec, int L, int dir, const RowTArgs &a, hipStream_t s);
 hipError_t launch_blue_row(int prec, int L, const BlueRowArgs &a, hipStream_t s);
 hipError_t launch_rowT_r2c(int prec, int L, const RowR2CArgs &a, hipStream_t s);
+// packing column pass of a long invrealdft over L x S points; twid: with the
+// inter-pass twiddle
+bool col_pack_supported(int prec, int L, int S);
+hipError_t launch_col_pack(int prec, int L, bool twid, const ColPackArgs &a, hipStream_t s);
 hipError_t launch_r2c(int prec, int L, const RtArgs &a, hipStream_t s);
 hipError_t launch_c2r(int prec, int L, const RtArgs &a, hipStream_t s);
 hipError_t launch_t23(int prec, int L, int op, const RtArgs &a, hipStream_t s);

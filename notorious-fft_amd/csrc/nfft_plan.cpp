@@ -1200,6 +1200,9 @@ bool R2C::init(int N_, int prec_)
     if (!built) return false;
     r2c_lpb = env_int("NFFT_R2C_LPB", lg2r && inner.n2 == (1 << lg2r) ? 2 * rowT_lpb_rt(prec, 1 << lg2r) : 0);
     fused = inner.algo == ALG_FOUR && !inner.pctr && (inner.n1 % 2) == 0 && env_int("NFFT_R2C_FUSE", 1) != 0;
+    packed = fused && !inner.xctr && col_pack_supported(prec, inner.n1, inner.n2);
+    if (packed) ptw = phase_table(F64, L / 16, 1, 0, N);
+    if (packed && !ptw) return false;
     scratch_per_line = L + inner.scratch_per_line;
     return true;
 }
@@ -1277,8 +1280,32 @@ hipError_t R2C::inv(const void *in, void *out, long long nlines, long long in_di
     void *isc = (char *)scratch + (size_t)chunk * L * cb;
     for (long long l0 = 0; l0 < nlines; l0 += chunk) {
         const long long cnt = std::min(chunk, nlines - l0);
+        hipError_t e;
+        if (packed) {
+            // pack + column pass into Z, then the rows
+            ColPackArgs p{};
+            p.c.in = (const char *)in + (size_t)l0 * in_dist * cb;
+            p.c.out = Z;
+            p.c.ncols = inner.n2;
+            p.c.S = inner.n2;
+            p.c.in_dist = in_dist;
+            p.c.out_dist = L;
+            p.c.ntrans = cnt;
+            p.c.tw = inner.tw_a;
+            p.c.tw2 = inner.tw2;
+            p.w = ptw;
+            p.half = half;
+            e = launch_col_pack(prec, inner.n1, !inner.row_twin, p, s);
+            if (e != hipSuccess) return e;
+            RowTArgs r{Z, (char *)out + (size_t)l0 * out_dist * rb, inner.n1, L, out_dist / 2, cnt, inner.tw_b, scale,
+                       inner.row_lpb, inner.row_pf};
+            if (inner.row_twin) r.twf = inner.tw2f;
+            e = launch_rowT(prec, inner.n2, 1, r, s);
+            if (e != hipSuccess) return e;
+            continue;
+        }
         EwArgs a{(const char *)in + (size_t)l0 * in_dist * cb, Z, cnt, in_dist, L, L, rtw, nullptr, 1.0, 1.0, half, 0};
-        hipError_t e = launch_ew(prec, EW_PACK, a, L, s);
+        e = launch_ew(prec, EW_PACK, a, L, s);
         if (e != hipSuccess) return e;
         e = inner.run(Z, (char *)out + (size_t)l0 * out_dist * rb, cnt, L, out_dist / 2, 1, scale, isc, chunk, s);
         if (e != hipSuccess) return e;

@@ -19,8 +19,10 @@ struct R2C {
                                 // (bit 0: realdft, bit 1: invrealdft)
     const void *tw = nullptr;   // stage twiddles (single)
     const void *rtw = nullptr;  // e^{-2 pi i k/N}, k < N/2
+    const void *ptw = nullptr;  // FP64 e^{-2 pi i k/N}, k < N/32 (packed)
     C2C inner;                  // multi-pass path
     bool fused = false;         // forward: unpack fused into the four-step row pass
+    bool packed = false;        // inverse: pack fused into the four-step column pass
     int r2c_lpb = 0;            // rows per workgroup of the fused row pass (0: default)
     long long scratch_per_line = 0;
     bool init(int N, int prec);
