@@ -4,8 +4,10 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
+#include <map>
 #include <memory>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "nfft_kernels.h"
@@ -162,22 +164,6 @@ bool xcd_topology(int *nq, signed char *qmap);
 // twrow: inter-pass twiddle in the row tiles (FP32 table) or the column tiles
 hipError_t launch_four_xcd(int n1, int dir, bool twrow, const XcdArgs &a, int grid, hipStream_t s);
 
-// mixed-radix tiles (nfft_k_smooth.hip); smooth_factor() builds the stage
-// schedule of a 7-smooth length (false otherwise) with radices up to maxr
-// (8, 10 or 25; the bound smooth_lines<..., MAXR> is compiled with).  The
-// standalone mixed-radix kernels are compiled for smooth_radix<T>()
-// (smooth_radix_of(prec) on the host).
-inline int smooth_radix_of(int prec) { return prec == F32 ? smooth_radix<float>() : smooth_radix<double>(); }
-bool smooth_factor(long long n, SmoothPlan *sp, int maxr);
-// mixed-radix four-step: n = N1 x N2, both 7-smooth and <= maxlen
-bool smooth_split(long long n, int maxlen, SmoothPlan *sp1, SmoothPlan *sp2, int maxr);
-hipError_t launch_smooth4(int prec, int dir, const Smooth4Args &a, hipStream_t s);
-// longest factor of a mixed-radix four-step tried first, and the points per
-// workgroup of its tile kernels (two LDS buffers each: 32 KiB, so that five
-// workgroups share a CU)
-int smooth_line_max(int prec);
-inline int smooth_tile_points(int prec) { return prec == F32 ? 2048 : 1024; }
-
 // Schedules of the mixed-radix lines and tiles (nfft_k_mix.hip).
 // How lanes map to the points of a workgroup's lines: neighbouring points
 // (contiguous lines), neighbouring lines (columns), or points on the first
@@ -200,7 +186,32 @@ bool mix_blue_fit(int prec, long long n, MixShape sh, MixPlan *p);
 // one-pass lines of a batch: 7-smooth n >= 2, and Bluestein of any n
 bool mix_plan(int prec, long long n, MixPlan *p);
 bool mix_blue_plan(int prec, long long n, MixPlan *p);
+bool smooth7(long long n);  // no prime factor above 7
 hipError_t launch_mix(int prec, const MixArgs &a, hipStream_t s);
+
+// Schedules of tiles, `points` points each on up to nth_max threads (more
+// points where columns of a whole segment need them and the threads allow).
+struct TileFit {
+    bool ok = false;
+    MixPlan plan;
+    double cost = 0;  // per line, memory included
+};
+struct TileFits {
+    int prec, points, nth_max;
+    std::map<std::tuple<int, int, int>, TileFit> seen;
+    int seg() const { return prec == F32 ? 16 : 8; }  // points of a 128-byte segment
+    const TileFit &get(int L, MixLanes lanes, bool blue);
+};
+// The phases of one transform in tiles: N = n1 x n2 in two, or Bluestein over
+// M = n1 x n2 >= 2N - 1 in three, with their tables (chirp and H excepted).
+struct TilePlan {
+    int n1 = 0, n2 = 0, phases = 0;
+    long long elems = 0;  // scratch per transform
+    MixPhase ph[3];
+};
+enum TileStatus { TILE_OK, TILE_NONE, TILE_FAILED };  // none: no such split; failed: error set
+TileStatus tile_plan(TileFits &fits, long long n, bool blue, TilePlan *p);
+hipError_t launch_mix_tile(int prec, const MixTileArgs &a, hipStream_t s);
 
 enum EwKind { EW_UNPACK = 0, EW_PACK = 1, EW_TRIG_PRE = 2, EW_TRIG_POST = 3, EW_N1 = 4 };
 hipError_t launch_ew(int prec, int kind, const EwArgs &a, long long nthreads_x, hipStream_t s);
@@ -250,11 +261,12 @@ const void *chirp_table(int prec, long long n, const double2 **chirp64);
 // 1D complex engine over contiguous lines
 // ---------------------------------------------------------------------------
 enum C2CAlgo {
-    ALG_LINE = 0, ALG_FOUR = 1, ALG_BLUE1 = 2, ALG_BLUE3 = 3, ALG_N1 = 4, ALG_SMOOTH4 = 6,
+    ALG_LINE = 0, ALG_FOUR = 1, ALG_BLUE1 = 2, ALG_BLUE3 = 3, ALG_N1 = 4,
     ALG_BIG = 7,     // power of two beyond the four-step: N1 x N2 over two sub-engines (six-step)
     ALG_BLUEBIG = 8, // Bluestein with M beyond the three-pass form: M-point sub-engine
     ALG_MIX = 9,     // 7-smooth length in one workgroup (nfft_kernels_mix.h)
-    ALG_MIXBLUE = 10 // Bluestein over a 7-smooth M in one workgroup
+    ALG_MIXBLUE = 10, // Bluestein over a 7-smooth M in one workgroup
+    ALG_TILE = 11     // 7-smooth N in two phases of tiles, Bluestein over a 7-smooth M in three
 };
 // Longest length a C2C engine accepts (2^30: offsets and exponents stay
 // within the 32-bit twiddle exponent and the int size of the C API).
@@ -277,11 +289,8 @@ struct C2C {
     int row_pf = 1;                   // row pass on the resident prefetching grid
     int row_twin = 0;                 // inter-pass twiddle applied by the row pass
     Tw2f tw2f{};                      // its FP32 table
-    SmoothPlan sp{};                  // ALG_SMOOTH4: N1
-    SmoothPlan sp2{};                 // ALG_SMOOTH4: N2
-    int sgroup = 1;                   // ALG_SMOOTH4: columns per tile
-    int sgroup2 = 1;                  // ALG_SMOOTH4: rows per tile
     MixPlan mx{};                     // ALG_MIX, ALG_MIXBLUE: schedule
+    std::shared_ptr<TilePlan> tiles;  // ALG_TILE
     // ALG_BIG: sub1 (length n1) and sub2 (n2); ALG_BLUEBIG: sub1 (length m).
     // Shared, so that copies of an engine (axis lists) use the same tables;
     // release() of the owner releases them.
@@ -305,8 +314,7 @@ struct C2C {
 
     // Set up tables for length n; returns false with the error set.
     // smooth_mode for 7-smooth non-power-of-two n: 2 = choose (tuned /
-    // measured rule), 1 = mixed radix, 0 = Bluestein, 3 = Bluestein over a
-    // power-of-two M (callers that use its chirp / filter tables themselves)
+    // rule), 1 = mixed radix, 0 = Bluestein
     // persist_mode = 0 keeps the two-launch four-step for powers of two
     // (callers that fuse their own work into its row pass)
     bool init(int n, int prec, int smooth_mode = 2, int persist_mode = 2);

@@ -10,10 +10,13 @@
 namespace nfft {
 
 // instantiated in nfft_k_mix_f32.hip / nfft_k_mix_f64.hip
-extern template __global__ void k_mix_line<float, false>(MixArgs);
-extern template __global__ void k_mix_line<float, true>(MixArgs);
-extern template __global__ void k_mix_line<double, false>(MixArgs);
-extern template __global__ void k_mix_line<double, true>(MixArgs);
+extern template __global__ void k_mix_line<float, false, float2>(MixArgs);
+extern template __global__ void k_mix_line<float, false, double2>(MixArgs);
+extern template __global__ void k_mix_line<float, true, float2>(MixArgs);
+extern template __global__ void k_mix_line<double, false, double2>(MixArgs);
+extern template __global__ void k_mix_line<double, true, double2>(MixArgs);
+extern template __global__ void k_mix_tile<float>(MixTileArgs);
+extern template __global__ void k_mix_tile<double>(MixTileArgs);
 
 namespace {
 
@@ -216,14 +219,15 @@ MixShape line_shape(int L)
     return sh;
 }
 
+}  // namespace
+
 bool smooth7(long long v)
 {
+    if (v < 1) return false;
     for (int q : {2, 3, 5, 7})
         while (v % q == 0) v /= q;
     return v == 1;
 }
-
-}  // namespace
 
 int mix_max(int prec) { return (int)(kMixLds / (prec == F32 ? 8 : 16)); }
 
@@ -237,7 +241,18 @@ bool mix_fit(int prec, long long n, bool blue, const MixShape &sh, MixPlan *p, d
     return true;
 }
 
-bool mix_plan(int prec, long long n, MixPlan *p) { return mix_fit(prec, n, false, line_shape((int)n), p); }
+bool mix_plan(int prec, long long n, MixPlan *p)
+{
+    if (n < 2 || !mix_fit(prec, n, false, line_shape((int)n), p)) return false;
+    // FP32 twiddle tables where that keeps the error at what a table entry per
+    // twiddle gives (radices up to 10 over several stages before; Bluestein
+    // between: N = 1000 2.1e-7 -> 1.2e-7).  Short lines lose 2-3 % of it (N =
+    // 480 1.055e-7 -> 1.084e-7), lines beyond 10240 points, with two of their
+    // three stages near radix 32, up to 8 % (N = 20000 1.416e-7 -> 1.537e-7);
+    // they take the FP64 table (2^26 points: N = 20000 368 -> 410 us).
+    p->tw64 = prec == F64 || n <= 512 || n > 10240;
+    return true;
+}
 
 bool mix_blue_fit(int prec, long long n, MixShape sh, MixPlan *p)
 {
@@ -264,10 +279,10 @@ bool mix_blue_plan(int prec, long long n, MixPlan *p)
     return mix_blue_fit(prec, n, sh, p);
 }
 
-template <typename T, bool BLUE> static hipError_t mix_go(const MixArgs &a0, hipStream_t s)
+template <typename T, bool BLUE, class TW> static hipError_t mix_go(const MixArgs &a0, hipStream_t s)
 {
     static const bool attr = [] {  // once per instantiation and process
-        (void)hipFuncSetAttribute((const void *)k_mix_line<T, BLUE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        (void)hipFuncSetAttribute((const void *)k_mix_line<T, BLUE, TW>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)kMixLds);
         (void)hipGetLastError();
         return true;
@@ -283,7 +298,7 @@ template <typename T, bool BLUE> static hipError_t mix_go(const MixArgs &a0, hip
     if (grid > 0x7fffffffLL || lds > kMixLds || a.pl.nth < 64 || a.pl.nth > mix_threads<T>()) return hipErrorInvalidValue;
     for (int i = 0; i < a.pl.steps; i++)  // every butterfly has its place in a thread
         if (a.pl.G * a.pl.st[i].nb > a.pl.nth * mix_reps(a.pl.st[i].radix)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_mix_line<T, BLUE>), dim3((unsigned)grid), dim3(a.pl.nth), lds, s, a);
+    hipLaunchKernelGGL((k_mix_line<T, BLUE, TW>), dim3((unsigned)grid), dim3(a.pl.nth), lds, s, a);
     return hipGetLastError();
 }
 
@@ -292,11 +307,150 @@ hipError_t launch_mix(int prec, const MixArgs &a, hipStream_t s)
     const bool blue = a.pl.blue != 0;
     if (blue && (!a.chirp || !a.H)) return hipErrorInvalidValue;
     const int slot = prof_on() ? prof_begin(s) : -1;
-    const hipError_t e = prec == F32 ? (blue ? mix_go<float, true>(a, s) : mix_go<float, false>(a, s))
-                                     : (blue ? mix_go<double, true>(a, s) : mix_go<double, false>(a, s));
+    const hipError_t e = prec == F32 ? (blue          ? mix_go<float, true, float2>(a, s)
+                                        : a.pl.tw64 ? mix_go<float, false, double2>(a, s)
+                                                    : mix_go<float, false, float2>(a, s))
+                                     : (blue ? mix_go<double, true, double2>(a, s) : mix_go<double, false, double2>(a, s));
     if (slot >= 0)
         prof_end(slot, s, blue ? "k_mix_line(bluestein)" : "k_mix_line", prec, a.pl.L,
                  2.0 * (double)a.nlines * (blue ? a.n : a.pl.L) * (prec == F32 ? 8.0 : 16.0));
+    return e;
+}
+
+// lines of L points, in tiles; strided lanes: neighbouring lines are the ones
+// contiguous in memory, so a tile should span a segment of them
+const TileFit &TileFits::get(int L, MixLanes lanes, bool blue)
+{
+    auto it = seen.find({L, (int)lanes, blue ? 1 : 0});
+    if (it != seen.end()) return it->second;
+    TileFit best;
+    auto consider = [&](int g, int nth_min, size_t lds_max) {
+        MixShape sh;
+        sh.g_min = sh.g_max = g;
+        sh.nth_min = nth_min;
+        sh.nth_max = nth_max;
+        sh.lanes = lanes;
+        sh.lds_max = lds_max;
+        TileFit f;
+        f.ok = mix_fit(prec, L, blue, sh, &f.plan, &f.cost);
+        // a point read and written takes half an issue slot of its CU's share
+        // of the memory bandwidth, more where a tile covers part of a segment
+        if (f.ok)
+            f.cost += 0.5 * (prec == F32 ? 1 : 2) * L *
+                      (lanes == MIX_LANES_POINTS ? 1.0 : std::max(1.0, (double)seg() / f.plan.G));
+        if (f.ok && (!best.ok || f.cost < best.cost)) best = f;
+        return f.ok;
+    };
+    int g = std::max(1, points / L);
+    if (lanes != MIX_LANES_POINTS && g > seg()) g -= g % seg();
+    g = std::min(g, 64);
+    // as many workgroups of kTileThreads per CU as their registers allow (4 / 2)
+    const size_t part = points <= 16 * kTileThreads ? (prec == F32 ? kMixLds / 4 : kMixLds / 2) : kMixLds;
+    for (int h = g; h >= 1 && !consider(h, kTileThreads, part); h = h > 1 ? (h + 1) / 2 : 0) {}
+    if (nth_max > kTileThreads && (!best.ok || (lanes != MIX_LANES_POINTS && g < seg())))
+        for (int h = seg(); h >= 1; h /= 2) consider(h, kTileThreads, kMixLds);
+    return seen.emplace(std::make_tuple(L, (int)lanes, blue ? 1 : 0), best).first->second;
+}
+
+TileStatus tile_plan(TileFits &fits, long long n, bool blue, TilePlan *p)
+{
+    // cost of all lines of a phase
+    auto phase = [](const TileFit &f, int lines) {
+        return f.ok ? f.cost * f.plan.G * ((lines + f.plan.G - 1) / f.plan.G) : 1e300;
+    };
+    const long long lo = 2 * n - 1;
+    const int amax = fits.nth_max > kTileThreads ? 1280 : 1024, bmax = fits.nth_max > kTileThreads ? 4096 : 2048;
+    double best = 1e299;
+    int n1 = 0, n2 = 0;
+    for (int a = 32; a <= amax; a++) {
+        if (!smooth7(a) || (!blue && n % a)) continue;
+        long long b = blue ? (lo + a - 1) / a : n / a;
+        int tries = blue ? 2 : 1;
+        for (; tries > 0 && b <= bmax; b++) {
+            // Bluestein: rows of whole segments, so that tiles of columns are aligned
+            if (!smooth7(b) || (blue && b % fits.seg())) continue;
+            tries--;
+            if (b < 32) continue;
+            double c = phase(fits.get(a, MIX_LANES_LINES, false), (int)b);
+            if (c >= best) continue;
+            if (blue) c = 2 * c + phase(fits.get((int)b, MIX_LANES_POINTS, true), a);
+            else c += phase(fits.get((int)b, MIX_LANES_TRANSPOSE, false), a);
+            if (c < best) {
+                best = c;
+                n1 = a;
+                n2 = (int)b;
+            }
+        }
+    }
+    if (best >= 1e299) return TILE_NONE;
+    Tw2 tw2;
+    const void *t1 = phase_table(F64, n1, 1, 0, n1), *t2 = phase_table(F64, n2, 1, 0, n2);
+    if (!t1 || !t2 || !tw2_table((long long)n1 * n2, &tw2)) return TILE_FAILED;
+    // the scratch holds rows of whole segments
+    const int pitch = (n2 + fits.seg() - 1) / fits.seg() * fits.seg();
+    p->n1 = n1;
+    p->n2 = n2;
+    p->elems = (long long)n1 * pitch;
+    MixPhase cols{};
+    cols.pl = fits.get(n1, MIX_LANES_LINES, false).plan;
+    cols.tw = t1;
+    cols.tw2 = tw2;
+    cols.ig = cols.og = 1;
+    cols.ip = n2;
+    cols.op = pitch;
+    cols.lines = n2;
+    cols.nv = (int)n;
+    cols.flags = MIX_HEAD | MIX_TW | (blue ? MIX_CHIRP_IN : 0);
+    MixPhase rows = cols;
+    rows.pl = fits.get(n2, blue ? MIX_LANES_POINTS : MIX_LANES_TRANSPOSE, blue).plan;
+    rows.tw = t2;
+    rows.ig = pitch;
+    rows.ip = 1;
+    rows.lines = n1;
+    p->ph[0] = cols;
+    if (blue) {
+        rows.og = pitch;
+        rows.op = 1;
+        rows.flags = MIX_TW;
+        cols.flags = MIX_TAIL | MIX_CHIRP_OUT;
+        p->ph[2] = cols;
+    } else {
+        rows.og = 1;
+        rows.op = n1;
+        rows.flags = MIX_TAIL;
+    }
+    p->ph[1] = rows;
+    p->phases = blue ? 3 : 2;
+    return TILE_OK;
+}
+
+template <typename T> static hipError_t mix_tile_go(const MixTileArgs &a, hipStream_t s)
+{
+    static const bool attr = [] {  // once per precision and process
+        (void)hipFuncSetAttribute((const void *)k_mix_tile<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMixLds);
+        (void)hipGetLastError();
+        return true;
+    }();
+    (void)attr;
+    const MixPlan &pl = a.ph.pl;
+    if (a.ntrans < 1) return hipSuccess;
+    const long long grid = a.ntrans * ((a.ph.lines + pl.G - 1) / pl.G);
+    const size_t lds = (size_t)pl.G * pl.lp * sizeof(Cx<T>);
+    if (grid > 0x7fffffffLL || lds > kMixLds || pl.nth < 64 || pl.nth > mix_threads<T>()) return hipErrorInvalidValue;
+    if ((pl.blue && !a.ph.H) || ((a.ph.flags & (MIX_CHIRP_IN | MIX_CHIRP_OUT)) && !a.ph.chirp)) return hipErrorInvalidValue;
+    for (int i = 0; i < pl.steps; i++)  // every butterfly has its place in a thread
+        if (pl.G * pl.st[i].nb > pl.nth * mix_reps(pl.st[i].radix)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_mix_tile<T>, dim3((unsigned)grid), dim3(pl.nth), lds, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_mix_tile(int prec, const MixTileArgs &a, hipStream_t s)
+{
+    const int slot = prof_on() ? prof_begin(s) : -1;
+    const hipError_t e = prec == F32 ? mix_tile_go<float>(a, s) : mix_tile_go<double>(a, s);
+    if (slot >= 0)
+        prof_end(slot, s, "k_mix_tile", prec, a.ph.pl.L,
+                 2.0 * (double)a.ntrans * a.ph.lines * a.ph.pl.L * (prec == F32 ? 8.0 : 16.0));
     return e;
 }
 

@@ -1,7 +1,9 @@
-// nfft_k_mix_f32.hip -- one-pass mixed-radix lines, FP32
+// nfft_k_mix_f32.hip -- mixed-radix lines and tiles, FP32
 #include "nfft_kernels_mix.h"
 
 namespace nfft {
-template __global__ void k_mix_line<float, false>(MixArgs);
-template __global__ void k_mix_line<float, true>(MixArgs);
+template __global__ void k_mix_line<float, false, double2>(MixArgs);
+template __global__ void k_mix_line<float, false, float2>(MixArgs);
+template __global__ void k_mix_line<float, true, float2>(MixArgs);
+template __global__ void k_mix_tile<float>(MixTileArgs);
 }  // namespace nfft

@@ -1,7 +1,8 @@
-// nfft_k_mix_f64.hip -- one-pass mixed-radix lines, FP64
+// nfft_k_mix_f64.hip -- mixed-radix lines and tiles, FP64
 #include "nfft_kernels_mix.h"
 
 namespace nfft {
-template __global__ void k_mix_line<double, false>(MixArgs);
-template __global__ void k_mix_line<double, true>(MixArgs);
+template __global__ void k_mix_line<double, false, double2>(MixArgs);
+template __global__ void k_mix_line<double, true, double2>(MixArgs);
+template __global__ void k_mix_tile<double>(MixTileArgs);
 }  // namespace nfft

@@ -6,8 +6,7 @@
 // 16 to 32, so that three stages cover up to 20480 points), one runtime
 // schedule per length.  Stage s of radix R and stride Ns maps butterfly j
 // (jq = j / Ns, k = j mod Ns) from points j + t L/R to points
-// jq Ns R + k + t Ns.  The stage loop differs from smooth_lines in what it
-// moves:
+// jq Ns R + k + t Ns.  What moves:
 //   - the first stage reads its points from global memory and the last one
 //     writes them there, so S stages make S - 1 exchanges through LDS and
 //     the line crosses HBM once each way;
@@ -48,6 +47,7 @@ struct MixPlan {
     float inG = 1.0f;           // its reciprocal for fdiv
     int nth = 0;                // threads per workgroup
     int lp = 0;                 // LDS points per line, padding included
+    int tw64 = 0;               // lines: FP64 twiddle table (FP64 lines: always)
     MixStep st[kMixMaxSteps];
 };
 
@@ -66,23 +66,29 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t mix_rsrc(const void *base, uin
 }
 
 // w^t, t < R, applied to v: entry e of the table is e^{-2 pi i e / L}, w the
-// entry `e`.  Powers t = Q h + l from the entries of l and Q h.
-template <typename T, int R>
-__device__ __forceinline__ void mix_twiddle(Cx<T> (&v)[R], __amdgpu_buffer_rsrc_t tw, int e)
+// entry `e`.  Powers t = Q h + l as products of the entries of l and Q h.
+// W: type of the table entries.  FP64 tables in FP32 transforms make each
+// power as exact as an entry of its own (mix_plan says which lines have them).
+template <typename W, int R, typename C>
+__device__ __forceinline__ void mix_twiddle(C (&v)[R], __amdgpu_buffer_rsrc_t tw, int e)
 {
-    using C = Cx<T>;
     constexpr int Q = R <= 5 ? R : R <= 9 ? 3 : R <= 16 ? 4 : R <= 25 ? 5 : 6;
     constexpr int NH = (R - 1) / Q;
-    const uint32_t eb = (uint32_t)e * (uint32_t)sizeof(C);
-    C lo[Q], hi[NH + 1];
+    const uint32_t eb = (uint32_t)e * (uint32_t)sizeof(W);
+    auto product = [](W a, W b) -> W {
+        if constexpr (sizeof(a.x) == 8) return dmul(a, b);
+        else return cmul(a, b);
+    };
+    W lo[Q], hi[NH + 1];
 #pragma unroll
-    for (int l = 1; l < Q; l++) lo[l] = buf_ld<C>(tw, eb * (uint32_t)l, 0);
+    for (int l = 1; l < Q; l++) lo[l] = buf_ld<W>(tw, eb * (uint32_t)l, 0);
 #pragma unroll
-    for (int h = 1; h <= NH; h++) hi[h] = buf_ld<C>(tw, eb * (uint32_t)(Q * h), 0);
+    for (int h = 1; h <= NH; h++) hi[h] = buf_ld<W>(tw, eb * (uint32_t)(Q * h), 0);
 #pragma unroll
     for (int t = 1; t < R; t++) {
         const int h = t / Q, l = t % Q;
-        v[t] = cmul(v[t], h == 0 ? lo[l] : l == 0 ? hi[h] : cmul(hi[h], lo[l]));
+        const W w = h == 0 ? lo[l] : l == 0 ? hi[h] : product(hi[h], lo[l]);
+        v[t] = cmul(v[t], cmk<C>((decltype(C::x))w.x, (decltype(C::x))w.y));
     }
 }
 
@@ -128,7 +134,7 @@ __device__ __forceinline__ void mix_step(const PL &pl, int s, Cx<T> *lds, __amdg
                 const C *p = lds + (__mul24(g, pl.lp) + __mul24(jq, up) + k);
 #pragma unroll
                 for (int t = 0; t < R; t++) v[i][t] = p[t * rs];
-                mix_twiddle<T, R>(v[i], tw, __mul24(k, st.q));
+                mix_twiddle<typename IO::W, R>(v[i], tw, __mul24(k, st.q));
             }
             dft_any<R, -1>(v[i]);
             if constexpr (BLUE) {
@@ -182,8 +188,9 @@ __device__ __forceinline__ void mix_lines(const PL &pl, Cx<T> *lds, const void *
 // transforms; the inverse of the convolution is conj(FFT(conj(.))), folded
 // into the products.  OFFS gives the byte offset of a line from the base of
 // `in` / `out`.
-template <typename T, bool BLUE, class OFFS> struct MixIoLine {
+template <typename T, bool BLUE, class OFFS, class TW = Cx<T>> struct MixIoLine {
     using C = Cx<T>;
+    using W = TW;  // twiddle table entries
     __amdgpu_buffer_rsrc_t in, out, chirp, H;  // in, out, chirp end with their last point
     OFFS offs;
     int glast;  // last line of this workgroup
@@ -257,7 +264,7 @@ struct MixArgs {
     long long nlines;
     long long in_dist, out_dist;
     MixPlan pl;
-    const void *tw;           // L entries e^{-2 pi i q / L}
+    const void *tw;           // L entries e^{-2 pi i q / L}, FP64 where pl.tw64
     int inverse;
     double scale;
     int n;                    // Bluestein: transform length
@@ -269,9 +276,9 @@ struct MixArgs {
 // one workgroup alternates loading, stages and storing.  2^26 points, before
 // (mixed-radix lines with two LDS buffers up to 2048 points, Bluestein or a
 // two-pass four-step) and now: FP32 N = 100 346 -> 213 us (5.0 TB/s), N =
-// 1000 489 -> 261, N = 10^4 800 -> 223 (4.8 TB/s), N = 20000 982 -> 363; FP64
+// 1000 489 -> 261, N = 10^4 800 -> 230 (4.7 TB/s), N = 20000 982 -> 410; FP64
 // N = 100 598 -> 435 us, N = 1000 709 -> 516, N = 10^4 1365 -> 527.
-template <typename T, bool BLUE> __global__ void __launch_bounds__(mix_threads<T>()) k_mix_line(MixArgs a)
+template <typename T, bool BLUE, class TW> __global__ void __launch_bounds__(mix_threads<T>()) k_mix_line(MixArgs a)
 {
     using C = Cx<T>;
     extern __shared__ char smem[];
@@ -280,7 +287,7 @@ template <typename T, bool BLUE> __global__ void __launch_bounds__(mix_threads<T
     const int cnt = (int)(rem < a.pl.G ? rem : a.pl.G);
     const MixDist d{(uint32_t)a.in_dist * (uint32_t)sizeof(C), (uint32_t)a.out_dist * (uint32_t)sizeof(C)};
     const uint32_t len = (uint32_t)(BLUE ? a.n : a.pl.L) * (uint32_t)sizeof(C);
-    const MixIoLine<T, BLUE, MixDist> io{mix_rsrc((const C *)a.in + l0 * a.in_dist, (uint32_t)(cnt - 1) * d.idist + len),
+    const MixIoLine<T, BLUE, MixDist, TW> io{mix_rsrc((const C *)a.in + l0 * a.in_dist, (uint32_t)(cnt - 1) * d.idist + len),
                                          mix_rsrc((C *)a.out + l0 * a.out_dist, (uint32_t)(cnt - 1) * d.odist + len),
                                          mix_rsrc(a.chirp, len),
                                          buf_rsrc(a.H),
@@ -307,7 +314,7 @@ template <typename T, bool BLUE> __global__ void __launch_bounds__(mix_threads<T
 enum { MIX_CHIRP_IN = 1, MIX_CHIRP_OUT = 2, MIX_TW = 4, MIX_HEAD = 8, MIX_TAIL = 16 };
 struct MixPhase {
     MixPlan pl;
-    const void *tw;            // L entries e^{-2 pi i q / L}
+    const void *tw;            // L entries e^{-2 pi i q / L}: FP64 (tiles) or the transform's type (groups)
     Tw2 tw2;                   // MIX_TW: two-level table of the whole length
     const void *chirp, *H;     // chirp entries below nv; filter in the layout of the rows
     int ig, ip, og, op;        // element distances of lines and points, input and output
@@ -320,32 +327,33 @@ struct MixPhase {
 // again after every store.
 typedef const MixPhase __attribute__((address_space(4))) MixPhaseK;
 
-// v[t] *= w^{e0 + t es} (w = e^{-2 pi i / N}): two table entries and chains
-// of FP64 products (FP32: two chains, which leaves the registers of radix 32
-// below 128; FP64: four, at most nine products deep).
+// v[t] *= w^{e0 + t es} (w = e^{-2 pi i / N}).  FP32: two table entries and
+// two chains of FP64 products, rounded once.  FP64: the entries of every t (a
+// chain would add an ulp per product).
 template <int R, typename C>
 __device__ __forceinline__ void mix_tw2(C (&v)[R], const Tw2 &tab, uint32_t e0, uint32_t es)
 {
-    constexpr int Q = sizeof(v[0].x) == 4 ? 2 : 4;
-    double2 st = tw2_get(tab, es), b[Q];
-    b[0] = tw2_get(tab, e0);
-    b[1] = dmul(b[0], st);
-    st = dmul(st, st);
-    if constexpr (Q == 4) {
-        b[2] = dmul(b[0], st);
-        b[3] = dmul(b[1], st);
+    if constexpr (sizeof(v[0].x) == 4) {
+        double2 st = tw2_get(tab, es), b[2];
+        b[0] = tw2_get(tab, e0);
+        b[1] = dmul(b[0], st);
         st = dmul(st, st);
-    }
 #pragma unroll
-    for (int t = 0; t < R; t++) {
-        v[t] = ctw64<-1>(v[t], b[t % Q]);
-        if (t + Q < R) b[t % Q] = dmul(b[t % Q], st);
+        for (int t = 0; t < R; t++) {
+            v[t] = ctw64<-1>(v[t], b[t % 2]);
+            if (t + 2 < R) b[t % 2] = dmul(b[t % 2], st);
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < R; t++) v[t] = ctw64<-1>(v[t], tw2_get(tab, e0 + (uint32_t)t * es));
     }
 }
 
-template <typename T> struct MixIoTile {
+// PH: MixPhase, as a kernel argument or in constant memory
+template <typename T, class PH> struct MixIoTile {
     using C = Cx<T>;
-    MixPhaseK &ph;
+    using W = double2;  // twiddle table entries
+    const PH &ph;
     __amdgpu_buffer_rsrc_t in, out, chirp, H;  // in / out / H at line c0 (chirped sides: at the transform)
     int c0, glast;
     T sg, sc;                                  // inverse: -1 and the scale of the result
@@ -407,13 +415,13 @@ template <typename T> struct MixIoTile {
 
 // Lines [c0, c0 + cnt) of phase `ph` of one transform (cnt <= ph.pl.G); src
 // and dst at the transform (or its scratch).
-template <typename T>
-__device__ __forceinline__ void mix_tile(MixPhaseK &ph, const Cx<T> *src, Cx<T> *dst, int c0, int cnt, int inverse,
+template <typename T, class PH>
+__device__ __forceinline__ void mix_tile(const PH &ph, const Cx<T> *src, Cx<T> *dst, int c0, int cnt, int inverse,
                                          T scale, Cx<T> *lds)
 {
     using C = Cx<T>;
     const uint32_t nb = (uint32_t)ph.nv * (uint32_t)sizeof(C);
-    MixIoTile<T> io{ph,
+    const MixIoTile<T, PH> io{ph,
                     ph.flags & MIX_CHIRP_IN ? mix_rsrc(src, nb) : buf_rsrc(src + (long long)c0 * ph.ig),
                     ph.flags & MIX_CHIRP_OUT ? mix_rsrc(dst, nb) : buf_rsrc(dst + (long long)c0 * ph.og),
                     mix_rsrc(ph.chirp, nb),
@@ -423,6 +431,42 @@ __device__ __forceinline__ void mix_tile(MixPhaseK &ph, const Cx<T> *src, Cx<T> 
                     inverse ? (T)-1 : (T)1,
                     scale};
     mix_lines<T, true>(ph.pl, lds, ph.tw, io);
+}
+
+// Item of workgroup b: kTileRun neighbouring items go to one XCD (workgroup b
+// runs on XCD b mod 8), since tiles whose edges share 128-byte lines then
+// share an L2 (the ragged batch of nfft_ragged.hip: 1.54 -> 1.42 ms).
+constexpr int kTileRun = 16;
+__device__ __forceinline__ long long mix_item(long long b, long long nitems)
+{
+    const long long w = b % (8 * kTileRun);
+    return b < nitems / (8 * kTileRun) * (8 * kTileRun) ? b - w + (w & 7) * kTileRun + (w >> 3) : b;
+}
+
+// One phase of a batch of transforms of one length.
+struct MixTileArgs {
+    const void *in;
+    void *out;
+    long long in_dist, out_dist;  // elements between transforms on either side
+    long long ntrans;
+    int inverse;
+    double scale;
+    MixPhase ph;
+};
+// Bound: memory, as the ragged tiles (four workgroups of 4096 points per CU in
+// FP32, two in FP64).  2^26 points, before (two LDS buffers per tile, radices
+// up to 10; Bluestein over the next power of two) and now: FP32 N = 20736 1134
+// -> 472 us, 196608 1225 -> 480, 10^6 1589 (Bluestein) -> 667, 33333 2496 ->
+// 1584; FP64 20736 1810 -> 839, 196608 1969 -> 923, 33331 4441 -> 3697.
+template <typename T> __global__ void __launch_bounds__(mix_threads<T>()) k_mix_tile(MixTileArgs a)
+{
+    using C = Cx<T>;
+    extern __shared__ char smem[];
+    const int G = a.ph.pl.G, tiles = (a.ph.lines + G - 1) / G;
+    const long long i = mix_item(blockIdx.x, a.ntrans * tiles), t = i / tiles;
+    const int c0 = (int)(i - t * tiles) * G;
+    mix_tile<T>(a.ph, (const C *)a.in + t * a.in_dist, (C *)a.out + t * a.out_dist, c0, min(G, a.ph.lines - c0),
+                a.inverse, (T)a.scale, (C *)smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -485,13 +529,8 @@ template <typename T> __global__ void __launch_bounds__(kTileThreads, (sizeof(T)
 {
     using C = Cx<T>;
     extern __shared__ char smem[];
-    // kTileRun neighbouring items go to one XCD (workgroup b runs on XCD b mod
-    // 8): tiles whose edges share 128-byte lines then share an L2
-    constexpr int kTileRun = 16;
-    const int full = a.nitems / (8 * kTileRun) * (8 * kTileRun);
     for (int b = blockIdx.x; b < a.nitems; b += gridDim.x) {
-        const int w = b % (8 * kTileRun);
-        const int i = b < full ? b - w + (w & 7) * kTileRun + (w >> 3) : b;
+        const int i = (int)mix_item(b, a.nitems);
         RagItemK &it = ((RagItemK *)a.items)[i];
         MixPhaseK &ph = ((MixPhaseK *)a.phases)[it.phase];
         mix_tile<T>(ph, (const C *)a.in + it.src, (C *)(it.in_place ? a.alt : a.out) + it.dst, it.c0, it.cnt, a.inverse, rag_scale<T>(a, it),

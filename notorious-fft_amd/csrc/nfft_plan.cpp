@@ -279,24 +279,6 @@ static int env_int(const char *name, int dflt)
 // ---------------------------------------------------------------------------
 // mixed radix vs Bluestein for 7-smooth lengths
 // ---------------------------------------------------------------------------
-// Tile width for `len` columns/rows at most `wmax` wide, balanced so that no
-// tile is much narrower than the others.
-static int balanced_width(int len, int wmax)
-{
-    wmax = std::max(1, std::min(len, wmax));
-    const int tiles = (len + wmax - 1) / wmax;
-    return (len + tiles - 1) / tiles;
-}
-
-// Measured on MI355X (2^28 FP32 / 2^27 FP64 elements), beyond the one-pass
-// lines (which win at every length they exist for): the mixed-radix four-step
-// wins for FP64 unless its tiles are a single column or row wide, and for
-// FP32 from 10^4 points with tiles >= 4 wide.
-static bool smooth_default(int prec, long long n, int wmin)
-{
-    return prec == F64 ? wmin >= 2 : (n >= 10000 && wmin >= 4);
-}
-
 static std::string smooth_key(int prec, long long n)
 {
     return "c2c-smooth p" + std::to_string(prec) + " n" + std::to_string(n);
@@ -706,39 +688,32 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
     // when NFFT_TUNE=1, else the measured default rule
     const int smooth_env = env_int("NFFT_SMOOTH", 1);  // 0: never, 2: whenever possible
     if (smooth_env == 2 && smooth_mode == 2) smooth_mode = 1;
-    if (smooth_mode != 0 && smooth_mode != 3 && smooth_env != 0 && !is_pow2(n)) {
-        SmoothPlan p1{}, p2{};
-        const int mr = smooth_radix_of(prec), lm = smooth_line_max(prec);
-        // One pass, a line or a group of lines per workgroup, up to mix_max;
-        // NFFT_SMOOTH=2 takes the four-step from smooth_line_max on.
-        const bool mix = (smooth_env != 2 || n <= lm) && mix_plan(prec, n, &mx);
-        const bool four = !mix && (smooth_split(n, lm, &p1, &p2, mr) ||
-                                   smooth_split(n, prec == F32 ? 8192 : 4096, &p1, &p2, mr));
-        if (mix || four) {
-            const int budget = smooth_tile_points(prec);
-            const int w1 = four ? balanced_width(p2.L, budget / p1.L) : 0;
-            const int w2 = four ? balanced_width(p1.L, budget / p2.L) : 0;
-            int use = smooth_mode == 1 ? 1 : tuned_choice(prec, n);
-            if (use < 0 && env_int("NFFT_TUNE", 0)) use = tune_smooth(n, prec);
-            if (use < 0) use = mix || smooth_default(prec, n, std::min(w1, w2)) ? 1 : 0;
-            if (use == 1 && mix) {
-                algo = ALG_MIX;
-                tw_a = phase_table(prec, n, 1, 0, n);
-                return tw_a != nullptr;
+    TileFits fits{prec, 16 * kTileThreads, prec == F32 ? mix_threads<float>() : mix_threads<double>(), {}};
+    if (smooth_mode != 0 && smooth_env != 0 && !is_pow2(n) && smooth7(n)) {
+        // One pass, a line or a group of lines per workgroup, up to mix_max
+        // (NFFT_SMOOTH=2: tiles before lines from 2048 / 1024 points on), else
+        // two phases of tiles; lengths with no split for them use Bluestein.
+        const bool line = mix_plan(prec, n, &mx);
+        const bool tiles_first = !line || (smooth_env == 2 && n > (prec == F32 ? 2048 : 1024));
+        int use = smooth_mode == 1 ? 1 : tuned_choice(prec, n);
+        if (use < 0 && env_int("NFFT_TUNE", 0)) use = tune_smooth(n, prec);
+        if (use != 0 && tiles_first) {
+            tiles = std::make_shared<TilePlan>();
+            const TileStatus st = tile_plan(fits, n, false, tiles.get());
+            if (st == TILE_FAILED) return false;
+            if (st == TILE_OK) {
+                algo = ALG_TILE;
+                n1 = tiles->n1;
+                n2 = tiles->n2;
+                scratch_per_line = tiles->elems;
+                return true;
             }
-            if (use == 1) {
-                sp = p1;
-                algo = ALG_SMOOTH4;
-                sp2 = p2;
-                n1 = p1.L;
-                n2 = p2.L;
-                sgroup = w1;
-                sgroup2 = w2;
-                tw_a = phase_table(prec, n1, 1, 0, n1);
-                tw_b = phase_table(prec, n2, 1, 0, n2);
-                scratch_per_line = n;
-                return tw_a && tw_b && tw2_table(n, &tw2);
-            }
+            tiles.reset();
+        }
+        if (use != 0 && line) {
+            algo = ALG_MIX;
+            tw_a = phase_table(mx.tw64 ? F64 : prec, n, 1, 0, n);
+            return tw_a != nullptr;
         }
     }
     // Bluestein
@@ -752,8 +727,34 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
     // = 10007 2.27 -> 1.06 ms, FP64 N = 4097 4.12 -> 2.10 ms).  Where both
     // fit, the power-of-two line is the faster (FP32 N = 1009 0.47 vs 0.76
     // ms, FP64 0.86 vs 1.65).
-    const bool mixblue = smooth_mode != 3 && m > line_max(prec) && mix_blue_plan(prec, n, &mx);
-    if (mixblue) {
+    const bool mixblue = m > line_max(prec) && mix_blue_plan(prec, n, &mx);
+    // Longer ones in three phases of tiles over a 7-smooth M, where that is
+    // enough shorter than the power of two, whose passes move a byte faster
+    // (2^26 points, power of two / tiles in us, after the ratio of the two M:
+    // FP32 N = 10301 1.52 2225 / 1649, 16381 1.00 1542 / 1411, 28001 1.14 1475
+    // / 1490, 30011 1.07 1395 / 1486, 44101 1.42 1984 / 1615, 110017 1.19 1782
+    // / 1784; FP64 5209 1.52 3404 / 3411, 12007 1.33 3206 / 3512, 20011 1.60
+    // 3732 / 3505, 35023 1.83 4296 / 3624, 90001 1.42 3594 / 3956; beyond
+    // 2^17 points the power of two: FP32 500009 1518 / 2107).
+    bool tileblue = false;
+    if (!mixblue && m > line_max(prec) && n < (1 << 17)) {
+        TileFits small{prec, 16 * kTileThreads, kTileThreads, {}};
+        tiles = std::make_shared<TilePlan>();
+        const TileStatus st = tile_plan(small, n, true, tiles.get());
+        if (st == TILE_FAILED) return false;
+        const long long mt = (long long)tiles->n1 * tiles->n2;
+        const double least = prec == F64 ? 1.6 : m <= (1 << 15) ? 1.0 : 1.2;
+        tileblue = st == TILE_OK && m >= least * mt;
+        if (!tileblue) tiles.reset();
+    }
+    if (tileblue) {
+        algo = ALG_TILE;
+        m1 = tiles->n1;
+        m2 = tiles->n2;
+        m = m1 * m2;
+        for (MixPhase &p : tiles->ph) p.chirp = chirp;
+        scratch_per_line = tiles->elems;
+    } else if (mixblue) {
         algo = ALG_MIXBLUE;
         m = mx.L;
         tw_a = phase_table(prec, m, 1, 0, m);
@@ -769,7 +770,8 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
         m2 = 1 << lg2;
         m1 = m / m2;
     }
-    if (!mixblue && m > line_max(prec) && m1 > col_max(prec)) {
+    const bool smooth_m = mixblue || tileblue;
+    if (!smooth_m && m > line_max(prec) && m1 > col_max(prec)) {
         // M beyond the three-pass form: chirp, FFT_M, x H, IFFT_M, chirp as
         // elementwise passes around an M-point engine
         if (m > kMaxLen) {
@@ -781,7 +783,7 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
         sub1 = std::make_shared<C2C>();
         if (!sub1->init(m, prec)) return false;
         scratch_per_line = m + sub1->scratch_per_line;
-    } else if (!mixblue && m > line_max(prec)) {
+    } else if (!smooth_m && m > line_max(prec)) {
         algo = ALG_BLUE3;
         tw_a = stage_table(prec, m1);
         tw_b = stage_table(prec, m2);
@@ -790,7 +792,7 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
     }
     // filter spectrum H = FFT_m(h) / m, computed in FP64 by this engine
     C2C h64;
-    if (!h64.init(m, F64, mixblue ? 1 : 2)) return false;
+    if (!h64.init(m, F64, smooth_m ? 1 : 2)) return false;
     hipStream_t st = setup_stream();
     void *hbuf = nullptr, *Hbuf = nullptr, *sbuf = nullptr;
     bool ok = hip_ok(dev_malloc(&hbuf, (size_t)m * 16), "hipMalloc") &&
@@ -799,7 +801,7 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
     if (ok && h64.scratch_per_line) ok = hip_ok(dev_malloc(&sbuf, (size_t)h64.scratch_per_line * 16), "hipMalloc");
     ok = ok && hip_ok(launch_blue_filter((double2 *)hbuf, chirp64, n, m, st), "filter") &&
          hip_ok(h64.run(hbuf, Hbuf, 1, m, m, -1, 1.0, sbuf, 1, st), "filter FFT") &&
-         hip_ok(launch_blue_hprep((const double2 *)Hbuf, H, prec, m, algo == ALG_BLUE3 ? m1 : 0, m2, 1.0 / m, st),
+         hip_ok(launch_blue_hprep((const double2 *)Hbuf, H, prec, m, algo == ALG_BLUE3 || tileblue ? m1 : 0, m2, 1.0 / m, st),
                 "filter prep") &&
          hip_ok(hipStreamSynchronize(st), "filter sync");
     (void)hipFree(hbuf);
@@ -810,6 +812,7 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
         if (H) (void)hipFree(H);
         H = nullptr;
     }
+    if (tileblue) tiles->ph[1].H = H;
     return ok;
 }
 
@@ -856,7 +859,10 @@ std::string C2C::describe() const
             snprintf(b, sizeof b, "four-step %dx%d", n1, n2);
         break;
     case ALG_BLUE1: snprintf(b, sizeof b, "bluestein N=%d M=%d single-pass", n, m); break;
-    case ALG_SMOOTH4: snprintf(b, sizeof b, "mixed-radix four-step %dx%d", n1, n2); break;
+    case ALG_TILE:
+        if (tiles->phases == 2) snprintf(b, sizeof b, "mixed-radix four-step %dx%d", n1, n2);
+        else snprintf(b, sizeof b, "bluestein N=%d M=%d in tiles (%dx%d)", n, m, m1, m2);
+        break;
     case ALG_MIX:
     case ALG_MIXBLUE: {
         int o = algo == ALG_MIX ? snprintf(b, sizeof b, "mixed-radix %d (", n)
@@ -902,26 +908,24 @@ hipError_t C2C::run(const void *in, void *out, long long nlines, long long in_di
         }
         return launch_mix(prec, a, s);
     }
-    case ALG_SMOOTH4: {
+    case ALG_TILE: {
         if (scratch_lines < 1 || !scratch) return hipErrorInvalidValue;
         for (long long l0 = 0; l0 < nlines; l0 += scratch_lines) {
-            Smooth4Args a{};
-            a.in = (const char *)in + (size_t)l0 * in_dist * cb;
-            a.out = (char *)out + (size_t)l0 * out_dist * cb;
-            a.scratch = scratch;
-            a.ntrans = std::min(scratch_lines, nlines - l0);
-            a.in_dist = in_dist;
-            a.out_dist = out_dist;
-            a.sp1 = sp;
-            a.sp2 = sp2;
-            a.w1 = sgroup;
-            a.w2 = sgroup2;
-            a.tw1 = tw_a;
-            a.tw2t = tw_b;
-            a.tw2 = tw2;
-            a.scale = scale;
-            hipError_t e = launch_smooth4(prec, dir, a, s);
-            if (e != hipSuccess) return e;
+            const long long cnt = std::min(scratch_lines, nlines - l0);
+            for (int p = 0; p < tiles->phases; p++) {
+                const bool head = p == 0, tail = p + 1 == tiles->phases;
+                MixTileArgs a{};
+                a.in = head ? (const char *)in + (size_t)l0 * in_dist * cb : scratch;
+                a.out = tail ? (char *)out + (size_t)l0 * out_dist * cb : scratch;
+                a.in_dist = head ? in_dist : tiles->elems;
+                a.out_dist = tail ? out_dist : tiles->elems;
+                a.ntrans = cnt;
+                a.inverse = dir > 0 ? 1 : 0;
+                a.scale = scale;
+                a.ph = tiles->ph[p];
+                const hipError_t e = launch_mix_tile(prec, a, s);
+                if (e != hipSuccess) return e;
+            }
         }
         return hipSuccess;
     }

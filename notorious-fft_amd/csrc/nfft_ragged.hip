@@ -40,7 +40,6 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <tuple>
 #include <vector>
 
 #include "../../include/notorious_fft_hip.h"
@@ -64,12 +63,6 @@ int env_int_rg(const char *name, int dflt)
 {
     const char *v = getenv(name);
     return v && *v ? atoi(v) : dflt;
-}
-bool smooth7(long long v)
-{
-    for (int q : {2, 3, 5, 7})
-        while (v % q == 0) v /= q;
-    return v == 1;
 }
 // Tile size (points per thread of a tile) and scratch budget (quarters of the
 // default) of the batch being created: set by the autotuner around its
@@ -238,77 +231,6 @@ static void tune_store(const std::string &key, int val)
 static int setup_fail(long long fails0) { return alloc_failures() > fails0 ? NFFT_E_ALLOC : NFFT_E_HIP; }
 
 namespace {
-// Schedules of the tiles of one batch: `points` per tile.
-struct TileFit {
-    bool ok = false;
-    MixPlan plan;
-    double cost = 0;  // per line, memory included
-};
-struct TileFits {
-    int prec, points;
-    std::map<std::tuple<int, int, int>, TileFit> seen;
-
-    // points of a 128-byte segment
-    int seg() const { return prec == F32 ? 16 : 8; }
-    // lines of L points, in tiles; strided: neighbouring lines are the ones
-    // contiguous in memory, so a tile should span 128 bytes of them
-    const TileFit &get(int L, MixLanes lanes, bool blue)
-    {
-        auto it = seen.find({L, (int)lanes, blue ? 1 : 0});
-        if (it != seen.end()) return it->second;
-        TileFit f;
-        int g = std::max(1, points / L);
-        if (lanes != MIX_LANES_POINTS && g > seg()) g -= g % seg();
-        g = std::min(g, 64);
-        for (; g >= 1 && !f.ok; g = g > 1 ? (g + 1) / 2 : 0) {
-            MixShape sh;
-            sh.g_min = sh.g_max = g;
-            sh.nth_min = sh.nth_max = kTileThreads;
-            sh.lanes = lanes;
-            // as many workgroups per CU as their registers allow (4 / 2)
-            if (points <= 16 * kTileThreads) sh.lds_max = prec == F32 ? kMixLds / 4 : kMixLds / 2;
-            f.ok = mix_fit(prec, L, blue, sh, &f.plan, &f.cost);
-        }
-        // a point read and written takes half an issue slot of its CU's share
-        // of the memory bandwidth, more where a tile covers part of a segment
-        if (f.ok)
-            f.cost += 0.5 * (prec == F32 ? 1 : 2) * L *
-                      (lanes == MIX_LANES_POINTS ? 1.0 : std::max(1.0, (double)seg() / f.plan.G));
-        return seen.emplace(std::make_tuple(L, (int)lanes, blue ? 1 : 0), f).first->second;
-    }
-    // cost of all lines of a phase
-    static double phase(const TileFit &f, int lines)
-    {
-        return f.ok ? f.cost * f.plan.G * ((lines + f.plan.G - 1) / f.plan.G) : 1e300;
-    }
-};
-
-// N = n1 x n2 (both 7-smooth) in two phases, or M = n1 x n2 >= 2N - 1 in three
-bool best_split(TileFits &fits, long long n, bool blue, int *n1, int *n2)
-{
-    double best = 1e299;
-    const long long lo = 2 * n - 1;
-    for (int a = 32; a <= 1024; a++) {
-        if (!smooth7(a) || (!blue && n % a)) continue;
-        int b = (int)(blue ? (lo + a - 1) / a : n / a), tries = blue ? 2 : 1;
-        for (; tries > 0 && b <= 2048; b++) {
-            // Bluestein: rows of whole segments, so that tiles of columns are aligned
-            if (!smooth7(b) || (blue && b % fits.seg())) continue;
-            tries--;
-            if (b < 32) continue;
-            double c = TileFits::phase(fits.get(a, MIX_LANES_LINES, false), b);
-            if (blue) c = 2 * c + TileFits::phase(fits.get(b, MIX_LANES_POINTS, true), a);
-            else c += TileFits::phase(fits.get(b, MIX_LANES_TRANSPOSE, false), a);
-            if (c < best) {
-                best = c;
-                *n1 = a;
-                *n2 = b;
-            }
-        }
-    }
-    return best < 1e299;
-}
-
 enum Kind { K_GROUP, K_GROUP_BLUE, K_TWO, K_THREE };
 struct Size {
     Kind kind = K_GROUP;
@@ -412,7 +334,7 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
     // schedules and tables of every size
     // 16 points per thread of a tile: four workgroups (FP32) share a CU
     const int gpt = std::max(1, env_int_rg("NFFT_RAGGED_GPT", t_rag_shape.gpt > 0 ? t_rag_shape.gpt : 16));
-    TileFits fits{prec, std::min(gpt, 32) * kTileThreads, {}};
+    TileFits fits{prec, std::min(gpt, 32) * kTileThreads, kTileThreads, {}};
     std::vector<MixPhase> phases;
     long long h_elems = 0;
     for (auto &kv : by_size) {
@@ -457,48 +379,26 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
             phases.push_back(ph);
             continue;
         }
-        if (!best_split(fits, n, blue, &z.n1, &z.n2)) {
+        TilePlan tp;
+        const TileStatus ts = tile_plan(fits, n, blue, &tp);
+        if (ts == TILE_FAILED) return fail("ragged setup: twiddle tables");
+        if (ts == TILE_NONE) {
             set_error("ragged setup: no split");
             ragged_free(r);
             return NFFT_E_UNSUPPORTED;
         }
         z.kind = blue ? K_THREE : K_TWO;
-        Tw2 tw2;
-        const void *t1 = phase_table(prec, z.n1, 1, 0, z.n1), *t2 = phase_table(prec, z.n2, 1, 0, z.n2);
-        if (!t1 || !t2 || !tw2_table((long long)z.n1 * z.n2, &tw2)) return fail("ragged setup: twiddle tables");
-        ph.tw2 = tw2;
-        // columns; the scratch holds rows of whole segments
-        const int pitch = (z.n2 + fits.seg() - 1) / fits.seg() * fits.seg();
-        z.elems = (long long)z.n1 * pitch;
-        ph.pl = fits.get(z.n1, MIX_LANES_LINES, false).plan;
-        ph.tw = t1;
-        ph.ig = ph.og = 1;
-        ph.ip = z.n2;
-        ph.op = pitch;
-        ph.lines = z.n2;
-        ph.flags = MIX_HEAD | MIX_TW | (blue ? MIX_CHIRP_IN : 0);
-        phases.push_back(ph);
-        MixPhase rows = ph;
-        rows.pl = fits.get(z.n2, blue ? MIX_LANES_POINTS : MIX_LANES_TRANSPOSE, blue).plan;
-        rows.tw = t2;
-        rows.ig = pitch;
-        rows.ip = 1;
-        rows.lines = z.n1;
+        z.n1 = tp.n1;
+        z.n2 = tp.n2;
+        z.elems = tp.elems;
         if (blue) {
-            z.m = z.n1 * z.n2;
+            z.m = tp.n1 * tp.n2;
             z.h = h_elems;
             h_elems += z.m;
-            rows.og = pitch;
-            rows.op = 1;
-            rows.flags = MIX_TW;
-            phases.push_back(rows);
-            ph.flags = MIX_TAIL | MIX_CHIRP_OUT;
-            phases.push_back(ph);
-        } else {
-            rows.og = 1;
-            rows.op = z.n1;
-            rows.flags = MIX_TAIL;
-            phases.push_back(rows);
+        }
+        for (int k = 0; k < tp.phases; k++) {
+            tp.ph[k].chirp = ph.chirp;
+            phases.push_back(tp.ph[k]);
         }
         for (size_t k = z.phase; k < phases.size(); k++)
             r->tile_lds = std::max(r->tile_lds, (size_t)phases[k].pl.lp * phases[k].pl.G * cb);

@@ -1,6 +1,7 @@
 """One-pass mixed-radix lines (nfft_kernels_mix.h) against pocketfft: one to
 six stages, groups of lines with a ragged last group, the longest lines of
-each precision, and Bluestein over a 7-smooth M in one workgroup.
+each precision, Bluestein over a 7-smooth M in one workgroup, and both in
+phases of tiles (last tiles of a few columns, rows padded to whole segments).
 
 Tolerance: each point passes about log2(N) levels of butterflies, with a
 handful of roundings (sums, one twiddle product of two rounded factors) per
@@ -49,6 +50,25 @@ def test_bluestein_one_pass(pkg, dev, prec, n):
     tol = 2 * 4 * EPS[prec] * math.sqrt(math.log2(n))
     for batch in (1, 3):
         x = rounded(ol.uniform(42, 2 * n * batch), prec)
+        for op, inplace in (("dft", False), ("invdft", True)):
+            got = run_plan(pkg, dev, op, [n], x, batch, prec, inplace=inplace)
+            err = ol.rel_l2(got, pocket(op, [n], x, batch))
+            assert err < tol, (prec, n, batch, op, inplace, err, desc)
+
+
+@pytest.mark.parametrize("prec,n", [("f32", n) for n in (20736, 22050, 65610, 196608, 1000000)] +
+                         [("f64", n) for n in (10290, 15625, 65610, 196608, 1000000)] +
+                         [("f32", n) for n in (10247, 10301, 16381, 33333, 65537, 100003)] +
+                         [("f64", n) for n in (17011, 33331, 65537, 70001)])
+def test_tiles(pkg, dev, prec, n):
+    plan = pkg.Plan("dft", prec, [n], 1)
+    desc = plan.describe()
+    plan.close()
+    blue = not desc.startswith("mixed-radix four-step")
+    assert not blue or "in tiles" in desc, desc
+    tol = (2 if blue else 1) * 4 * EPS[prec] * math.sqrt(math.log2(n))
+    for batch in (1, 3):
+        x = rounded(ol.uniform(44, 2 * n * batch), prec)
         for op, inplace in (("dft", False), ("invdft", True)):
             got = run_plan(pkg, dev, op, [n], x, batch, prec, inplace=inplace)
             err = ol.rel_l2(got, pocket(op, [n], x, batch))
