@@ -47,15 +47,28 @@ __global__ void __launch_bounds__((wpow_threads<L, LPB>())) k_col_wpow(WpowArgs 
     __shared__ double red[NTH / 64];
     if constexpr (S::S > 1) stage_tw_to_lds<T, L>(ltw, (const double2 *)a.tw);
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
-    const long long tile = blockIdx.x + (long long)gridDim.x * blockIdx.y;  // (transform, column tile)
+    // neighbouring tiles on one XCD: 2048-point columns fit 8 FP32 columns, half
+    // a 128-byte line, whose other half the next tile reads and writes
+    const long long tile = xcd_logical(blockIdx.x + (long long)gridDim.x * blockIdx.y,
+                                       (long long)gridDim.x * gridDim.y);  // (transform, column tile)
     const long long t = tile / gridDim.x;
     const int c0 = (int)(tile % gridDim.x) * LPB, c = c0 + b;
     const bool valid = c < a.ncols;
+    // uniform: every column of the tile exists and tile offsets fit 32 bits
+    const bool full = c0 + LPB <= a.ncols && off_fits<C>((long long)L * a.ncols);
     C *col = (C *)a.buf + t * a.dist + c;
     const T *w = (const T *)a.w + c;
+    const auto rs = buf_rsrc((C *)a.buf + t * a.dist + c0);
+    const uint32_t off = (uint32_t)(j * a.ncols + b) * (uint32_t)sizeof(C);
+    const uint32_t qst = (uint32_t)(S::NT * a.ncols) * (uint32_t)sizeof(C);
     C reg[S::R];
+    if (full) {
 #pragma unroll
-    for (int q = 0; q < S::R; q++) reg[q] = valid ? col[(long long)(j + S::NT * q) * a.ncols] : czero<T>();
+        for (int q = 0; q < S::R; q++) reg[q] = buf_ld<C>(rs, off, q * qst);
+    } else {
+#pragma unroll
+        for (int q = 0; q < S::R; q++) reg[q] = valid ? col[(long long)(j + S::NT * q) * a.ncols] : czero<T>();
+    }
     __syncthreads();  // stage table in LDS
     LayCol<LPB> lay{b};
     line_fft_tw<T, L, -1>(reg, lds, lay, j, StageTwLds<T>{ltw});
@@ -69,7 +82,10 @@ __global__ void __launch_bounds__((wpow_threads<L, LPB>())) k_col_wpow(WpowArgs 
         reg[q] = cscale(y, (T)2 * w2);
     }
     line_fft_tw<T, L, 1>(reg, lds, lay, j, StageTwLds<T>{ltw});
-    if (valid) {
+    if (full) {
+#pragma unroll
+        for (int q = 0; q < S::R; q++) buf_st<C>(rs, off, q * qst, reg[q]);
+    } else if (valid) {
 #pragma unroll
         for (int q = 0; q < S::R; q++) col[(long long)(j + S::NT * q) * a.ncols] = reg[q];
     }
