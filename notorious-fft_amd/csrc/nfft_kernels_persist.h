@@ -58,10 +58,12 @@ struct PersistArgs {
     int grab;                     // consecutive items taken per queue access (>= 1)
 };
 
-// Counter block: [0] queue head, [1] error flag of this launch, [2] sticky
-// error (previous launches), [3, 3+T) pass-1 tiles done per transform,
-// [3+T, 3+2T) pass-2 tiles done per transform.
-__host__ __device__ constexpr long long persist_ctr_words(long long ntrans) { return 3 + 2 * ntrans; }
+// Counter block (32-bit words): [1] error flag of this launch, [2] sticky
+// error (previous launches); then, each in a 128-byte line of its own (they
+// are polled while others are added to): the queue head, and per transform
+// the pass-1 and the pass-2 tiles done.
+constexpr int kPersistLine = 32;
+__host__ __device__ constexpr long long persist_ctr_words(long long ntrans) { return kPersistLine * (2 + 2 * ntrans); }
 
 // Agent-scope (sc1) store / load of one complex element.
 __device__ __forceinline__ void coh_store(Cx<float> *p, Cx<float> v)
@@ -158,11 +160,13 @@ __device__ __forceinline__ bool persist_decode(long long i, long long T, long lo
 __device__ __forceinline__ void persist_wait(const unsigned *c, unsigned need, unsigned *err, long long timeout)
 {
     const unsigned long long t0 = wall_clock64();
-    while (__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
-        if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-        if ((long long)(wall_clock64() - t0) > timeout) {
-            atomicOr(err, 1u);
-            return;
+    for (unsigned i = 1; __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need; i++) {
+        if (i % 256 == 0) {  // one line for every workgroup: not at each poll
+            if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+            if ((long long)(wall_clock64() - t0) > timeout) {
+                atomicOr(err, 1u);
+                return;
+            }
         }
         __builtin_amdgcn_s_sleep(1);
     }
@@ -182,7 +186,9 @@ k_four_persist(PersistArgs a)
     __shared__ C lds[Sh::LDS];
     __shared__ int s_item[3];  // kind, transform, tile
     const long long ntr = a.ntrans;
-    unsigned *head = a.ctr, *err = a.ctr + 1, *done1 = a.ctr + 3, *done2 = a.ctr + 3 + ntr;
+    unsigned *head = a.ctr + kPersistLine, *err = a.ctr + 1;
+    auto done1 = [&](long long tr) { return a.ctr + kPersistLine * (2 + 2 * tr); };
+    auto done2 = [&](long long tr) { return a.ctr + kPersistLine * (3 + 2 * tr); };
     // Lane 0 of wave 0 publishes the finished item and fetches the next one
     // in a single region at the top of the loop, entered through a
     // wave-uniform branch: a second lane-divergent region between the
@@ -203,7 +209,7 @@ k_four_persist(PersistArgs a)
         if (wave0) {
             if (threadIdx.x == 0) {
                 if (kind != 0)  // completion of the previous item
-                    __hip_atomic_fetch_add(kind == 1 ? done1 + t : done2 + t, 1u, __ATOMIC_RELAXED,
+                    __hip_atomic_fetch_add(kind == 1 ? done1(t) : done2(t), 1u, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
                 int nk = 0, ntile = 0;
                 long long nt = 0;
@@ -213,8 +219,8 @@ k_four_persist(PersistArgs a)
                 }
                 const long long i = base + sub++;
                 if (persist_decode(i, ntr, a.lag, Sh::A, Sh::B, &nk, &nt, &ntile)) {
-                    if (nk == 2) persist_wait(done1 + nt, (unsigned)Sh::A, err, a.timeout);
-                    else if (nt >= a.slots) persist_wait(done2 + (nt - a.slots), (unsigned)Sh::B, err, a.timeout);
+                    if (nk == 2) persist_wait(done1(nt), (unsigned)Sh::A, err, a.timeout);
+                    else if (nt >= a.slots) persist_wait(done2(nt - a.slots), (unsigned)Sh::B, err, a.timeout);
                 }
                 s_item[0] = nk;
                 s_item[1] = (int)nt;

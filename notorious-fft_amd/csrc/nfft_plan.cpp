@@ -506,7 +506,7 @@ static bool persist_default(int prec, long long n) { return prec == F64 && n >= 
 // in the 256 MB Infinity Cache.
 static const long long kPersistSlotBytes = 128LL << 20;
 // Transforms per persistent launch (bounds the counter block).
-static const long long kPersistCap = 1LL << 15;
+static const long long kPersistCap = 1LL << 13;
 
 static bool persist_setup(C2C &c)
 {
