@@ -13,6 +13,7 @@
 #include "nfft_kernels.h"
 #include "nfft_kernels_persist.h"
 #include "nfft_kernels_xcd.h"
+#include "nfft_kernels_team.h"
 #include "nfft_kernels_smooth.h"
 #include "nfft_kernels_mix.h"
 #include "nfft_kernels_rt.h"
@@ -164,6 +165,13 @@ bool xcd_topology(int *nq, signed char *qmap);
 // twrow: inter-pass twiddle in the row tiles (FP32 table) or the column tiles
 hipError_t launch_four_xcd(int n1, int dir, bool twrow, const XcdArgs &a, int grid, hipStream_t s);
 
+// Team four-step (nfft_k_team.hip): the shape of a length, if it has one
+struct TeamCfg {
+    int id = -1, n1 = 0, n2 = 0, tiles = 0, per_cu = 0;  // per_cu: resident workgroups
+};
+bool team_find(int prec, long long n, TeamCfg *cfg);
+hipError_t launch_four_team(const TeamCfg &c, int dir, const TeamArgs &a, int grid, hipStream_t s);
+
 // Schedules of the mixed-radix lines and tiles (nfft_k_mix.hip).
 // How lanes map to the points of a workgroup's lines: neighbouring points
 // (contiguous lines), neighbouring lines (columns), or points on the first
@@ -311,6 +319,13 @@ struct C2C {
     int xgrid = 0;                    // workgroups of the launch
     int xnq = 0;                      // XCD queues and the XCC_ID -> queue map
     signed char xqmap[kXcdIds] = {};
+    // ALG_FOUR in one launch through the XCDs' L2 (k_four_team) when tctr is
+    // set and a batch has at least tmin transforms
+    unsigned *tctr = nullptr;         // owned: counter block for up to xcap transforms
+    TeamCfg tcfg{};
+    int tslots = 0;                   // intermediate slots per queue
+    long long tmin = 0;
+    const void *ttw_a = nullptr, *ttw_b = nullptr;  // stage tables of its split
 
     // Set up tables for length n; returns false with the error set.
     // smooth_mode for 7-smooth non-power-of-two n: 2 = choose (tuned /

@@ -578,6 +578,41 @@ static int xcd_setup(C2C &c)
     return 1;
 }
 
+// The team four-step (k_four_team) of the lengths that have a shape for it,
+// beside the length's other path, which runs smaller batches than tmin and
+// the ones with less scratch than its slots.  NFFT_TEAM=0 turns it off.
+// Returns false on an error (error set).
+static bool team_setup(C2C &c)
+{
+    if (env_int("NFFT_TEAM", 1) == 0 || !team_find(c.prec, c.n, &c.tcfg)) return true;
+    int dev = 0, ncu = 0, khz = 0;
+    if (!hip_ok(hipGetDevice(&dev), "hipGetDevice") ||
+        !hip_ok(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "device attribute") ||
+        !hip_ok(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev), "device attribute"))
+        return false;
+    if (!xcd_topology(&c.xnq, c.xqmap)) return true;  // not applicable on this device
+    c.ttw_a = stage_table(c.prec, c.tcfg.n1);
+    c.ttw_b = stage_table(c.prec, c.tcfg.n2);
+    if (!c.ttw_a || !c.ttw_b) return false;
+    const size_t bytes = (size_t)team_ctr_words(kXcdCap, c.xnq) * sizeof(unsigned);
+    if (!hip_ok(dev_malloc(&c.tctr, bytes), "hipMalloc")) return false;
+    if (!hip_ok(hipMemset(c.tctr, 0, bytes), "hipMemset")) {
+        (void)hipFree(c.tctr);
+        c.tctr = nullptr;
+        return false;
+    }
+    c.xcap = kXcdCap;
+    c.xgrid = std::max(1, ncu) * c.tcfg.per_cu;
+    c.ptimeout = (long long)(kPersistTimeoutSec * 1000.0 * std::max(khz, 1000));
+    // three quarters of an L2; two at least, so that a team can start on its
+    // next transform while the last one's rows are read
+    c.tslots = (int)std::max(2LL, (3LL << 20) / ((long long)c.n * (long long)cx_bytes(c.prec)));
+    // two tiles a workgroup (2^15 x 96 43.6 against 48.1 us, x 128 55.1 / 52.1;
+    // 2^17 x 32 55.7 / 50.8)
+    c.tmin = (2LL * c.xgrid + c.tcfg.tiles - 1) / c.tcfg.tiles;
+    return true;
+}
+
 bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
 {
     n = n_;
@@ -680,7 +715,11 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
         }
         tw_a = stage_table(prec, n1);
         tw_b = stage_table(prec, n2);
-        return tw_a && tw_b && tw2_table(n, &tw2);
+        if (!tw_a || !tw_b || !tw2_table(n, &tw2)) return false;
+        // where no other split or path is asked for
+        const bool asked = t_four_force.lg2 >= 0 || tuned_four(prec, n).lg2 >= 0 || env_int("NFFT_TUNE", 0) ||
+                           getenv("NFFT_FOUR_N2") || getenv("NFFT_PERSIST") || getenv("NFFT_XCD");
+        return persist_mode == 0 || asked || xctr || team_setup(*this);
     }
     // 7-smooth lengths: mixed radix (the reference uses Bluestein for every
     // non-power-of-two length; results agree to rounding) where it is the
@@ -824,6 +863,8 @@ void C2C::release()
     pctr = nullptr;
     if (xctr) (void)hipFree(xctr);
     xctr = nullptr;
+    if (tctr) (void)hipFree(tctr);
+    tctr = nullptr;
     for (auto *sub : {&sub1, &sub2}) {
         if (*sub) (*sub)->release();
         sub->reset();
@@ -832,7 +873,7 @@ void C2C::release()
 
 bool C2C::device_fault() const
 {
-    for (unsigned *c : {pctr, xctr}) {
+    for (unsigned *c : {pctr, xctr, tctr}) {
         if (!c) continue;
         unsigned w[2] = {0, 0};
         if (hipMemcpy(w, c + 1, sizeof w, hipMemcpyDeviceToHost) != hipSuccess) return true;
@@ -843,7 +884,7 @@ bool C2C::device_fault() const
 
 std::string C2C::describe() const
 {
-    char b[128];
+    char b[192];
     switch (algo) {
     case ALG_LINE:
         snprintf(b, sizeof b, halves ? "line %d (exchanges in two LDS halves)" : "line %d", n);
@@ -857,6 +898,11 @@ std::string C2C::describe() const
                      n1, n2, xgrid);
         else
             snprintf(b, sizeof b, "four-step %dx%d", n1, n2);
+        if (tctr) {
+            const size_t o = strlen(b);
+            snprintf(b + o, sizeof b - o, "; from %lld transforms %dx%d in teams of %d workgroups", tmin, tcfg.n1, tcfg.n2,
+                     tcfg.tiles);
+        }
         break;
     case ALG_BLUE1: snprintf(b, sizeof b, "bluestein N=%d M=%d single-pass", n, m); break;
     case ALG_TILE:
@@ -931,6 +977,32 @@ hipError_t C2C::run(const void *in, void *out, long long nlines, long long in_di
     }
     case ALG_FOUR: {
         if (scratch_lines < 1 || !scratch) return hipErrorInvalidValue;
+        if (tctr && !t_noalloc && nlines >= tmin && scratch_lines >= (long long)xnq * tslots) {
+            // one launch per xcap transforms; the scratch holds the slots
+            for (long long l0 = 0; l0 < nlines; l0 += xcap) {
+                const long long cnt = std::min(xcap, nlines - l0);
+                TeamArgs a{};
+                a.in = (const char *)in + (size_t)l0 * in_dist * cb;
+                a.out = (char *)out + (size_t)l0 * out_dist * cb;
+                a.ntrans = cnt;
+                a.in_dist = in_dist;
+                a.out_dist = out_dist;
+                a.scratch = scratch;
+                a.slots = tslots;
+                a.ctr = tctr;
+                a.tw_a = ttw_a;
+                a.tw_b = ttw_b;
+                a.tw2 = tw2;
+                a.scale = scale;
+                a.timeout = ptimeout;
+                a.nq = xnq;
+                for (int i = 0; i < kXcdIds; i++) a.qmap[i] = xqmap[i];
+                hipError_t e = launch_persist_reset(tctr, team_ctr_words(cnt, xnq), s);
+                if (e == hipSuccess) e = launch_four_team(tcfg, dir, a, xgrid, s);
+                if (e != hipSuccess) return e;
+            }
+            return hipSuccess;
+        }
         if (pctr && !t_noalloc) {
             // one persistent launch per kPersistCap transforms; the scratch
             // holds the rotating intermediate slots
