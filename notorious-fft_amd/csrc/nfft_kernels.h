@@ -378,7 +378,7 @@ k_col(ColArgs a)
     if constexpr (TWL) stage_tw_to_lds<T, L>(ltw, (const double2 *)a.tw);
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
     const long long lin = blockIdx.x + (long long)gridDim.x * (blockIdx.y + (long long)gridDim.y * blockIdx.z);
-    const long long lg = xcd_logical(lin, (long long)gridDim.x * gridDim.y * gridDim.z);
+    const long long lg = xcd_columns<T>(lin, (long long)gridDim.x * gridDim.y * gridDim.z);
     const int c0 = (int)(lg % gridDim.x) * LPB, c = c0 + b;
     const long long t = lg / gridDim.x;
     const bool valid = c < a.ncols && t < a.ntrans;

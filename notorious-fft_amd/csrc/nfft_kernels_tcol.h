@@ -66,7 +66,7 @@ k_t23_col(TrigColArgs a)
     using C = Cx<T>;
     __shared__ C lds[N * LPB];
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
-    const TrigCol<C> col(a, xcd_logical(blockIdx.x, gridDim.x) * LPB, b);
+    const TrigCol<C> col(a, xcd_columns<T>(blockIdx.x, gridDim.x) * LPB, b);
     const C *w = (const C *)a.t1;
     const T sc = (T)a.scale;
     const LayCol<LPB> lay{b};
@@ -128,7 +128,7 @@ k_t4_col(TrigColArgs a)
     using C = Cx<T>;
     __shared__ C lds[N * LPB];
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
-    const TrigCol<C> col(a, xcd_logical(blockIdx.x, gridDim.x) * LPB, b);
+    const TrigCol<C> col(a, xcd_columns<T>(blockIdx.x, gridDim.x) * LPB, b);
     const C *pre = (const C *)a.t1, *post = (const C *)a.t2;
     const T sc = (T)2 * (T)a.scale;
     const LayCol<2 * LPB> lay[2] = {{b}, {b + LPB}};  // real parts, imaginary parts

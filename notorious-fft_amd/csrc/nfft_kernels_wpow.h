@@ -49,7 +49,7 @@ __global__ void __launch_bounds__((wpow_threads<L, LPB>())) k_col_wpow(WpowArgs 
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
     // neighbouring tiles on one XCD: 2048-point columns fit 8 FP32 columns, half
     // a 128-byte line, whose other half the next tile reads and writes
-    const long long tile = xcd_logical(blockIdx.x + (long long)gridDim.x * blockIdx.y,
+    const long long tile = xcd_columns<T>(blockIdx.x + (long long)gridDim.x * blockIdx.y,
                                        (long long)gridDim.x * gridDim.y);  // (transform, column tile)
     const long long t = tile / gridDim.x;
     const int c0 = (int)(tile % gridDim.x) * LPB, c = c0 + b;
