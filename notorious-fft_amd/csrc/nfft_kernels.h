@@ -176,8 +176,8 @@ __global__ void __launch_bounds__(Sched<L>::NT *line_lpb<L>()) k_line(LineArgs a
 // 16 points (set l of thread j: points j + l NT/2 + NT q), with each
 // Stockham exchange made through an LDS buffer of half a line in two steps.
 // Every value a stage writes lands in a half known at compile time:
-//   - stage 0 (Ns = 1, radix R0, m = 16 / R0 >= 2 butterflies per set):
-//     butterfly i < m / 2 of either set writes points < L / 2;
+//   - stage 0 (Ns = 1, radix R0, m = 16 / R0 butterflies per set): butterfly
+//     i < m / 2 of either set writes points < L / 2; with R0 = 16, set 0 does;
 //   - a twiddled stage s < S - 1 (Ns <= L / 256, so 16 Ns divides L / 2):
 //     set 0 (j < NT / 2) writes the lower half, set 1 the upper;
 //   - the reads of q < 8 (points < 8 NT = L / 2) come from the lower half.
@@ -203,15 +203,16 @@ template <typename T, int L> __host__ __device__ constexpr int line_h_wpe()
     return w < 1 ? 1 : (w > 4 ? 4 : (int)w);
 }
 
-template <typename T, int L, int DIR>
-__device__ __forceinline__ void line_fft_halves(Cx<T> (&reg)[2][16], Cx<T> *lds, int j0, const double2 *__restrict__ tw)
+// lay: LDS index of point p < L / 2 of the half; twsrc: stage bases.
+template <typename T, int L, int DIR, class Lay, class Tw>
+__device__ __forceinline__ void line_fft_halves(Cx<T> (&reg)[2][16], Cx<T> *lds, const Lay &lay, int j0, const Tw &twsrc)
 {
     using S = Sched<L>;
     using C = Cx<T>;
-    static_assert(line_h_ok<T, L>(), "half-buffer line shape");
+    static_assert(S::S >= 2 && S::R == 16 && (S::NT / 2) * 2 == S::NT, "half-buffer line shape");
     constexpr int H = L / 2, NH = S::NT / 2;
     const int jj[2] = {j0, j0 + NH};
-    double2 bw[2][4];
+    typename Tw::B bw[2][4];
     sfor<0, S::S>([&](auto sc) {
         constexpr int s = decltype(sc)::value;
         constexpr int Rs = S::radix(s), Ns = S::ns(s), m = S::R / Rs;
@@ -220,15 +221,14 @@ __device__ __forceinline__ void line_fft_halves(Cx<T> (&reg)[2][16], Cx<T> *lds,
             constexpr int s2 = decltype(sn)::value;
             constexpr bool same = NH % S::ns(s2) == 0;
 #pragma unroll
-            for (int l = 0; l < (same ? 1 : 2); l++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) bw[l][e] = tw[S::twoff(s2) + (jj[l] & (S::ns(s2) - 1)) * 4 + e];
+            for (int l = 0; l < (same ? 1 : 2); l++) twsrc.load(S::twoff(s2) + (jj[l] & (S::ns(s2) - 1)) * 4, bw[l]);
             if constexpr (same) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) bw[1][e] = bw[0][e];
             }
         };
-        if constexpr (s == 0) bases(std::integral_constant<int, 1>{});
+        if constexpr (s == 0 && Tw::kAhead) bases(std::integral_constant<int, 1>{});
+        if constexpr (s > 0 && !Tw::kAhead) bases(sc);
 #pragma unroll
         for (int l = 0; l < 2; l++) {
 #pragma unroll
@@ -247,9 +247,8 @@ __device__ __forceinline__ void line_fft_halves(Cx<T> (&reg)[2][16], Cx<T> *lds,
             __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (s + 1 < S::S) {
-            static_assert(s > 0 || m >= 2, "stage 0 splits by butterfly");
             static_assert(s == 0 || (H % (16 * Ns) == 0 && NH % Ns == 0), "twiddled stages split by set");
-            if constexpr (s > 0) bases(std::integral_constant<int, s + 1>{});
+            if constexpr (s > 0 && Tw::kAhead) bases(std::integral_constant<int, s + 1>{});
             C lo[2][8];
 #pragma unroll
             for (int h = 0; h < 2; h++) {
@@ -257,18 +256,18 @@ __device__ __forceinline__ void line_fft_halves(Cx<T> (&reg)[2][16], Cx<T> *lds,
                 for (int l = 0; l < 2; l++)
 #pragma unroll
                     for (int i = 0; i < m; i++) {
-                        if ((s == 0 ? (2 * i >= m ? 1 : 0) : l) != h) continue;
+                        if ((s == 0 && m >= 2 ? (2 * i >= m ? 1 : 0) : l) != h) continue;
                         const int v = jj[l] + S::NT * i;
                         const int base = (v / Ns) * Ns * Rs + (v & (Ns - 1)) - h * H;
 #pragma unroll
-                        for (int r = 0; r < Rs; r++) lds[lpad<T>(base + r * Ns)] = reg[l][i + r * m];
+                        for (int r = 0; r < Rs; r++) lds[lay(base + r * Ns)] = reg[l][i + r * m];
                     }
                 __syncthreads();
 #pragma unroll
                 for (int l = 0; l < 2; l++)
 #pragma unroll
                     for (int q = 0; q < 8; q++) {
-                        const C v = lds[lpad<T>(jj[l] + S::NT * q)];  // point jj + NT (q + 8 h) - h H
+                        const C v = lds[lay(jj[l] + S::NT * q)];  // point jj + NT (q + 8 h) - h H
                         if (h == 0) lo[l][q] = v;
                         else reg[l][q + 8] = v;
                     }
@@ -300,7 +299,7 @@ __global__ void __launch_bounds__(Sched<L>::NT / 2, (line_h_wpe<T, L>())) k_line
     for (int l = 0; l < 2; l++)
 #pragma unroll
         for (int q = 0; q < 16; q++) reg[l][q] = buf_ld<C>(rs, off, (uint32_t)((l * NH + S::NT * q) * sizeof(C)));
-    line_fft_halves<T, L, DIR>(reg, lds, j, (const double2 *)a.tw);
+    line_fft_halves<T, L, DIR>(reg, lds, LayLine<T, L>{0}, j, StageTwGlobal{(const double2 *)a.tw});
     const T sc = (T)a.scale;
     const auto rd = buf_rsrc((C *)a.out + line * a.out_dist);
 #pragma unroll
@@ -338,6 +337,7 @@ struct ColArgs {
     int conj;                  // Bluestein: conjugate input / output
     double scale;
     int lpb;                   // columns per workgroup (0: default for L)
+    int four;                  // first pass of a four-step
 };
 
 template <int L, int LPB> __host__ __device__ constexpr int col_threads() { return Sched<L>::NT * LPB; }
@@ -450,6 +450,84 @@ k_col(ColArgs a)
             if (sc != (T)1) v = cscale(v, sc);
             dst[(long long)(j + S::NT * q) * a.S] = v;
         }
+    }
+}
+
+// k_col_h: k_col (plain or twiddle) with the exchanges through half a tile of
+// LDS (as k_line_h), NT / 2 threads per column and two sets of 16 points each:
+// two of k_col's tiles on a CU at a time, or one of twice the columns.
+// Bounds and where which is used: col_form (nfft_launch_impl.h).
+template <typename T, int L, int LPB> __host__ __device__ constexpr size_t col_h_lds()
+{
+    return ((size_t)L / 2 * LPB + Sched<L>::TWN) * sizeof(Cx<T>);
+}
+template <typename T, int L, int LPB> __host__ __device__ constexpr int col_h_wpe()
+{
+    const int wg = (int)(160 * 1024 / col_h_lds<T, L, LPB>());
+    const int w = (wg < 1 ? 1 : wg) * (Sched<L>::NT / 2 * LPB / 64) / 4, most = sizeof(T) == 4 ? 4 : 2;
+    return w < 1 ? 1 : w > most ? most : w;
+}
+
+template <typename T, int L, int LPB, int DIR, int MODE>
+__global__ void __launch_bounds__((Sched<L>::NT / 2 * LPB), (col_h_wpe<T, L, LPB>())) k_col_h(ColArgs a)
+{
+    using S = Sched<L>;
+    using C = Cx<T>;
+    constexpr int NH = S::NT / 2;
+    __shared__ C lds[L / 2 * LPB];
+    __shared__ C ltw[S::TWN];
+    const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
+    const long long lin = blockIdx.x + (long long)gridDim.x * (blockIdx.y + (long long)gridDim.y * blockIdx.z);
+    const long long lg = xcd_columns<T>(lin, (long long)gridDim.x * gridDim.y * gridDim.z);
+    const int c0 = (int)(lg % gridDim.x) * LPB, c = c0 + b;
+    const long long t = lg / gridDim.x;
+    const bool valid = c < a.ncols && t < a.ntrans;
+    const bool full = c0 + LPB <= a.ncols && t < a.ntrans && off_fits<C>((long long)L * a.S);
+    const uint32_t qst = (uint32_t)(S::NT * a.S) * (uint32_t)sizeof(C), lst = (uint32_t)(NH * a.S) * (uint32_t)sizeof(C);
+    const uint32_t loff = (uint32_t)(j * a.S + b) * (uint32_t)sizeof(C);
+    C reg[2][16];
+    if (full) {
+        const auto rs = buf_rsrc((const C *)a.in + t * a.in_dist + c0);
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) reg[l][q] = buf_ld<C>(rs, loff, l * lst + q * qst);
+    } else {
+        const C *src = (const C *)a.in + t * a.in_dist + c;
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 16; q++)
+                reg[l][q] = valid ? src[(long long)(j + l * NH + S::NT * q) * a.S] : czero<T>();
+    }
+    stage_tw_to_lds<T, L>(ltw, (const double2 *)a.tw);  // visible after the first exchange's barriers
+    line_fft_halves<T, L, DIR>(reg, lds, LayCol<LPB>{b}, j, StageTwLds<T>{ltw});
+    if constexpr (MODE == COL_TWIDDLE) {
+        const uint32_t cc = valid ? (uint32_t)c : 0u;
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+            apply_tw2_series<DIR>(reg[l], a.tw2, cc * (uint32_t)(j + l * NH), cc * (uint32_t)S::NT);
+    }
+    if (!valid) return;
+    const T sc = (T)a.scale;
+    if (sc != (T)1) {
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) reg[l][q] = cscale(reg[l][q], sc);
+    }
+    if (full) {
+        const auto rd = buf_rsrc((C *)a.out + t * a.out_dist + c0);
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) buf_st<C>(rd, loff, l * lst + q * qst, reg[l][q]);
+    } else {
+        C *dst = (C *)a.out + t * a.out_dist + c;
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) dst[(long long)(j + l * NH + S::NT * q) * a.S] = reg[l][q];
     }
 }
 

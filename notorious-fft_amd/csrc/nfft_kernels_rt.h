@@ -140,7 +140,7 @@ __global__ void __launch_bounds__(Sched<L>::NT / 2, (line_h_wpe<T, L>())) k_r2c_
 #pragma unroll
             for (int q = 0; q < 16; q++) reg[l][q] = buf_ld<C>(rs, off, (uint32_t)((l * NH + S::NT * q) * sizeof(C)));
     }
-    line_fft_halves<T, L, -1>(reg, lds, j, (const double2 *)a.tw);
+    line_fft_halves<T, L, -1>(reg, lds, LayLine<T, L>{0}, j, StageTwGlobal{(const double2 *)a.tw});
     const C *w = (const C *)a.t1;
     const C wj[2] = {w[jj[0]], w[jj[1]]};  // w[k] = w[jj] w[NT q] (the second workgroup-uniform)
     const T sc = (T)a.scale, sk = a.half ? (T)2 * sc : sc;  // half: adjoint weighting 2 on 0 < k < L
@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(Sched<L>::NT / 2, (line_h_wpe<T, L>())) k_c2r_
             }
             reg[l][q] = pack_pair(xk, xm, q == 0 ? wj[l] : cmul(wj[l], w[S::NT * q]));
         }
-    line_fft_halves<T, L, 1>(reg, lds, j, (const double2 *)a.tw);
+    line_fft_halves<T, L, 1>(reg, lds, LayLine<T, L>{0}, j, StageTwGlobal{(const double2 *)a.tw});
     const T sc = (T)a.scale;
     const auto rd = buf_rsrc((T *)a.out + line * a.out_dist);
     const uint32_t off = (uint32_t)j * (uint32_t)sizeof(C);

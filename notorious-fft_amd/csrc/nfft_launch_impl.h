@@ -127,6 +127,57 @@ hipError_t col_launch(int dir, int mode, const ColArgs &a, hipStream_t s)
 // use; other lengths always take the default width.
 template <int L> constexpr bool tunable_len() { return L >= 128 && L <= 2048; }
 
+// How a plain (or FP64 twiddle) pass of L-point columns runs, of the default
+// width w = col_lpb: 0 k_col; 1 k_col_h, w columns in half the LDS, two
+// workgroups a CU that load, transform and store past each other; 2 k_col_h,
+// 2 w columns, twice the run per row.  Two workgroups a CU need 512 tiles (2048^2
+// FP32, 256 tiles: 28.2 / 29.7 / 33.2 us for 0 / 1 / 2).  The wide tile
+// wins where 1 keeps losing whole lines between the workgroups of a row:
+// rows of whole 128-byte lines, or 2 MiB and more apart (a tile then touches
+// as many pages as it has rows).  us for 0 / 1 / 2, 2^27 FP32 or 2^26 FP64
+// points unless stated, other axes included:
+//   FP32 512: S = 1024 763 / 777 / 774, S = 2^18 1241 / 1258 / 1183
+//   FP32 1024: S = 64 927 / 917 / 947, 1024 815 / 785 / 825, 2049 996 / 935 /
+//     972, 2^18 (2^28 points) 2790 / 2545 / 2485
+//   FP32 2048: S = 64 964 / 921 / 958, 8192 983 / 1021 / 969, 1025 (2^23
+//     points) 135 / 124 / 145, 8193 1126 / 1062 / 1095
+//   FP32 4096: S = 64 1129 / 1016 / 1049, 1024 964 / 939 / 874, 1025 (2^23
+//     points) 150 / 139 / 147, (2^26) 1172 / 1102 / 1068
+//   FP64 512: S = 1024 822 / 821 / 820, 2^17 1387 / 1307 / 1245
+//   FP64 1024: S = 1024 819 / 820 / 841 (2^23 points 95 / 87 / 94), 1025 969
+//     / 984 / 956
+//   FP64 2048: S = 2048 (2^23 points) 96 / 94 / 107, 1024 860 / 945 / 852, 1025
+//     1068 / 1087 / 1009
+//   FP64 4096: S = 1024 1010 / 1088 / 908, 1025 1227 / 1330 / 1127
+template <typename T, int L> int col_form(int mode, const ColArgs &a)
+{
+    constexpr bool f32 = sizeof(T) == 4;
+    // FP32 four-step passes stay bit-identical to the single launch's
+    if (a.lpb || mode > (f32 ? COL_PLAIN : COL_TWIDDLE) || (f32 && a.four)) return 0;
+    const long long w = col_lpb<T, L>(), tiles = (a.ncols + w - 1) / w * a.ntrans, row = a.S * (long long)sizeof(Cx<T>);
+    const bool lines = row % 128 == 0, far = row >= (2LL << 20);
+    if (tiles < 512) return 0;
+    if (L == 512) return far ? 2 : 0;
+    if (L == 1024) return f32 ? (far ? 2 : 1) : (lines ? 1 : 0);
+    if (L == 2048) return f32 ? (lines && a.S >= 512 && tiles >= 1024 ? 2 : 1) : (tiles >= 4096 ? 2 : a.four ? 0 : 1);
+    if (L == 4096) return f32 ? ((lines ? a.S >= 512 : tiles >= 4096) ? 2 : 1) : (tiles >= 1024 ? 2 : 0);
+    return 0;
+}
+
+template <typename T, int L, int LPB> hipError_t col_h_launch(int dir, int mode, const ColArgs &a, hipStream_t s)
+{
+    unsigned gy, gz;
+    grid_trans(a.ntrans, gy, gz);
+    const dim3 g((unsigned)((a.ncols + LPB - 1) / LPB), gy, gz), b(Sched<L>::NT / 2 * LPB);
+    if (mode == COL_PLAIN && dir < 0) hipLaunchKernelGGL((k_col_h<T, L, LPB, -1, COL_PLAIN>), g, b, 0, s, a);
+    else if (mode == COL_PLAIN) hipLaunchKernelGGL((k_col_h<T, L, LPB, 1, COL_PLAIN>), g, b, 0, s, a);
+    else if constexpr (sizeof(T) == 8) {
+        if (dir < 0) hipLaunchKernelGGL((k_col_h<T, L, LPB, -1, COL_TWIDDLE>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((k_col_h<T, L, LPB, 1, COL_TWIDDLE>), g, b, 0, s, a);
+    } else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
 template <typename T> hipError_t col_impl(int L, int dir, int mode, const ColArgs &a, hipStream_t s)
 {
     switch (L) {
@@ -141,6 +192,12 @@ template <typename T> hipError_t col_impl(int L, int dir, int mode, const ColArg
                 case 32: if constexpr (col_fits_v<T, LL, 32>()) return col_launch<T, LL, 32>(dir, mode, a, s); break;                                       \
                 default: break;                                                                               \
                 }                                                                                             \
+            }                                                                                                 \
+            if constexpr (LL >= 512) {                                                                        \
+                const int form = col_form<T, LL>(mode, a);                                                    \
+                if constexpr (LL != 512 && !(LL == 4096 && sizeof(T) == 8))                                   \
+                    if (form == 1) return col_h_launch<T, LL, col_lpb<T, LL>()>(dir, mode, a, s);                 \
+                if (form == 2) return col_h_launch<T, LL, 2 * col_lpb<T, LL>()>(dir, mode, a, s);             \
             }                                                                                                 \
             return col_launch<T, LL, col_lpb<T, LL>()>(dir, mode, a, s);                                      \
         }                                                                                                     \

@@ -1074,6 +1074,7 @@ hipError_t C2C::run(const void *in, void *out, long long nlines, long long in_di
             c.tw2 = tw2;
             c.scale = 1.0;
             c.lpb = col_lpb;
+            c.four = 1;
             hipError_t e = launch_col(prec, n1, dir, row_twin ? COL_PLAIN : COL_TWIDDLE, c, s);
             if (e != hipSuccess) return e;
             RowTArgs r{scratch, (char *)out + (size_t)l0 * out_dist * cb, n1, n, out_dist, cnt, tw_b, scale, row_lpb,
@@ -1321,6 +1322,7 @@ hipError_t R2C::fwd(const void *in, void *out, long long nlines, long long in_di
             c.tw2 = inner.tw2;
             c.scale = 1.0;
             c.lpb = inner.col_lpb;
+            c.four = 1;
             e = launch_col(prec, inner.n1, -1, COL_TWIDDLE, c, s);
             if (e != hipSuccess) return e;
             RowR2CArgs r{Z, dst, inner.n1, L, out_dist, cnt, inner.tw_b, rtw, scale, dbl, r2c_lpb};

@@ -1,0 +1,52 @@
+"""Strided axes and FP64 four-step columns through half a tile of LDS
+(k_col_h): each length and width at the smallest number of tiles that takes
+it, with whole and with partial tiles, forward and inverse, against pocketfft,
+and the far strides against torch.fft in FP64.
+
+Tolerance: the suite's, 1e-6 (FP32) / 1e-14 (FP64) log2 of the points."""
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+from gpu_util import pocket, rounded, run_plan, tol_for
+
+pytestmark = pytest.mark.gpu
+
+# prec, op, dims, batch
+CASES = [
+    # the default width, two workgroups a CU
+    ("f32", "dft", [1024, 16], 512), ("f32", "invdft", [1024, 64], 128), ("f32", "realdft", [1024, 32], 256),
+    ("f32", "realdft", [2048, 16], 256), ("f32", "dft", [2048, 8], 513), ("f32", "realdft", [4096, 16], 171),
+    ("f64", "dft", [1024, 16], 256), ("f64", "invdft", [2048, 8], 256), ("f64", "realdft", [2048, 16], 171),
+    # twice the width
+    ("f32", "invdft", [2048, 512], 16), ("f32", "dft", [4096, 512], 4), ("f32", "realdft", [4096, 2], 4096),
+    ("f64", "dft", [2048, 4], 4096), ("f64", "invdft", [4096, 4], 512), ("f64", "realdft", [4096, 4], 512),
+    # FP64 four-steps
+    ("f64", "dft", [1 << 20], 4), ("f64", "invdft", [1 << 20], 5), ("f64", "dft", [1 << 21], 16),
+]
+
+
+@pytest.mark.parametrize("prec,op,dims,batch", CASES)
+def test_half_tile_columns(pkg, dev, prec, op, dims, batch):
+    p = int(np.prod(dims))
+    x = rounded(ol.uniform(71, p * batch * (1 if op == "realdft" else 2)), prec)
+    err = ol.rel_l2(run_plan(pkg, dev, op, dims, x, batch, prec), pocket(op, dims, x, batch))
+    assert err < tol_for(prec, p), err
+
+
+@pytest.mark.parametrize("prec,dims", [("f32", [512, 1 << 18]), ("f32", [1024, 512, 512]), ("f64", [512, 512, 256])])
+def test_half_tile_columns_far_apart(pkg, dev, prec, dims):
+    import torch
+    p = int(np.prod(dims))
+    dt = torch.float32 if prec == "f32" else torch.float64
+    x = torch.empty(2 * p, dtype=dt, device=dev)
+    pkg.fill_uniform(x.data_ptr(), x.numel(), 72, 0, prec)
+    y = torch.empty_like(x)
+    plan = pkg.Plan("dft", prec, dims, 1)
+    plan.execute("dft", x.data_ptr(), y.data_ptr())
+    torch.cuda.synchronize()
+    plan.check()
+    plan.close()
+    want = torch.fft.fftn(torch.view_as_complex(x.double().view(dims + [2])))
+    got = torch.view_as_complex(y.double().view(dims + [2]))
+    assert float((got - want).norm() / want.norm()) < tol_for(prec, p)
