@@ -146,9 +146,11 @@ struct WpowArgs {
     long long dist;            // elements per transform (L * S)
     long long ntrans;          // batch
     const void *tw;            // FP64 stage table of L
+    int form;                  // kernel (col_wpow_tiles)
 };
 bool col_wpow_supported(int prec, int L);
-long long col_wpow_tiles(int prec, int L, int ncols);
+// workgroups per transform, and the kernel a batch of this many takes
+long long col_wpow_tiles(int prec, int L, int ncols, long long batch, int *form);
 hipError_t launch_col_wpow(int prec, int L, const WpowArgs &a, hipStream_t s);
 long long wpow_mask_chunks(long long P);
 hipError_t launch_wpow_mask(int prec, void *buf, const void *w, double *partial, long long P, long long ntrans,

@@ -13,18 +13,38 @@ template <typename T, int L> constexpr bool wpow_fits()
     return col_fits_v<T, L, lpb>() && wpow_threads<L, lpb>() % 64 == 0;
 }
 
-template <typename T> hipError_t col_wpow_impl(int L, const WpowArgs &a, hipStream_t s, long long *per)
+template <typename T, int L, int LPB> void wpow_h_go(unsigned gx, const WpowArgs &a, hipStream_t s)
+{
+    hipLaunchKernelGGL((k_col_wpow_h<T, L, LPB>), dim3(gx, (unsigned)a.ntrans), dim3(Sched<L>::NT / 2 * LPB), 0, s, a);
+}
+
+// launch == false: only the form that the whole batch takes and its workgroups
+// per transform
+template <typename T> hipError_t col_wpow_impl(int L, WpowArgs &a, hipStream_t s, long long *per, bool launch)
 {
     switch (L) {
 #define NFFT_CASE(LL)                                                                                         \
     case LL:                                                                                                  \
         if constexpr (wpow_fits<T, LL>()) {                                                                   \
             constexpr int lpb = col_lpb<T, LL>();                                                             \
-            const unsigned gx = (unsigned)((a.ncols + lpb - 1) / lpb);                                        \
+            if (!launch) {                                                                                    \
+                ColArgs c{};                                                                                  \
+                c.ncols = a.ncols;                                                                            \
+                c.S = a.ncols;                                                                                \
+                c.ntrans = a.ntrans;                                                                          \
+                a.form = LL >= 512 ? col_form<T, LL>(COL_PLAIN, c) : 0;                                       \
+            }                                                                                                 \
+            const int w = a.form == 2 ? 2 * lpb : lpb;                                                        \
+            const unsigned gx = (unsigned)((a.ncols + w - 1) / w);                                            \
             *per = gx;                                                                                        \
-            if (!s && !a.buf) return hipSuccess; /* size query */                                           \
-            hipLaunchKernelGGL((k_col_wpow<T, LL, lpb>), dim3(gx, (unsigned)a.ntrans), dim3((wpow_threads<LL, lpb>())), \
-                               0, s, a);                                                                      \
+            if (!launch) return hipSuccess;                                                                   \
+            if constexpr (LL >= 512) {                                                                        \
+                if (a.form == 1) wpow_h_go<T, LL, lpb>(gx, a, s);                                             \
+                if (a.form == 2) wpow_h_go<T, LL, 2 * lpb>(gx, a, s);                                         \
+            }                                                                                                 \
+            if (a.form == 0)                                                                                  \
+                hipLaunchKernelGGL((k_col_wpow<T, LL, lpb>), dim3(gx, (unsigned)a.ntrans),                    \
+                                   dim3((wpow_threads<LL, lpb>())), 0, s, a);                                 \
             return hipGetLastError();                                                                         \
         }                                                                                                     \
         break;
@@ -38,30 +58,30 @@ template <typename T> hipError_t col_wpow_impl(int L, const WpowArgs &a, hipStre
 
 bool col_wpow_supported(int prec, int L)
 {
-    long long per = 0;
-    WpowArgs a{};
-    a.ncols = 1;
-    return (prec == F32 ? col_wpow_impl<float>(L, a, nullptr, &per) : col_wpow_impl<double>(L, a, nullptr, &per)) ==
-           hipSuccess;
+    int form = 0;
+    return col_wpow_tiles(prec, L, 1, 1, &form) > 0;
 }
 
-long long col_wpow_tiles(int prec, int L, int ncols)
+long long col_wpow_tiles(int prec, int L, int ncols, long long batch, int *form)
 {
     long long per = 0;
     WpowArgs a{};
     a.ncols = ncols;
-    if ((prec == F32 ? col_wpow_impl<float>(L, a, nullptr, &per) : col_wpow_impl<double>(L, a, nullptr, &per)) !=
-        hipSuccess)
+    a.ntrans = batch;
+    if ((prec == F32 ? col_wpow_impl<float>(L, a, nullptr, &per, false)
+                     : col_wpow_impl<double>(L, a, nullptr, &per, false)) != hipSuccess)
         return 0;
+    *form = a.form;
     return per;
 }
 
-hipError_t launch_col_wpow(int prec, int L, const WpowArgs &a, hipStream_t s)
+hipError_t launch_col_wpow(int prec, int L, const WpowArgs &a0, hipStream_t s)
 {
+    WpowArgs a = a0;
     if (a.ntrans < 1 || a.ntrans > 65535 || !a.buf) return hipErrorInvalidValue;
     long long per = 0;
     const int slot = prof_on() ? prof_begin(s) : -1;
-    const hipError_t e = prec == F32 ? col_wpow_impl<float>(L, a, s, &per) : col_wpow_impl<double>(L, a, s, &per);
+    const hipError_t e = prec == F32 ? col_wpow_impl<float>(L, a, s, &per, true) : col_wpow_impl<double>(L, a, s, &per, true);
     if (slot >= 0)
         prof_end(slot, s, "k_col_wpow", prec, L,
                  (double)a.ntrans * a.dist * (prec == F32 ? 16.0 : 32.0) + (double)a.dist * (prec == F32 ? 4 : 8));

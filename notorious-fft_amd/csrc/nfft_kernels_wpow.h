@@ -93,6 +93,89 @@ __global__ void __launch_bounds__((wpow_threads<L, LPB>())) k_col_wpow(WpowArgs 
     if (threadIdx.x == 0) a.partial[tile] = tot;
 }
 
+// The same with the exchanges through half a tile of LDS, two sets of 16 points
+// per thread, where col_form (nfft_launch_impl.h) takes k_col_h: two workgroups
+// a CU, or twice the columns.
+template <typename T, int L, int LPB>
+__global__ void __launch_bounds__((Sched<L>::NT / 2 * LPB), (col_h_wpe<T, L, LPB>())) k_col_wpow_h(WpowArgs a)
+{
+    using S = Sched<L>;
+    using C = Cx<T>;
+    constexpr int NH = S::NT / 2, NTH = NH * LPB;
+    static_assert(NTH % 64 == 0, "whole waves");
+    __shared__ C lds[L / 2 * LPB];
+    __shared__ C ltw[S::TWN];
+    __shared__ double red[NTH / 64];
+    const int b = threadIdx.x % LPB;
+    int j = threadIdx.x / LPB;
+    const long long tile = xcd_columns<T>(blockIdx.x + (long long)gridDim.x * blockIdx.y,
+                                          (long long)gridDim.x * gridDim.y);
+    const long long t = tile / gridDim.x;
+    const int c0 = (int)(tile % gridDim.x) * LPB, c = c0 + b;
+    const bool valid = c < a.ncols;
+    const bool full = c0 + LPB <= a.ncols && off_fits<C>((long long)L * a.ncols);
+    C *col = (C *)a.buf + t * a.dist + c;
+    const T *w = (const T *)a.w + (valid ? c : 0);  // columns past the last one weigh zero
+    const auto rs = buf_rsrc((C *)a.buf + t * a.dist + c0);
+    const auto off = [&] { return (uint32_t)(j * a.ncols + b) * (uint32_t)sizeof(C); };
+    const uint32_t qst = (uint32_t)(S::NT * a.ncols) * (uint32_t)sizeof(C);
+    const uint32_t lst = (uint32_t)(NH * a.ncols) * (uint32_t)sizeof(C);
+    const auto row = [&](int l, int q) { return (long long)(j + l * NH + S::NT * q) * a.ncols; };
+    C reg[2][16];
+    if (full) {
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) reg[l][q] = buf_ld<C>(rs, off(), l * lst + q * qst);
+    } else {
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) reg[l][q] = valid ? col[row(l, q)] : czero<T>();
+    }
+    stage_tw_to_lds<T, L>(ltw, (const double2 *)a.tw);  // visible after the first exchange's barriers
+    line_fft_halves<T, L, -1>(reg, lds, LayCol<LPB>{b}, j, StageTwLds<T>{ltw});
+    double part = 0.0;
+    // The points fill half the registers: eight weights at a time, the sum
+    // formed here (not put off until after the second transform, its points
+    // kept for it), and no address kept through a transform.
+#pragma unroll
+    for (int l = 0; l < 2; l++)
+#pragma unroll
+        for (int h = 0; h < 16; h += 8) {
+            asm volatile("" : "+v"(j));
+            __builtin_amdgcn_sched_barrier(0);
+            T w2[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) w2[q] = w[row(l, h + q)];
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                w2[q] = valid ? w2[q] * w2[q] : (T)0;
+                const C y = reg[l][h + q];
+                part += (double)w2[q] * ((double)y.x * y.x + (double)y.y * y.y);
+                reg[l][h + q] = cscale(y, (T)2 * w2[q]);
+            }
+            asm volatile("" : "+v"(part));
+        }
+    asm volatile("" : "+v"(j));
+    __builtin_amdgcn_sched_barrier(0);
+    line_fft_halves<T, L, 1>(reg, lds, LayCol<LPB>{b}, j, StageTwLds<T>{ltw});
+    asm volatile("" : "+v"(j));
+    if (full) {
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) buf_st<C>(rs, off(), l * lst + q * qst, reg[l][q]);
+    } else if (valid) {
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) col[row(l, q)] = reg[l][q];
+    }
+    const double tot = block_sum<NTH>(part, red);
+    if (threadIdx.x == 0) a.partial[tile] = tot;
+}
+
 // Elementwise weighting of a spectrum (batch x P complex), with loss partials
 // per workgroup: blockIdx.y = transform, blockIdx.x = chunk of P.
 template <typename T>

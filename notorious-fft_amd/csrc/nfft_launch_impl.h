@@ -149,6 +149,10 @@ template <int L> constexpr bool tunable_len() { return L >= 128 && L <= 2048; }
 //   FP64 2048: S = 2048 (2^23 points) 96 / 94 / 107, 1024 860 / 945 / 852, 1025
 //     1068 / 1087 / 1009
 //   FP64 4096: S = 1024 1010 / 1088 / 908, 1025 1227 / 1330 / 1127
+// The weighted power's fused pass (k_col_wpow_h) takes the same: FP32 2048^2 x
+// 16 737 / 744 / 720, x 2 93 / 91 / 89, 1024^2 x 30 316 / 293 / 312, 4096 x 1024
+// x 8 410 / 422 / 374; FP64 2048^2 x 16 1485 / 1461 / 1390, 4096 x 1024 x 8 925
+// / 945 / 847.
 template <typename T, int L> int col_form(int mode, const ColArgs &a)
 {
     constexpr bool f32 = sizeof(T) == 4;

@@ -1885,7 +1885,8 @@ int nfft_plan::weighted_power(const void *x, const void *w, void *grad, double *
     const long long S = P / dims[0];
     const bool fused = d >= 2 && env_int("NFFT_FUSE", 1) != 0 && ax[0].algo == ALG_LINE &&
                        col_wpow_supported(prec, dims[0]) && S <= 0x7fffffffLL;
-    const long long per = fused ? col_wpow_tiles(prec, dims[0], (int)S) : wpow_mask_chunks(P);
+    int form = 0;
+    const long long per = fused ? col_wpow_tiles(prec, dims[0], (int)S, batch, &form) : wpow_mask_chunks(P);
     if (per < 1) {
         set_error("weighted power: no kernel for this shape");
         return NFFT_E_UNSUPPORTED;
@@ -1916,6 +1917,7 @@ int nfft_plan::weighted_power(const void *x, const void *w, void *grad, double *
             a.dist = P;
             a.ntrans = std::min(kGroup, batch - t0);
             a.tw = ax[0].tw_a;
+            a.form = form;
             e = launch_col_wpow(prec, dims[0], a, s);
         }
         // adjoint (unnormalised inverse) along axes d-1..1

@@ -1,5 +1,5 @@
-"""Strided axes and FP64 four-step columns through half a tile of LDS
-(k_col_h): each length and width at the smallest number of tiles that takes
+"""Strided axes, FP64 four-step columns and the weighted power through half a
+tile of LDS (k_col_h, k_col_wpow_h): each length and width at the smallest number of tiles that takes
 it, with whole and with partial tiles, forward and inverse, against pocketfft,
 and the far strides against torch.fft in FP64.
 
@@ -9,6 +9,7 @@ import pytest
 
 import oracle_lib as ol
 from gpu_util import pocket, rounded, run_plan, tol_for
+from test_gpu_c5 import gauss_mask, np_ref, run_wpow
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +51,15 @@ def test_half_tile_columns_far_apart(pkg, dev, prec, dims):
     want = torch.fft.fftn(torch.view_as_complex(x.double().view(dims + [2])))
     got = torch.view_as_complex(y.double().view(dims + [2]))
     assert float((got - want).norm() / want.norm()) < tol_for(prec, p)
+
+
+@pytest.mark.parametrize("prec,dims,batch", [("f32", [1024, 18], 256), ("f32", [4096, 6], 256), ("f64", [2048, 9], 171),
+                                             ("f32", [2048, 512], 16), ("f64", [2048, 4], 4096), ("f64", [4096, 5], 342)])
+def test_half_tile_weighted_power(pkg, dev, prec, dims, batch, monkeypatch):
+    p = int(np.prod(dims))
+    x = rounded(ol.uniform(73, 2 * p * batch), prec)
+    w = rounded(gauss_mask(dims), prec)
+    lref, gref = np_ref(x, w, dims, batch)
+    loss, grad = run_wpow(pkg, dev, prec, dims, batch, x, w, monkeypatch)
+    assert np.max(np.abs(loss - lref) / lref) < tol_for(prec, p)
+    assert ol.rel_l2(grad, gref) < tol_for(prec, p)
