@@ -182,6 +182,17 @@ template <typename T, int L, int LPB> hipError_t col_h_launch(int dir, int mode,
     return hipGetLastError();
 }
 
+// Columns per workgroup where the default tiles would leave CUs without one:
+// four, and up to four times the workgroups.  us, default / four: FP32 1024^2
+// (64 tiles) 18.3 / 16.0, x 2 27.1 / 23.9, x 3 25.9 / 26.3, 1024^2 realdft and back
+// 34.9 / 29.4, 2^20 (a four-step's 64 tiles) 25.0 / 22.7, x 2 31.8 / 32.1, 2^19 x 3
+// 24.0 / 26.1; FP64 512^2 13.2 / 12.2, 1024^2 21.5 / 20.5.
+template <typename T, int L> int col_narrow(const ColArgs &a)
+{
+    const long long w = col_lpb<T, L>(), tiles = (a.ncols + w - 1) / w * a.ntrans;
+    return L >= 256 && L <= 2048 && tiles <= (a.four ? 64 : 128) ? 4 : 0;
+}
+
 template <typename T> hipError_t col_impl(int L, int dir, int mode, const ColArgs &a, hipStream_t s)
 {
     switch (L) {
@@ -189,7 +200,7 @@ template <typename T> hipError_t col_impl(int L, int dir, int mode, const ColArg
     case LL:                                                                                                  \
         if constexpr (col_fits<T, LL>()) {                                                                    \
             if constexpr (tunable_len<LL>()) {                                                                \
-                switch (a.lpb) {                                                                              \
+                switch (a.lpb ? a.lpb : col_narrow<T, LL>(a)) {                                                \
                 case 4: if constexpr (col_fits_v<T, LL, 4>()) return col_launch<T, LL, 4>(dir, mode, a, s); break;                                         \
                 case 8: if constexpr (col_fits_v<T, LL, 8>()) return col_launch<T, LL, 8>(dir, mode, a, s); break;                                         \
                 case 16: if constexpr (col_fits_v<T, LL, 16>()) return col_launch<T, LL, 16>(dir, mode, a, s); break;                                       \

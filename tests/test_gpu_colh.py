@@ -1,7 +1,8 @@
-"""Strided axes, FP64 four-step columns and the weighted power through half a
+"""Column tiles by rule.  Strided axes, FP64 four-step columns and the weighted power through half a
 tile of LDS (k_col_h, k_col_wpow_h): each length and width at the smallest number of tiles that takes
 it, with whole and with partial tiles, forward and inverse, against pocketfft,
-and the far strides against torch.fft in FP64.
+and the far strides against torch.fft in FP64.  Narrow tiles: partial ones, the
+most tiles that take them and one more, and a four-step's.
 
 Tolerance: the suite's, 1e-6 (FP32) / 1e-14 (FP64) log2 of the points."""
 import numpy as np
@@ -63,3 +64,17 @@ def test_half_tile_weighted_power(pkg, dev, prec, dims, batch, monkeypatch):
     loss, grad = run_wpow(pkg, dev, prec, dims, batch, x, w, monkeypatch)
     assert np.max(np.abs(loss - lref) / lref) < tol_for(prec, p)
     assert ol.rel_l2(grad, gref) < tol_for(prec, p)
+
+
+@pytest.mark.parametrize("prec,op,dims,batch", [
+    ("f32", "dft", [256, 2], 1), ("f64", "realdft", [512, 16], 1), ("f32", "invdft", [1024, 2048], 1),
+    ("f32", "dft", [1024, 2064], 1), ("f64", "dft", [2048, 512], 1), ("f32", "realdft", [2048, 64], 2),
+    ("f32", "dft", [1 << 20], 1), ("f64", "invdft", [1 << 18], 1), ("f32", "dct2", [512, 8], 1),
+    ("f32", "dct3", [1024, 32, 2], 1), ("f64", "dst2", [512, 2048], 1), ("f64", "dct4", [1024, 16], 1),
+    ("f32", "dst3", [512, 32], 128), ("f32", "dct2", [512, 32], 129)])
+def test_narrow_columns(pkg, dev, prec, op, dims, batch):
+    p = int(np.prod(dims))
+    x = rounded(ol.uniform(74, p * batch * (2 if op in ("dft", "invdft") else 1)), prec)
+    want = ol.run_oracle(op, dims, x, batch) if op[:2] in ("dc", "ds") else pocket(op, dims, x, batch)
+    err = ol.rel_l2(run_plan(pkg, dev, op, dims, x, batch, prec), want)
+    assert err < tol_for(prec, p), err
