@@ -130,25 +130,29 @@ template <int L> constexpr bool tunable_len() { return L >= 128 && L <= 2048; }
 // How a plain (or FP64 twiddle) pass of L-point columns runs, of the default
 // width w = col_lpb: 0 k_col; 1 k_col_h, w columns in half the LDS, two
 // workgroups a CU that load, transform and store past each other; 2 k_col_h,
-// 2 w columns, twice the run per row.  Two workgroups a CU need 512 tiles (2048^2
-// FP32, 256 tiles: 28.2 / 29.7 / 33.2 us for 0 / 1 / 2).  The wide tile
-// wins where 1 keeps losing whole lines between the workgroups of a row:
-// rows of whole 128-byte lines, or 2 MiB and more apart (a tile then touches
-// as many pages as it has rows).  us for 0 / 1 / 2, 2^27 FP32 or 2^26 FP64
-// points unless stated, other axes included:
+// 2 w columns, twice the run per row.  Two workgroups a CU need more tiles than
+// CUs (2048^2 FP32, 256 tiles: 32.7 / 34.5 / 38.1 us for 0 / 1 / 2).  The wide
+// tile wins where 1 keeps losing whole lines between the workgroups of a row,
+// in large arrays and with rows of whole 128-byte lines, or 2 MiB and more
+// apart (a tile touches as many pages as it has rows).  us for 0 / 1 / 2, other
+// axes included, 2^27 FP32 or 2^26 FP64 points unless another number of
+// tiles is stated; S: columns:
 //   FP32 512: S = 1024 763 / 777 / 774, S = 2^18 1241 / 1258 / 1183
 //   FP32 1024: S = 64 927 / 917 / 947, 1024 815 / 785 / 825, 2049 996 / 935 /
-//     972, 2^18 (2^28 points) 2790 / 2545 / 2485
-//   FP32 2048: S = 64 964 / 921 / 958, 8192 983 / 1021 / 969, 1025 (2^23
-//     points) 135 / 124 / 145, 8193 1126 / 1062 / 1095
-//   FP32 4096: S = 64 1129 / 1016 / 1049, 1024 964 / 939 / 874, 1025 (2^23
-//     points) 150 / 139 / 147, (2^26) 1172 / 1102 / 1068
+//     972, 513 (297 tiles) 87 / 81 / 82, 2^18 (2^28 points) 2790 / 2545 / 2485
+//   FP32 2048: S = 64 964 / 921 / 958, 8192 983 / 1021 / 969, 2048 (768 tiles)
+//     77 / 72 / 83, 1025 (387 tiles) 105 / 93 / 97, 8193 1126 / 1062 / 1095
+//   FP32 4096: S = 64 1129 / 1016 / 1049, 1024 964 / 939 / 874, 4096 (1024
+//     tiles) 137 / 140 / 117, 2049 (513 tiles) 153 / 146 / 151, (1026) 286 /
+//     278 / 272
 //   FP64 512: S = 1024 822 / 821 / 820, 2^17 1387 / 1307 / 1245
-//   FP64 1024: S = 1024 819 / 820 / 841 (2^23 points 95 / 87 / 94), 1025 969
-//     / 984 / 956
-//   FP64 2048: S = 2048 (2^23 points) 96 / 94 / 107, 1024 860 / 945 / 852, 1025
-//     1068 / 1087 / 1009
-//   FP64 4096: S = 1024 1010 / 1088 / 908, 1025 1227 / 1330 / 1127
+//   FP64 1024: S = 1024 819 / 820 / 841, (1024 tiles) 112 / 107 / 109, 1025 969 /
+//     984 / 956, 513 (585 tiles) 147 / 140 / 154
+//   FP64 2048: S = 2048 (1536 tiles) 176 / 174 / 165, 1024 860 / 945 / 852, 1025
+//     (771 tiles) 207 / 186 / 192, (4112) 1068 / 1087 / 1009; four-step 2^21 x 3
+//     98 / 100, x 20 598 / - / 558
+//   FP64 4096: S = 1024 1010 / 1088 / 908, 64 (960 tiles) 151 / 152 / 143, 1025
+//     1227 / 1330 / 1127
 // The weighted power's fused pass (k_col_wpow_h) takes the same: FP32 2048^2 x
 // 16 737 / 744 / 720, x 2 93 / 91 / 89, 1024^2 x 30 316 / 293 / 312, 4096 x 1024
 // x 8 410 / 422 / 374; FP64 2048^2 x 16 1485 / 1461 / 1390, 4096 x 1024 x 8 925
@@ -160,11 +164,13 @@ template <typename T, int L> int col_form(int mode, const ColArgs &a)
     if (a.lpb || mode > (f32 ? COL_PLAIN : COL_TWIDDLE) || (f32 && a.four)) return 0;
     const long long w = col_lpb<T, L>(), tiles = (a.ncols + w - 1) / w * a.ntrans, row = a.S * (long long)sizeof(Cx<T>);
     const bool lines = row % 128 == 0, far = row >= (2LL << 20);
-    if (tiles < 512) return 0;
+    if (tiles <= 256) return 0;
     if (L == 512) return far ? 2 : 0;
-    if (L == 1024) return f32 ? (far ? 2 : 1) : (lines ? 1 : 0);
-    if (L == 2048) return f32 ? (lines && a.S >= 512 && tiles >= 1024 ? 2 : 1) : (tiles >= 4096 ? 2 : a.four ? 0 : 1);
-    if (L == 4096) return f32 ? ((lines ? a.S >= 512 : tiles >= 4096) ? 2 : 1) : (tiles >= 1024 ? 2 : 0);
+    if (L == 1024) return f32 ? (far ? 2 : 1) : (lines || tiles < 4096 ? 1 : 0);
+    if (L == 2048)
+        return f32 ? (lines && a.S >= 512 && tiles >= 1024 ? 2 : 1)
+                   : (tiles >= (lines ? 1024 : 4096) ? 2 : a.four ? 0 : 1);
+    if (L == 4096) return f32 ? ((lines ? a.S >= 512 : tiles >= 1024) ? 2 : 1) : (tiles > 512 ? 2 : 0);
     return 0;
 }
 
