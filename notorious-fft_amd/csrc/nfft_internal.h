@@ -185,6 +185,9 @@ struct MixShape {
     int nth_min = 64, nth_max = 1024;
     MixLanes lanes = MIX_LANES_POINTS;
     size_t lds_max = kMixLds;
+    // a few workgroups: the schedule that ends first, of more and smaller
+    // radices, rather than the one with the fewest instructions
+    bool few = false;
 };
 int mix_max(int prec);
 // The cheapest schedule of length n within a shape (blue: a Bluestein line's,
@@ -194,7 +197,8 @@ bool mix_fit(int prec, long long n, bool blue, const MixShape &sh, MixPlan *p, d
 // The same over the 7-smooth M >= 2n - 1 that is cheapest; sh.g_max in points.
 bool mix_blue_fit(int prec, long long n, MixShape sh, MixPlan *p);
 // one-pass lines of a batch: 7-smooth n >= 2, and Bluestein of any n
-bool mix_plan(int prec, long long n, MixPlan *p);
+// lines: in a batch, 0 many
+bool mix_plan(int prec, long long n, long long lines, MixPlan *p);
 bool mix_blue_plan(int prec, long long n, MixPlan *p);
 bool smooth7(long long n);  // no prime factor above 7
 hipError_t launch_mix(int prec, const MixArgs &a, hipStream_t s);
@@ -209,6 +213,7 @@ struct TileFit {
 struct TileFits {
     int prec, points, nth_max;
     std::map<std::tuple<int, int, int>, TileFit> seen;
+    bool few = false;  // as MixShape's
     int seg() const { return prec == F32 ? 16 : 8; }  // points of a 128-byte segment
     const TileFit &get(int L, MixLanes lanes, bool blue);
 };
@@ -334,7 +339,9 @@ struct C2C {
     // rule), 1 = mixed radix, 0 = Bluestein
     // persist_mode = 0 keeps the two-launch four-step for powers of two
     // (callers that fuse their own work into its row pass)
-    bool init(int n, int prec, int smooth_mode = 2, int persist_mode = 2);
+    // lines: transforms in a batch (0: many); small batches of lengths other
+    // than powers of two take more, shorter workgroups
+    bool init(int n, int prec, int smooth_mode = 2, int persist_mode = 2, long long lines = 0);
     void release();
     std::string describe() const;
     // dir: -1 forward, +1 inverse (unnormalised); scale applied to the output.

@@ -125,6 +125,21 @@ double cost_of(const MixPlan &p, int prec, double conflict)
     return c / p.G * (1.0 + 6.0 / (wg * wv));
 }
 
+// Time of one workgroup that has its CU to itself, in issue slots: the rounds
+// of its busiest SIMD, and per stage a trip through LDS, a table load and a
+// barrier.
+double latency_of(const MixPlan &p, int prec)
+{
+    double c = 0;
+    for (int s = 0; s < p.steps; s++) {
+        const int total = p.G * p.st[s].nb, R = p.st[s].radix, reps = (total + p.nth - 1) / p.nth;
+        const int waves = (std::min(p.nth, total) + 63) / 64;
+        const bool mid = p.blue && s == p.stages - 1;
+        c += reps * ((waves + 3) / 4) * (R * (dft_ops(R) * (mid ? 2 : 1) + 16) * (prec == 0 ? 1.0 : 1.5) + 50) + 350;
+    }
+    return c;
+}
+
 struct Search {
     int prec, L;
     bool blue;
@@ -159,7 +174,7 @@ struct Search {
                 if (!ok) continue;
                 if (nth > shape.nth_min && nth - 64 >= most) break;  // only idle waves beyond
                 p.nth = nth;
-                const double c = cost_of(p, prec, conflict);
+                const double c = shape.few ? latency_of(p, prec) : cost_of(p, prec, conflict);
                 if (c < best) {
                     best = c;
                     plan = p;
@@ -187,13 +202,13 @@ struct Found {
     double cost;
     MixPlan plan;
 };
-typedef std::tuple<int, int, int, int, int, int, int, int, size_t> Key;
+typedef std::tuple<int, int, int, int, int, int, int, int, size_t, bool> Key;
 std::mutex g_mix_mu;
 std::map<Key, Found> g_mix_plans;  // schedules are searched once per process
 
 const Found &find(int prec, int L, bool blue, const MixShape &sh)
 {
-    const Key key(L, prec, blue ? 1 : 0, sh.g_min, sh.g_max, sh.nth_min, sh.nth_max, (int)sh.lanes, sh.lds_max);
+    const Key key(L, prec, blue ? 1 : 0, sh.g_min, sh.g_max, sh.nth_min, sh.nth_max, (int)sh.lanes, sh.lds_max, sh.few);
     std::lock_guard<std::mutex> lk(g_mix_mu);
     auto it = g_mix_plans.find(key);
     if (it == g_mix_plans.end()) {
@@ -202,8 +217,8 @@ const Found &find(int prec, int L, bool blue, const MixShape &sh)
         se.L = L;
         se.blue = blue;
         se.shape = sh;
-        // the fewest stages possible and one more
-        for (int stages = 1, found = 0; stages <= kMixMaxStages && found < 2; stages++) {
+        // the fewest stages possible and one more (few workgroups: two more)
+        for (int stages = 1, found = 0; stages <= kMixMaxStages && found < (sh.few ? 3 : 2); stages++) {
             se.split(L, 0, 32, stages);
             if (se.best < 1e299) found++;
         }
@@ -241,16 +256,25 @@ bool mix_fit(int prec, long long n, bool blue, const MixShape &sh, MixPlan *p, d
     return true;
 }
 
-bool mix_plan(int prec, long long n, MixPlan *p)
+bool mix_plan(int prec, long long n, long long lines, MixPlan *p)
 {
-    if (n < 2 || !mix_fit(prec, n, false, line_shape((int)n), p)) return false;
+    MixShape sh = line_shape((int)n);
+    // Small batches end with their longest workgroup: few lines in each, radices
+    // around 10 (us, large batches' schedule / this / two LDS buffers: FP32 N = 1200
+    // x 40 9.6 / 6.2 / 8.7, 10^4 x 20 13 / 11 / 16; FP64 720 x 40 10.2 / 6.2 / 6.5,
+    // 2000 x 60 11.2 / 7.1 / 12.5).
+    if (lines > 0 && lines * n <= (n > 512 ? 1 << 19 : 1 << 20)) {  // (FP64 1000 x 1000 11.2 / 14.3)
+        sh.g_min = sh.g_max = (int)std::min<long long>(sh.g_max, (lines + 1023) / 1024);
+        sh.few = true;
+    }
+    if (n < 2 || !mix_fit(prec, n, false, sh, p)) return false;
     // FP32 twiddle tables where that keeps the error at what a table entry per
     // twiddle gives (radices up to 10 over several stages before; Bluestein
     // between: N = 1000 2.1e-7 -> 1.2e-7).  Short lines lose 2-3 % of it (N =
     // 480 1.055e-7 -> 1.084e-7), lines beyond 10240 points, with two of their
     // three stages near radix 32, up to 8 % (N = 20000 1.416e-7 -> 1.537e-7);
     // they take the FP64 table (2^26 points: N = 20000 368 -> 410 us).
-    p->tw64 = prec == F64 || n <= 512 || n > 10240;
+    p->tw64 = prec == F64 || n <= 512 || n > 10240 || sh.few;
     return true;
 }
 
@@ -331,11 +355,12 @@ const TileFit &TileFits::get(int L, MixLanes lanes, bool blue)
         sh.nth_max = nth_max;
         sh.lanes = lanes;
         sh.lds_max = lds_max;
+        sh.few = few;
         TileFit f;
         f.ok = mix_fit(prec, L, blue, sh, &f.plan, &f.cost);
         // a point read and written takes half an issue slot of its CU's share
         // of the memory bandwidth, more where a tile covers part of a segment
-        if (f.ok)
+        if (f.ok && !few)
             f.cost += 0.5 * (prec == F32 ? 1 : 2) * L *
                       (lanes == MIX_LANES_POINTS ? 1.0 : std::max(1.0, (double)seg() / f.plan.G));
         if (f.ok && (!best.ok || f.cost < best.cost)) best = f;
@@ -355,7 +380,8 @@ const TileFit &TileFits::get(int L, MixLanes lanes, bool blue)
 TileStatus tile_plan(TileFits &fits, long long n, bool blue, TilePlan *p)
 {
     // cost of all lines of a phase
-    auto phase = [](const TileFit &f, int lines) {
+    auto phase = [&](const TileFit &f, int lines) {
+        if (fits.few) return f.ok ? f.cost : 1e300;  // all tiles at a time
         return f.ok ? f.cost * f.plan.G * ((lines + f.plan.G - 1) / f.plan.G) : 1e300;
     };
     const long long lo = 2 * n - 1;

@@ -613,10 +613,11 @@ static bool team_setup(C2C &c)
     return true;
 }
 
-bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
+bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode, long long lines)
 {
     n = n_;
     prec = prec_;
+    if (env_int("NFFT_FEW", 1) == 0) lines = 0;  // plan every batch as a large one
     if (n < 1) {
         set_error("transform length must be >= 1");
         return false;
@@ -732,8 +733,16 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
         // One pass, a line or a group of lines per workgroup, up to mix_max
         // (NFFT_SMOOTH=2: tiles before lines from 2048 / 1024 points on), else
         // two phases of tiles; lengths with no split for them use Bluestein.
-        const bool line = mix_plan(prec, n, &mx);
-        const bool tiles_first = !line || (smooth_env == 2 && n > (prec == F32 ? 2048 : 1024));
+        const bool line = mix_plan(prec, n, lines, &mx);
+        // small batches: four times the tiles, also where a line would fill its
+        // workgroup (us, FP32 N = 15000 x 17 11.8 against 14.1, 50000 x 5 14.7 / 17.4,
+        // 30000 x 30 26.5 / 18.7; FP64 15000 x 40 28.9 / 21.4)
+        const bool few = lines > 0 && lines * n <= 5 << 16;
+        if (few) {
+            fits.points /= 4;
+            fits.few = true;
+        }
+        const bool tiles_first = !line || (few && n > 12000) || (smooth_env == 2 && n > (prec == F32 ? 2048 : 1024));
         int use = smooth_mode == 1 ? 1 : tuned_choice(prec, n);
         if (use < 0 && env_int("NFFT_TUNE", 0)) use = tune_smooth(n, prec);
         if (use != 0 && tiles_first) {
@@ -766,7 +775,11 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
     // = 10007 2.27 -> 1.06 ms, FP64 N = 4097 4.12 -> 2.10 ms).  Where both
     // fit, the power-of-two line is the faster (FP32 N = 1009 0.47 vs 0.76
     // ms, FP64 0.86 vs 1.65).
-    const bool mixblue = m > line_max(prec) && mix_blue_plan(prec, n, &mx);
+    // Small batches leave CUs idle that the power of two's three passes use (us,
+    // power of two / one pass: FP32 N = 10007 x 1 20 / 33, x 40 31 / 34, x 100 42 / 35;
+    // FP64 4099 x 1 16 / 27, x 60 27 / 28, x 100 35 / 29).
+    const bool mixblue =
+        m > line_max(prec) && (lines == 0 || lines * m > (prec == F32 ? 11 << 17 : 15 << 16)) && mix_blue_plan(prec, n, &mx);
     // Longer ones in three phases of tiles over a 7-smooth M, where that is
     // enough shorter than the power of two, whose passes move a byte faster
     // (2^26 points, power of two / tiles in us, after the ratio of the two M:
@@ -776,7 +789,9 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode)
     // 3732 / 3505, 35023 1.83 4296 / 3624, 90001 1.42 3594 / 3956; beyond
     // 2^17 points the power of two: FP32 500009 1518 / 2107).
     bool tileblue = false;
-    if (!mixblue && m > line_max(prec) && n < (1 << 17)) {
+    // (small batches as above: FP32 20011 x 1 15 / 27 us, x 80 48 / 51, 40009 x 40 55 /
+    // 48; FP64 20011 x 20 34 / 47, x 80 82 / 99, 40009 x 40 87 / 100)
+    if (!mixblue && m > line_max(prec) && n < (1 << 17) && (lines == 0 || lines * m > (prec == F32 ? 8LL << 20 : 32LL << 20))) {
         TileFits small{prec, 16 * kTileThreads, kTileThreads, {}};
         tiles = std::make_shared<TilePlan>();
         const TileStatus st = tile_plan(small, n, true, tiles.get());
@@ -1592,7 +1607,7 @@ bool nfft_plan::init(int kind_, int prec_, int d_, const int *dims_, long long b
     if (kind == NFFT_KIND_DFT) {
         ax.resize(d);
         for (int i = 0; i < d; i++) {
-            if (!ax[i].init(dims[i], prec)) return false;
+            if (!ax[i].init(dims[i], prec, 2, 2, batch * (P / dims[i]))) return false;
             dsc += (i ? " | " : "") + ax[i].describe();
         }
         const long long lines = batch * P / last;

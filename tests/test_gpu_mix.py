@@ -24,6 +24,29 @@ LINES32 = LINES + [10290, 15625, 16807, 19683, 20000, 20412, 20480]
 LINES64 = LINES + [10240]
 
 
+@pytest.fixture(autouse=True)
+def _large(monkeypatch, request):
+    """These lengths as large batches run them, whatever the batch here."""
+    if "small" not in request.node.name:
+        monkeypatch.setenv("NFFT_FEW", "0")
+
+
+# lines and batches of one and of several to a workgroup; tiles instead of a
+# full line; Bluestein on either side of the batch where it changes
+@pytest.mark.parametrize("prec,n,batch", [
+    ("f32", 3, 1), ("f32", 30, 30000), ("f64", 30, 2049), ("f64", 210, 7), ("f32", 480, 257), ("f64", 720, 40),
+    ("f64", 1000, 300), ("f32", 1200, 436), ("f32", 1200, 437), ("f32", 10206, 3), ("f64", 10240, 2),
+    ("f32", 12005, 1), ("f32", 20480, 2), ("f64", 15000, 18), ("f64", 50000, 1), ("f32", 30000, 10), ("f32", 30000, 11),
+    ("f32", 10007, 44), ("f32", 10007, 45), ("f64", 4099, 60), ("f64", 4099, 61), ("f32", 40009, 64), ("f32", 40009, 65)])
+def test_small_batches(pkg, dev, prec, n, batch):
+    blue = any(n % p == 0 for p in (4099, 10007, 40009))
+    tol = (2 if blue else 1) * 4 * EPS[prec] * math.sqrt(math.log2(n))
+    x = rounded(ol.uniform(45, 2 * n * batch), prec)
+    for op, inplace in (("dft", False), ("invdft", True)):
+        err = ol.rel_l2(run_plan(pkg, dev, op, [n], x, batch, prec, inplace=inplace), pocket(op, [n], x, batch))
+        assert err < tol, (op, err)
+
+
 @pytest.mark.parametrize("prec,n", [("f32", n) for n in LINES32] + [("f64", n) for n in LINES64])
 def test_lines(pkg, dev, prec, n):
     plan = pkg.Plan("dft", prec, [n], 1)
