@@ -734,12 +734,13 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode, long long l
         // (NFFT_SMOOTH=2: tiles before lines from 2048 / 1024 points on), else
         // two phases of tiles; lengths with no split for them use Bluestein.
         const bool line = mix_plan(prec, n, lines, &mx);
-        // small batches: four times the tiles, also where a line would fill its
-        // workgroup (us, FP32 N = 15000 x 17 11.8 against 14.1, 50000 x 5 14.7 / 17.4,
+        // small batches: two or four times the tiles (us, two / four: FP64 N = 20000 x 5
+        // 15.0 / 14.1, 30000 x 8 15.6 / 17.0, FP32 50000 x 5 13.5 / 14.8), also where a line
+        // would fill its workgroup ( FP32 N = 15000 x 17 11.8 against 14.1, 50000 x 5 14.7 / 17.4,
         // 30000 x 30 26.5 / 18.7; FP64 15000 x 40 28.9 / 21.4)
         const bool few = lines > 0 && lines * n <= 5 << 16;
         if (few) {
-            fits.points /= 4;
+            fits.points /= n > 24000 ? 2 : 4;
             fits.few = true;
         }
         const bool tiles_first = !line || (few && n > 12000) || (smooth_env == 2 && n > (prec == F32 ? 2048 : 1024));
