@@ -268,13 +268,13 @@ bool mix_plan(int prec, long long n, long long lines, MixPlan *p)
         sh.few = true;
     }
     if (n < 2 || !mix_fit(prec, n, false, sh, p)) return false;
-    // FP32 twiddle tables where that keeps the error at what a table entry per
-    // twiddle gives (radices up to 10 over several stages before; Bluestein
-    // between: N = 1000 2.1e-7 -> 1.2e-7).  Short lines lose 2-3 % of it (N =
-    // 480 1.055e-7 -> 1.084e-7), lines beyond 10240 points, with two of their
-    // three stages near radix 32, up to 8 % (N = 20000 1.416e-7 -> 1.537e-7);
-    // they take the FP64 table (2^26 points: N = 20000 368 -> 410 us).
-    p->tw64 = prec == F64 || n <= 512 || n > 10240 || sh.few;
+    // FP32 twiddle tables where Bluestein's error was the larger before (from
+    // 513 to 10000 points; N = 1000 2.1e-7 -> 1.2e-7).  Shorter lines and those
+    // beyond 10000 points would lose up to 3 % to products of two rounded
+    // entries (N = 480 1.055e-7 -> 1.084e-7, 10125 1.413e-7 -> 1.459e-7, 10240
+    // 1.259e-7 -> 1.293e-7; 10000 gains, 1.466e-7 -> 1.446e-7) and have the FP64
+    // table (2^26 points: N = 10080 304 -> 323 us).
+    p->tw64 = prec == F64 || n <= 512 || n > 10000 || sh.few;
     return true;
 }
 

@@ -18,7 +18,7 @@
 //     whole blocks apart: the padding costs one term per butterfly, none per
 //     point, and takes the strided writes of the first stages off one bank;
 //   - the twiddles w^t of a butterfly come from about 2 sqrt(R) table
-//     entries and one product each.
+//     entries (two where an FP32 transform has FP64 entries) and products.
 // The inverse transform conjugates on the way in and out.
 //
 // Bounds and measurements stand at k_mix_line.
@@ -67,11 +67,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t mix_rsrc(const void *base, uin
 
 // w^t, t < R, applied to v: entry e of the table is e^{-2 pi i e / L}, w the
 // entry `e`.  Powers t = Q h + l as products of the entries of l and Q h.
-// W: type of the table entries.  FP64 tables in FP32 transforms make each
-// power as exact as an entry of its own (mix_plan says which lines have them).
+// W: type of the table entries.  FP32 transforms with FP64 entries (mix_plan
+// says which lines have them, tiles always do) read those of w and w^Q alone,
+// form the powers and apply them in FP64 and round once: with the powers
+// rounded and applied in FP32 lengths were up to 5 % further off than with a
+// table entry and four passes (N = 20000 1.42e-7 -> 1.49e-7; now 1.43e-7; N =
+// 288 1.039e-7 -> 1.075e-7; now 1.030e-7), and the loads cost as much as the
+// FP64 products (2^26 points: N = 20000 394 -> 359 us, 12000 375 -> 344, 288
+// 202 -> 211, 480 202 -> 216, tiles of 10^6 636 -> 664).
 template <typename W, int R, typename C>
 __device__ __forceinline__ void mix_twiddle(C (&v)[R], __amdgpu_buffer_rsrc_t tw, int e)
 {
+    constexpr bool wide = sizeof(W) > sizeof(C);
     constexpr int Q = R <= 5 ? R : R <= 9 ? 3 : R <= 16 ? 4 : R <= 25 ? 5 : 6;
     constexpr int NH = (R - 1) / Q;
     const uint32_t eb = (uint32_t)e * (uint32_t)sizeof(W);
@@ -81,14 +88,19 @@ __device__ __forceinline__ void mix_twiddle(C (&v)[R], __amdgpu_buffer_rsrc_t tw
     };
     W lo[Q], hi[NH + 1];
 #pragma unroll
-    for (int l = 1; l < Q; l++) lo[l] = buf_ld<W>(tw, eb * (uint32_t)l, 0);
+    for (int l = 1; l < Q; l++) lo[l] = wide && l > 1 ? product(lo[l / 2], lo[l - l / 2]) : buf_ld<W>(tw, eb * (uint32_t)l, 0);
 #pragma unroll
-    for (int h = 1; h <= NH; h++) hi[h] = buf_ld<W>(tw, eb * (uint32_t)(Q * h), 0);
+    for (int h = 1; h <= NH; h++) hi[h] = wide && h > 1 ? product(hi[h / 2], hi[h - h / 2]) : buf_ld<W>(tw, eb * (uint32_t)(Q * h), 0);
 #pragma unroll
     for (int t = 1; t < R; t++) {
         const int h = t / Q, l = t % Q;
         const W w = h == 0 ? lo[l] : l == 0 ? hi[h] : product(hi[h], lo[l]);
-        v[t] = cmul(v[t], cmk<C>((decltype(C::x))w.x, (decltype(C::x))w.y));
+        if constexpr (wide) {
+            const double2 z = dmul(make_double2(v[t].x, v[t].y), w);
+            v[t] = cmk<C>((float)z.x, (float)z.y);
+        } else {
+            v[t] = cmul(v[t], w);
+        }
     }
 }
 
