@@ -326,7 +326,7 @@ template <typename T, bool BLUE, class TW> __global__ void __launch_bounds__(mix
 enum { MIX_CHIRP_IN = 1, MIX_CHIRP_OUT = 2, MIX_TW = 4, MIX_HEAD = 8, MIX_TAIL = 16 };
 struct MixPhase {
     MixPlan pl;
-    const void *tw;            // L entries e^{-2 pi i q / L}: FP64 (tiles) or the transform's type (groups)
+    const void *tw;            // L entries e^{-2 pi i q / L}: FP64, groups of Bluestein lines of the transform's type
     Tw2 tw2;                   // MIX_TW: two-level table of the whole length
     const void *chirp, *H;     // chirp entries below nv; filter in the layout of the rows
     int ig, ip, og, op;        // element distances of lines and points, input and output
@@ -512,7 +512,11 @@ template <typename T> __device__ __forceinline__ T rag_scale(const RagArgs &a, R
     return a.inverse && !it.pow2 ? (T)1 / (T)it.n : (T)1;
 }
 
-// Groups of short transforms.
+// Groups of short transforms.  Lines have FP64 twiddle entries at every length
+// (FP32 ones: 2 % further off on average than an entry per twiddle, N = 3136
+// 1.20e-7 -> 1.29e-7, 14000 1.34e-7 -> 1.42e-7; now 4 % nearer, 1.19e-7 and
+// 1.33e-7, for 1 to 3 % of the batch's time).  Bluestein lines, whose error is
+// the convolution's, have entries of their type.
 template <typename T, bool BLUE> __global__ void __launch_bounds__(mix_threads<T>()) k_rag_group(RagArgs a)
 {
     using C = Cx<T>;
@@ -529,7 +533,8 @@ template <typename T, bool BLUE> __global__ void __launch_bounds__(mix_threads<T
     }
     const uint32_t len = (uint32_t)it.n * (uint32_t)sizeof(C);
     const uint32_t end = (uint32_t)(offs[it.cnt - 1] - base) * (uint32_t)sizeof(C) + len;
-    const MixIoLine<T, BLUE, MixOffs<C>> io{mix_rsrc(in, end), mix_rsrc(out, end), mix_rsrc(ph.chirp, len),
+    using W = typename std::conditional<BLUE, C, double2>::type;
+    const MixIoLine<T, BLUE, MixOffs<C>, W> io{mix_rsrc(in, end), mix_rsrc(out, end), mix_rsrc(ph.chirp, len),
                                             buf_rsrc(ph.H),    MixOffs<C>{offs, base}, it.cnt - 1,
                                             it.n,              a.inverse ? (T)-1 : (T)1, rag_scale<T>(a, it)};
     mix_lines<T, BLUE>(ph.pl, (C *)smem, ph.tw, io);

@@ -372,7 +372,7 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
                 z.h = h_elems;
                 h_elems += z.m;
             }
-            ph.tw = phase_table(prec, ph.pl.L, 1, 0, ph.pl.L);
+            ph.tw = phase_table(blue ? prec : F64, ph.pl.L, 1, 0, ph.pl.L);
             if (!ph.tw) return fail("ragged setup: twiddle table");
             size_t &lds = r->group_lds[z.cls][blue ? 1 : 0];
             lds = std::max(lds, (size_t)ph.pl.lp * ph.pl.G * cb);

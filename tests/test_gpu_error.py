@@ -4,6 +4,8 @@ the lengths had when every twiddle was a table entry of its own.
 The bounds are rel-L2 errors of Gaussian samples measured with that engine
 (the two-buffer lines, four-steps and Bluestein passes these lines replaced),
 plus 2 %: three standard deviations of an error estimated from 2^15 points."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -45,4 +47,36 @@ def test_f32_lines_and_tiles(pkg, dev, few, bounds, monkeypatch):
         err = _error(run_plan(pkg, dev, "dft", [n], x, batch, "f32"), _exact(x, n, "f32"))
         if not err < 1.02 * bound:
             over[n] = (err, bound)
+    assert not over, over
+
+
+def _ragged_over(pkg, dev, prec, bounds):
+    """{n: (error, bound)} of the lengths beyond their bound, all in one batch."""
+    import torch
+    lib = pkg.core()
+    reps = {n: max(3, 32768 // n) for n in bounds}
+    sizes = [n for n in bounds for _ in range(reps[n])]
+    h = ctypes.c_void_p()
+    pkg.check(lib.nfft_ragged_create(ctypes.byref(h), 0 if prec == "f32" else 1, len(sizes),
+                                     (ctypes.c_int * len(sizes))(*sizes), 0), "ragged_create")
+    x = {n: _samples(n, reps[n], prec) for n in bounds}
+    xd = torch.from_numpy(np.concatenate([x[n] for n in bounds])).to(dev)
+    yd = torch.empty_like(xd)
+    pkg.check(lib.nfft_ragged_execute(h, 0, xd.data_ptr(), yd.data_ptr(), None), "ragged_execute")
+    pkg.check(lib.nfft_ragged_check(h, None), "ragged_check")
+    y = yd.cpu().numpy()
+    lib.nfft_ragged_destroy(h)
+    over, off = {}, 0
+    for n, bound in bounds.items():
+        err = _error(y[off:off + x[n].size], _exact(x[n], n, prec))
+        off += x[n].size
+        if not err < 1.02 * bound:
+            over[n] = (err, bound)
+    return over
+
+
+def test_f32_ragged_lines(pkg, dev):
+    bounds = {84: 8.96e-8, 300: 1.036e-7, 1000: 1.184e-7, 1134: 1.280e-7, 1620: 1.261e-7, 3136: 1.204e-7,
+              3584: 1.217e-7, 13720: 1.355e-7, 14000: 1.341e-7, 15360: 1.314e-7, 20160: 1.403e-7}
+    over = _ragged_over(pkg, dev, "f32", bounds)
     assert not over, over
