@@ -80,3 +80,12 @@ def test_f32_ragged_lines(pkg, dev):
               3584: 1.217e-7, 13720: 1.355e-7, 14000: 1.341e-7, 15360: 1.314e-7, 20160: 1.403e-7}
     over = _ragged_over(pkg, dev, "f32", bounds)
     assert not over, over
+
+
+@pytest.mark.parametrize("prec,bounds", [
+    ("f32", {41: 1.358e-7, 67: 1.406e-7, 139: 1.653e-7, 577: 1.812e-7, 1051: 1.780e-7, 1103: 1.808e-7}),
+    ("f64", {41: 3.52e-16, 67: 3.64e-16, 139: 3.86e-16, 577: 4.29e-16, 1051: 4.28e-16, 1103: 4.37e-16})])
+def test_ragged_bluestein(pkg, dev, prec, bounds):
+    """Lengths just above a power of two: M is about 4 n as a power of two."""
+    over = _ragged_over(pkg, dev, prec, bounds)
+    assert not over, over
