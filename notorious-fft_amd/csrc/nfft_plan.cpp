@@ -1634,7 +1634,7 @@ bool nfft_plan::init(int kind_, int prec_, int d_, const int *dims_, long long b
         const long long Pl = P / last;  // leading product
         ax.resize(d - 1);
         for (int i = 0; i + 1 < d; i++) {
-            if (!ax[i].init(dims[i], prec)) return false;
+            if (!ax[i].init(dims[i], prec, 2, 2, batch * Pl * H / dims[i])) return false;
             dsc += " | " + ax[i].describe();
         }
         const long long lines = batch * Pl;

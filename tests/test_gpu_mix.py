@@ -109,3 +109,21 @@ def test_axes(pkg, dev, prec, dims):
         got = run_plan(pkg, dev, op, dims, x, 2, prec)
         err = ol.rel_l2(got, pocket(op, dims, x, 2))
         assert err < tol, (prec, dims, op, err)
+
+
+@pytest.mark.parametrize("prec,dims,batch", [("f32", [10007, 4], 1), ("f32", [10007, 4], 40), ("f64", [5003, 16], 2),
+                                             ("f32", [1200, 8], 3), ("f64", [15000, 8], 1)])
+def test_small_realdft_leading_axes(pkg, dev, prec, dims, batch):
+    """The leading axes of a realdft are planned for the lines they have."""
+    n, h = dims[0], dims[1] // 2 + 1
+    plan, axis = pkg.Plan("realdft", prec, dims, batch), pkg.Plan("dft", prec, [n], batch * h)
+    desc, want = plan.describe(), axis.describe()
+    plan.close()
+    axis.close()
+    assert desc.endswith("| " + want), (desc, want)
+    tol = 2 * 4 * EPS[prec] * math.sqrt(math.log2(n * dims[1]))
+    x = rounded(ol.uniform(46, n * dims[1] * batch), prec)
+    y = pocket("realdft", dims, x, batch)
+    assert ol.rel_l2(run_plan(pkg, dev, "realdft", dims, x, batch, prec), y) < tol
+    y = rounded(y, prec)
+    assert ol.rel_l2(run_plan(pkg, dev, "invrealdft", dims, y, batch, prec), pocket("invrealdft", dims, y, batch)) < tol
