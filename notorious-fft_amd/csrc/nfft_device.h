@@ -583,20 +583,14 @@ __device__ __forceinline__ long long xcd_logical(long long lin, long long total)
     return x * q + (x < r ? x : r) + k;
 }
 
-// Order of column tiles.  FP32: runs of 32 neighbouring tiles to an XCD in
-// turn, so that the eight XCDs work within one window of every row they
-// stride over instead of eight far apart: pages and channels are shared, lines
-// still meet in one L2.  What is left over is cut into eight.  2^19 x 256 827
-// -> 782 us, 2^18 x 512 817 -> 796, 2048^2 x 16 436 -> 426, DCT 1024^2 x 16
-// there and back 155 -> 150, weighted power 2048^2 x 16 772 -> 741, 512^3 1247
-// -> 1243, 2^21 x 64 894 -> 896.  Runs of 8 / 128: 2^19 796 / 837 us, 2048^2
-// 440 / 469.  FP64, with 128-byte rows of half as many columns, gains nothing
-// (2^20 x 64 844 -> 850 us).
-template <typename T> __device__ __forceinline__ long long xcd_columns(long long lin, long long total)
+// Order of column tiles (col_order, nfft_internal.h): the workgroups' own, an
+// eighth to each XCD, or runs of 32 to an XCD in turn and what is left in eighths.
+enum TileOrder { ORDER_PLAIN = 0, ORDER_EIGHTHS = 1, ORDER_RUNS = 2 };
+__device__ __forceinline__ long long xcd_order(long long lin, long long total, int order)
 {
+    if (order == ORDER_PLAIN) return lin;
     constexpr int run = 32;
-    if constexpr (sizeof(T) != 4) return xcd_logical(lin, total);
-    const long long whole = total / (8 * run) * (8 * run);
+    const long long whole = order == ORDER_RUNS ? total / (8 * run) * (8 * run) : 0;
     if (lin >= whole) return whole + xcd_logical(lin - whole, total - whole);
     const long long w = lin % (8 * run);
     return lin - w + (w & 7) * run + (w >> 3);

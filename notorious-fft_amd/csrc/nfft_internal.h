@@ -52,6 +52,24 @@ inline int col_max(int /*prec*/) { return 4096; }
 inline int rowT_max(int prec) { return prec == F32 ? 2048 : 1024; }
 inline int bluerow_max(int prec) { return prec == F32 ? 4096 : 2048; }
 
+// Order of the column tiles of a pass over `points` complex points.
+// ORDER_EIGHTHS: an eighth of the tiles to each XCD, so that tiles that share
+// 128-byte lines meet in one L2, and arrays that the eight L2s hold together
+// are read back by the XCD that wrote them.  ORDER_RUNS, larger FP32 arrays:
+// runs of 32 neighbouring tiles to an XCD in turn, so that the eight XCDs work
+// within one window of every row they stride over: pages and channels are
+// shared.  us, eighths / runs: FP32 2^19 x 256 827 / 782, 2^18 x 512 817 / 796,
+// 2048^2 x 16 436 / 426, weighted power 2048^2 x 16 772 / 741, 2^21 x 64 894 /
+// 896; 32 MiB: 2^16 x 64 30.2 / 30.7, 2^18 x 16 32.8 / 31.1; 16 MiB: 2^16 x 32
+// 21.6 / 28.0, 2^17 x 16 21.7 / 28.1, 2^18 x 8 22.6 / 28.4.  Runs of 8 / 128: 2^19 796
+// / 837, 2048^2 440 / 469.  FP64, with 128-byte rows of half as many columns,
+// gains nothing from them (2^20 x 64 844 -> 850).
+constexpr long long kL2Bytes = 32LL << 20;
+inline int col_order(int prec, long long points)
+{
+    return prec == 0 && points * 8 >= kL2Bytes ? ORDER_RUNS : ORDER_EIGHTHS;
+}
+
 // Columns per workgroup of k_col / rows of k_rowT, k_blue_row: powers of two,
 // 128-byte global segments where the LDS budget allows, >= 256 threads.
 template <typename T, int L> __host__ __device__ constexpr int col_lpb()
@@ -147,6 +165,7 @@ struct WpowArgs {
     long long ntrans;          // batch
     const void *tw;            // FP64 stage table of L
     int form;                  // kernel (col_wpow_tiles)
+    int order;                 // TileOrder (col_order)
 };
 bool col_wpow_supported(int prec, int L);
 // workgroups per transform, and the kernel a batch of this many takes

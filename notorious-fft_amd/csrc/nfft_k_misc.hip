@@ -40,8 +40,10 @@ hipError_t launch_blue_line(int prec, int M, const BlueArgs &a, hipStream_t s)
     NFFT_TIMED("k_blue_line", M, 2.0 * a.nlines * a.n * cxb(prec),
                prec == F32 ? blue_line_impl<float>(M, a, s) : blue_line_impl<double>(M, a, s));
 }
-hipError_t launch_col(int prec, int L, int dir, int mode, const ColArgs &a, hipStream_t s)
+hipError_t launch_col(int prec, int L, int dir, int mode, const ColArgs &a0, hipStream_t s)
 {
+    ColArgs a = a0;
+    a.order = col_order(prec, a.ntrans * a.ncols * L);
     static const char *names[4] = {"k_col_plain", "k_col_twiddle", "k_col_blue_in", "k_col_blue_out"};
     const double tile = (double)a.ntrans * a.ncols * L * cxb(prec);
     const double nvb = (double)a.ntrans * a.nv * cxb(prec);

@@ -35,6 +35,7 @@ template <typename T> hipError_t col_wpow_impl(int L, WpowArgs &a, hipStream_t s
                 a.form = LL >= 512 ? col_form<T, LL>(COL_PLAIN, c) : 0;                                       \
             }                                                                                                 \
             const int w = a.form == 2 ? 2 * lpb : lpb;                                                        \
+            a.order = col_order(sizeof(T) == 4 ? F32 : F64, a.ntrans * a.dist);                               \
             const unsigned gx = (unsigned)((a.ncols + w - 1) / w);                                            \
             *per = gx;                                                                                        \
             if (!launch) return hipSuccess;                                                                   \

@@ -338,6 +338,7 @@ struct ColArgs {
     double scale;
     int lpb;                   // columns per workgroup (0: default for L)
     int four;                  // first pass of a four-step
+    int order;                 // TileOrder (col_order)
 };
 
 template <int L, int LPB> __host__ __device__ constexpr int col_threads() { return Sched<L>::NT * LPB; }
@@ -378,7 +379,7 @@ k_col(ColArgs a)
     if constexpr (TWL) stage_tw_to_lds<T, L>(ltw, (const double2 *)a.tw);
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
     const long long lin = blockIdx.x + (long long)gridDim.x * (blockIdx.y + (long long)gridDim.y * blockIdx.z);
-    const long long lg = xcd_columns<T>(lin, (long long)gridDim.x * gridDim.y * gridDim.z);
+    const long long lg = xcd_order(lin, (long long)gridDim.x * gridDim.y * gridDim.z, a.order);
     const int c0 = (int)(lg % gridDim.x) * LPB, c = c0 + b;
     const long long t = lg / gridDim.x;
     const bool valid = c < a.ncols && t < a.ntrans;
@@ -478,7 +479,7 @@ __global__ void __launch_bounds__((Sched<L>::NT / 2 * LPB), (col_h_wpe<T, L, LPB
     __shared__ C ltw[S::TWN];
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
     const long long lin = blockIdx.x + (long long)gridDim.x * (blockIdx.y + (long long)gridDim.y * blockIdx.z);
-    const long long lg = xcd_columns<T>(lin, (long long)gridDim.x * gridDim.y * gridDim.z);
+    const long long lg = xcd_order(lin, (long long)gridDim.x * gridDim.y * gridDim.z, a.order);
     const int c0 = (int)(lg % gridDim.x) * LPB, c = c0 + b;
     const long long t = lg / gridDim.x;
     const bool valid = c < a.ncols && t < a.ntrans;

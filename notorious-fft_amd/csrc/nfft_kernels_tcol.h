@@ -35,6 +35,7 @@ struct TrigColArgs {
     const void *t2;        // type 4: e^{-i pi (2n+1)/(4N)}
     double scale;
     double w0;             // weight of the DC term
+    int order;             // TileOrder (col_order)
 };
 
 // Column `c0 + b` of all arrays as a buffer view at the tile's first array
@@ -66,7 +67,7 @@ k_t23_col(TrigColArgs a)
     using C = Cx<T>;
     __shared__ C lds[N * LPB];
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
-    const TrigCol<C> col(a, xcd_columns<T>(blockIdx.x, gridDim.x) * LPB, b);
+    const TrigCol<C> col(a, xcd_order(blockIdx.x, gridDim.x, a.order) * LPB, b);
     const C *w = (const C *)a.t1;
     const T sc = (T)a.scale;
     const LayCol<LPB> lay{b};
@@ -128,7 +129,7 @@ k_t4_col(TrigColArgs a)
     using C = Cx<T>;
     __shared__ C lds[N * LPB];
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
-    const TrigCol<C> col(a, xcd_columns<T>(blockIdx.x, gridDim.x) * LPB, b);
+    const TrigCol<C> col(a, xcd_order(blockIdx.x, gridDim.x, a.order) * LPB, b);
     const C *pre = (const C *)a.t1, *post = (const C *)a.t2;
     const T sc = (T)2 * (T)a.scale;
     const LayCol<2 * LPB> lay[2] = {{b}, {b + LPB}};  // real parts, imaginary parts

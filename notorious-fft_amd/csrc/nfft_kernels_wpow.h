@@ -47,10 +47,10 @@ __global__ void __launch_bounds__((wpow_threads<L, LPB>())) k_col_wpow(WpowArgs 
     __shared__ double red[NTH / 64];
     if constexpr (S::S > 1) stage_tw_to_lds<T, L>(ltw, (const double2 *)a.tw);
     const int b = threadIdx.x % LPB, j = threadIdx.x / LPB;
-    // neighbouring tiles on one XCD: 2048-point columns fit 8 FP32 columns, half
-    // a 128-byte line, whose other half the next tile reads and writes
-    const long long tile = xcd_columns<T>(blockIdx.x + (long long)gridDim.x * blockIdx.y,
-                                       (long long)gridDim.x * gridDim.y);  // (transform, column tile)
+    // neighbouring tiles on one XCD where they share lines: 2048-point columns fit 8
+    // FP32 columns, half a 128-byte line, whose other half the next tile reads and writes
+    const long long tile = xcd_order(blockIdx.x + (long long)gridDim.x * blockIdx.y,
+                                     (long long)gridDim.x * gridDim.y, a.order);  // (transform, column tile)
     const long long t = tile / gridDim.x;
     const int c0 = (int)(tile % gridDim.x) * LPB, c = c0 + b;
     const bool valid = c < a.ncols;
@@ -108,8 +108,8 @@ __global__ void __launch_bounds__((Sched<L>::NT / 2 * LPB), (col_h_wpe<T, L, LPB
     __shared__ double red[NTH / 64];
     const int b = threadIdx.x % LPB;
     int j = threadIdx.x / LPB;
-    const long long tile = xcd_columns<T>(blockIdx.x + (long long)gridDim.x * blockIdx.y,
-                                          (long long)gridDim.x * gridDim.y);
+    const long long tile = xcd_order(blockIdx.x + (long long)gridDim.x * blockIdx.y,
+                                     (long long)gridDim.x * gridDim.y, a.order);
     const long long t = tile / gridDim.x;
     const int c0 = (int)(tile % gridDim.x) * LPB, c = c0 + b;
     const bool valid = c < a.ncols;

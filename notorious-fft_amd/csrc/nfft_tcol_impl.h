@@ -25,8 +25,10 @@ hipError_t tcol_go(int op, const TrigColArgs &a, long long grid, hipStream_t s)
 }
 
 // query: only whether a kernel takes these arguments
-template <typename T> hipError_t tcol_impl(int N, int op, const TrigColArgs &a, hipStream_t s, bool query)
+template <typename T> hipError_t tcol_impl(int N, int op, const TrigColArgs &a0, hipStream_t s, bool query)
 {
+    TrigColArgs a = a0;
+    a.order = col_order(sizeof(T) == 4 ? F32 : F64, a.total * N);
     switch (N) {
 #define NFFT_CASE(LL)                                                                                           \
     case LL:                                                                                                    \

@@ -78,3 +78,26 @@ def test_narrow_columns(pkg, dev, prec, op, dims, batch):
     want = ol.run_oracle(op, dims, x, batch) if op[:2] in ("dc", "ds") else pocket(op, dims, x, batch)
     err = ol.rel_l2(run_plan(pkg, dev, op, dims, x, batch, prec), want)
     assert err < tol_for(prec, p), err
+
+
+@pytest.mark.parametrize("prec,dims,batch", [("f32", [64, 64], 3), ("f32", [64, 64], 1025), ("f32", [2048, 64], 5),
+                                             ("f32", [256, 33], 3), ("f64", [64, 64], 7), ("f64", [32, 512], 4),
+                                             ("f64", [128, 24], 9)])
+def test_weighted_power_tile_orders(pkg, dev, prec, dims, batch, monkeypatch):
+    """Tiles in each order: arrays that the L2s hold, of tiles that are whole
+    lines and that are not, and larger ones."""
+    p = int(np.prod(dims))
+    x = rounded(ol.uniform(75, 2 * p * batch), prec)
+    w = rounded(gauss_mask(dims), prec)
+    lref, gref = np_ref(x, w, dims, batch)
+    loss, grad = run_wpow(pkg, dev, prec, dims, batch, x, w, monkeypatch)
+    assert np.max(np.abs(loss - lref) / lref) < tol_for(prec, p)
+    assert ol.rel_l2(grad, gref) < tol_for(prec, p)
+
+
+@pytest.mark.parametrize("n,batch", [(1 << 16, 63), (1 << 16, 64), (1 << 17, 33), (1 << 18, 7)])
+def test_four_step_tile_orders(pkg, dev, n, batch):
+    """FP32 batches that the L2s hold, and the smallest larger one."""
+    x = rounded(ol.uniform(76, 2 * n * batch), "f32")
+    err = ol.rel_l2(run_plan(pkg, dev, "dft", [n], x, batch, "f32"), pocket("dft", [n], x, batch))
+    assert err < tol_for("f32", n), err
