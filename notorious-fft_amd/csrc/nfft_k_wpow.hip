@@ -18,6 +18,24 @@ template <typename T, int L, int LPB> void wpow_h_go(unsigned gx, const WpowArgs
     hipLaunchKernelGGL((k_col_wpow_h<T, L, LPB>), dim3(gx, (unsigned)a.ntrans), dim3(Sched<L>::NT / 2 * LPB), 0, s, a);
 }
 
+// The order of other column passes; but tiles that share no 128-byte line keep
+// the workgroups' own order, the row passes' too, in arrays below the 256 MiB of
+// the memory-side cache: what fits one workgroup of either is then on one XCD
+// throughout, and no XCD starts far from the part written last (us, workgroups'
+// order / eighths: FP32 64^2 x 256 23.1 / 30.5, 256 x 64 x 128 36.4 / 44.3, 512 x 32 x
+// 128 40.0 / 46.6, 1024^2 x 2 42.3 / 46.3; FP64 64^2 x 128 24.3 / 31.8, 512 x 32 x 64 37.0 /
+// 38.8, 256^2 x 200 203 / 221; 400 MiB of it 500 / 470).  Not FP64 columns of up to 64
+// points in several tiles, whose rows are runs of 1 KiB and more (32 x 512 x 64
+// 36.4 / 32.1, 64 x 256 x 64 33.7 / 30.3).
+template <typename T> int wpow_order(int L, int w, const WpowArgs &a)
+{
+    constexpr long long cb = (long long)sizeof(Cx<T>);
+    const bool lines = w * cb % 128 == 0 && a.ncols * cb % 128 == 0;
+    const bool wide = cb == 16 && L <= 64 && a.ncols > w;
+    if (lines && !wide && a.ntrans * a.dist * cb < 8 * kL2Bytes) return ORDER_PLAIN;
+    return col_order(sizeof(T) == 4 ? F32 : F64, a.ntrans * a.dist);
+}
+
 // launch == false: only the form that the whole batch takes and its workgroups
 // per transform
 template <typename T> hipError_t col_wpow_impl(int L, WpowArgs &a, hipStream_t s, long long *per, bool launch)
@@ -35,7 +53,7 @@ template <typename T> hipError_t col_wpow_impl(int L, WpowArgs &a, hipStream_t s
                 a.form = LL >= 512 ? col_form<T, LL>(COL_PLAIN, c) : 0;                                       \
             }                                                                                                 \
             const int w = a.form == 2 ? 2 * lpb : lpb;                                                        \
-            a.order = col_order(sizeof(T) == 4 ? F32 : F64, a.ntrans * a.dist);                               \
+            a.order = wpow_order<T>(LL, w, a);                                                                \
             const unsigned gx = (unsigned)((a.ncols + w - 1) / w);                                            \
             *per = gx;                                                                                        \
             if (!launch) return hipSuccess;                                                                   \
