@@ -15,8 +15,9 @@ extern template __global__ void k_mix_line<float, false, double2>(MixArgs);
 extern template __global__ void k_mix_line<float, true, float2>(MixArgs);
 extern template __global__ void k_mix_line<double, false, double2>(MixArgs);
 extern template __global__ void k_mix_line<double, true, double2>(MixArgs);
-extern template __global__ void k_mix_tile<float>(MixTileArgs);
-extern template __global__ void k_mix_tile<double>(MixTileArgs);
+extern template __global__ void k_mix_tile<float, false>(MixTileArgs);
+extern template __global__ void k_mix_tile<float, true>(MixTileArgs);
+extern template __global__ void k_mix_tile<double, false>(MixTileArgs);
 
 namespace {
 
@@ -450,10 +451,10 @@ TileStatus tile_plan(TileFits &fits, long long n, bool blue, TilePlan *p)
     return TILE_OK;
 }
 
-template <typename T> static hipError_t mix_tile_go(const MixTileArgs &a, hipStream_t s)
+template <typename T, bool ONCE> static hipError_t mix_tile_go(const MixTileArgs &a, hipStream_t s)
 {
-    static const bool attr = [] {  // once per precision and process
-        (void)hipFuncSetAttribute((const void *)k_mix_tile<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMixLds);
+    static const bool attr = [] {  // once per instantiation and process
+        (void)hipFuncSetAttribute((const void *)k_mix_tile<T, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMixLds);
         (void)hipGetLastError();
         return true;
     }();
@@ -466,14 +467,15 @@ template <typename T> static hipError_t mix_tile_go(const MixTileArgs &a, hipStr
     if ((pl.blue && !a.ph.H) || ((a.ph.flags & (MIX_CHIRP_IN | MIX_CHIRP_OUT)) && !a.ph.chirp)) return hipErrorInvalidValue;
     for (int i = 0; i < pl.steps; i++)  // every butterfly has its place in a thread
         if (pl.G * pl.st[i].nb > pl.nth * mix_reps(pl.st[i].radix)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_mix_tile<T>, dim3((unsigned)grid), dim3(pl.nth), lds, s, a);
+    hipLaunchKernelGGL((k_mix_tile<T, ONCE>), dim3((unsigned)grid), dim3(pl.nth), lds, s, a);
     return hipGetLastError();
 }
 
 hipError_t launch_mix_tile(int prec, const MixTileArgs &a, hipStream_t s)
 {
     const int slot = prof_on() ? prof_begin(s) : -1;
-    const hipError_t e = prec == F32 ? mix_tile_go<float>(a, s) : mix_tile_go<double>(a, s);
+    const hipError_t e = prec == F64 ? mix_tile_go<double, false>(a, s)
+                         : a.blue ? mix_tile_go<float, false>(a, s) : mix_tile_go<float, true>(a, s);
     if (slot >= 0)
         prof_end(slot, s, "k_mix_tile", prec, a.ph.pl.L,
                  2.0 * (double)a.ntrans * a.ph.lines * a.ph.pl.L * (prec == F32 ? 8.0 : 16.0));

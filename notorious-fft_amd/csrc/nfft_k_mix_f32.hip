@@ -5,5 +5,6 @@ namespace nfft {
 template __global__ void k_mix_line<float, false, double2>(MixArgs);
 template __global__ void k_mix_line<float, false, float2>(MixArgs);
 template __global__ void k_mix_line<float, true, float2>(MixArgs);
-template __global__ void k_mix_tile<float>(MixTileArgs);
+template __global__ void k_mix_tile<float, false>(MixTileArgs);
+template __global__ void k_mix_tile<float, true>(MixTileArgs);
 }  // namespace nfft

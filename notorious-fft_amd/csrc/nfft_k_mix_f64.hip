@@ -4,5 +4,5 @@
 namespace nfft {
 template __global__ void k_mix_line<double, false, double2>(MixArgs);
 template __global__ void k_mix_line<double, true, double2>(MixArgs);
-template __global__ void k_mix_tile<double>(MixTileArgs);
+template __global__ void k_mix_tile<double, false>(MixTileArgs);
 }  // namespace nfft

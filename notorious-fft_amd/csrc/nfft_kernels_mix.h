@@ -67,18 +67,20 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t mix_rsrc(const void *base, uin
 
 // w^t, t < R, applied to v: entry e of the table is e^{-2 pi i e / L}, w the
 // entry `e`.  Powers t = Q h + l as products of the entries of l and Q h.
-// W: type of the table entries.  FP32 transforms with FP64 entries (mix_plan
-// says which lines have them, tiles always do) read those of w and w^Q alone,
-// form the powers and apply them in FP64 and round once: with the powers
-// rounded and applied in FP32 lengths were up to 5 % further off than with a
-// table entry and four passes (N = 20000 1.42e-7 -> 1.49e-7; now 1.43e-7; N =
-// 288 1.039e-7 -> 1.075e-7; now 1.030e-7), and the loads cost as much as the
-// FP64 products (2^26 points: N = 20000 394 -> 359 us, 12000 375 -> 344, 288
-// 202 -> 211, 480 202 -> 216, tiles of 10^6 636 -> 664).
-template <typename W, int R, typename C>
+// W: type of the table entries.
+// ONCE, FP32 transforms with FP64 entries (mix_plan says which lines have
+// them, tiles do): the entries of w and w^Q alone, powers formed and
+// applied in FP64 and rounded once.  With the powers rounded and applied in
+// FP32 lengths were up to 5 % further off than with a table entry and four
+// passes (N = 20000 1.42e-7 -> 1.49e-7; now 1.43e-7; N = 288 1.039e-7 ->
+// 1.075e-7; now 1.030e-7), and the loads cost as much as the FP64 products
+// (2^26 points: N = 20000 394 -> 359 us, 12000 375 -> 344, 288 202 -> 211, 480
+// 202 -> 216, tiles of 10^6 636 -> 664).  Not the tiles of Bluestein, whose
+// error is the convolution's (N = 33333 1533 -> 1632).
+template <typename W, int R, bool ONCE, typename C>
 __device__ __forceinline__ void mix_twiddle(C (&v)[R], __amdgpu_buffer_rsrc_t tw, int e)
 {
-    constexpr bool wide = sizeof(W) > sizeof(C);
+    static_assert(!ONCE || sizeof(W) > sizeof(C), "FP32 transform, FP64 entries");
     constexpr int Q = R <= 5 ? R : R <= 9 ? 3 : R <= 16 ? 4 : R <= 25 ? 5 : 6;
     constexpr int NH = (R - 1) / Q;
     const uint32_t eb = (uint32_t)e * (uint32_t)sizeof(W);
@@ -88,18 +90,18 @@ __device__ __forceinline__ void mix_twiddle(C (&v)[R], __amdgpu_buffer_rsrc_t tw
     };
     W lo[Q], hi[NH + 1];
 #pragma unroll
-    for (int l = 1; l < Q; l++) lo[l] = wide && l > 1 ? product(lo[l / 2], lo[l - l / 2]) : buf_ld<W>(tw, eb * (uint32_t)l, 0);
+    for (int l = 1; l < Q; l++) lo[l] = ONCE && l > 1 ? product(lo[l / 2], lo[l - l / 2]) : buf_ld<W>(tw, eb * (uint32_t)l, 0);
 #pragma unroll
-    for (int h = 1; h <= NH; h++) hi[h] = wide && h > 1 ? product(hi[h / 2], hi[h - h / 2]) : buf_ld<W>(tw, eb * (uint32_t)(Q * h), 0);
+    for (int h = 1; h <= NH; h++) hi[h] = ONCE && h > 1 ? product(hi[h / 2], hi[h - h / 2]) : buf_ld<W>(tw, eb * (uint32_t)(Q * h), 0);
 #pragma unroll
     for (int t = 1; t < R; t++) {
         const int h = t / Q, l = t % Q;
         const W w = h == 0 ? lo[l] : l == 0 ? hi[h] : product(hi[h], lo[l]);
-        if constexpr (wide) {
+        if constexpr (ONCE) {
             const double2 z = dmul(make_double2(v[t].x, v[t].y), w);
             v[t] = cmk<C>((float)z.x, (float)z.y);
         } else {
-            v[t] = cmul(v[t], w);
+            v[t] = cmul(v[t], cmk<C>((decltype(C::x))w.x, (decltype(C::x))w.y));
         }
     }
 }
@@ -146,7 +148,7 @@ __device__ __forceinline__ void mix_step(const PL &pl, int s, Cx<T> *lds, __amdg
                 const C *p = lds + (__mul24(g, pl.lp) + __mul24(jq, up) + k);
 #pragma unroll
                 for (int t = 0; t < R; t++) v[i][t] = p[t * rs];
-                mix_twiddle<typename IO::W, R>(v[i], tw, __mul24(k, st.q));
+                mix_twiddle<typename IO::W, R, IO::kOnce>(v[i], tw, __mul24(k, st.q));
             }
             dft_any<R, -1>(v[i]);
             if constexpr (BLUE) {
@@ -203,6 +205,7 @@ __device__ __forceinline__ void mix_lines(const PL &pl, Cx<T> *lds, const void *
 template <typename T, bool BLUE, class OFFS, class TW = Cx<T>> struct MixIoLine {
     using C = Cx<T>;
     using W = TW;  // twiddle table entries
+    static constexpr bool kOnce = sizeof(W) > sizeof(C);
     __amdgpu_buffer_rsrc_t in, out, chirp, H;  // in, out, chirp end with their last point
     OFFS offs;
     int glast;  // last line of this workgroup
@@ -361,10 +364,12 @@ __device__ __forceinline__ void mix_tw2(C (&v)[R], const Tw2 &tab, uint32_t e0, 
     }
 }
 
-// PH: MixPhase, as a kernel argument or in constant memory
-template <typename T, class PH> struct MixIoTile {
+// PH: MixPhase, as a kernel argument or in constant memory.  ONCE: as
+// mix_twiddle's.
+template <typename T, class PH, bool ONCE> struct MixIoTile {
     using C = Cx<T>;
     using W = double2;  // twiddle table entries
+    static constexpr bool kOnce = ONCE;
     const PH &ph;
     __amdgpu_buffer_rsrc_t in, out, chirp, H;  // in / out / H at line c0 (chirped sides: at the transform)
     int c0, glast;
@@ -427,13 +432,13 @@ template <typename T, class PH> struct MixIoTile {
 
 // Lines [c0, c0 + cnt) of phase `ph` of one transform (cnt <= ph.pl.G); src
 // and dst at the transform (or its scratch).
-template <typename T, class PH>
+template <typename T, bool ONCE, class PH>
 __device__ __forceinline__ void mix_tile(const PH &ph, const Cx<T> *src, Cx<T> *dst, int c0, int cnt, int inverse,
                                          T scale, Cx<T> *lds)
 {
     using C = Cx<T>;
     const uint32_t nb = (uint32_t)ph.nv * (uint32_t)sizeof(C);
-    const MixIoTile<T, PH> io{ph,
+    const MixIoTile<T, PH, ONCE> io{ph,
                     ph.flags & MIX_CHIRP_IN ? mix_rsrc(src, nb) : buf_rsrc(src + (long long)c0 * ph.ig),
                     ph.flags & MIX_CHIRP_OUT ? mix_rsrc(dst, nb) : buf_rsrc(dst + (long long)c0 * ph.og),
                     mix_rsrc(ph.chirp, nb),
@@ -461,7 +466,7 @@ struct MixTileArgs {
     void *out;
     long long in_dist, out_dist;  // elements between transforms on either side
     long long ntrans;
-    int inverse;
+    int inverse, blue;            // blue: a phase of Bluestein
     double scale;
     MixPhase ph;
 };
@@ -470,14 +475,14 @@ struct MixTileArgs {
 // up to 10; Bluestein over the next power of two) and now: FP32 N = 20736 1134
 // -> 472 us, 196608 1225 -> 480, 10^6 1589 (Bluestein) -> 667, 33333 2496 ->
 // 1584; FP64 20736 1810 -> 839, 196608 1969 -> 923, 33331 4441 -> 3697.
-template <typename T> __global__ void __launch_bounds__(mix_threads<T>()) k_mix_tile(MixTileArgs a)
+template <typename T, bool ONCE> __global__ void __launch_bounds__(mix_threads<T>()) k_mix_tile(MixTileArgs a)
 {
     using C = Cx<T>;
     extern __shared__ char smem[];
     const int G = a.ph.pl.G, tiles = (a.ph.lines + G - 1) / G;
     const long long i = mix_item(blockIdx.x, a.ntrans * tiles), t = i / tiles;
     const int c0 = (int)(i - t * tiles) * G;
-    mix_tile<T>(a.ph, (const C *)a.in + t * a.in_dist, (C *)a.out + t * a.out_dist, c0, min(G, a.ph.lines - c0),
+    mix_tile<T, ONCE>(a.ph, (const C *)a.in + t * a.in_dist, (C *)a.out + t * a.out_dist, c0, min(G, a.ph.lines - c0),
                 a.inverse, (T)a.scale, (C *)smem);
 }
 
@@ -550,7 +555,7 @@ template <typename T> __global__ void __launch_bounds__(kTileThreads, (sizeof(T)
         const int i = (int)mix_item(b, a.nitems);
         RagItemK &it = ((RagItemK *)a.items)[i];
         MixPhaseK &ph = ((MixPhaseK *)a.phases)[it.phase];
-        mix_tile<T>(ph, (const C *)a.in + it.src, (C *)(it.in_place ? a.alt : a.out) + it.dst, it.c0, it.cnt, a.inverse, rag_scale<T>(a, it),
+        mix_tile<T, sizeof(T) == 4>(ph, (const C *)a.in + it.src, (C *)(it.in_place ? a.alt : a.out) + it.dst, it.c0, it.cnt, a.inverse, rag_scale<T>(a, it),
                     (C *)smem);
         __syncthreads();  // the next tile overwrites the buffer
     }

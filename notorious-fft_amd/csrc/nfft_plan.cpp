@@ -983,6 +983,7 @@ hipError_t C2C::run(const void *in, void *out, long long nlines, long long in_di
                 a.out_dist = tail ? out_dist : tiles->elems;
                 a.ntrans = cnt;
                 a.inverse = dir > 0 ? 1 : 0;
+                a.blue = tiles->phases == 3 ? 1 : 0;
                 a.scale = scale;
                 a.ph = tiles->ph[p];
                 const hipError_t e = launch_mix_tile(prec, a, s);
