@@ -789,17 +789,27 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode, long long l
     // / 1784; FP64 5209 1.52 3404 / 3411, 12007 1.33 3206 / 3512, 20011 1.60
     // 3732 / 3505, 35023 1.83 4296 / 3624, 90001 1.42 3594 / 3956; beyond
     // 2^17 points the power of two: FP32 500009 1518 / 2107).
+    // They begin where the power of two's passes over M points per line no
+    // longer find their intermediate in the 256 MiB memory-side cache (us, FP32,
+    // power of two / tiles at 128 and 224 MiB of it: N = 12007 138 / 157 and 297 /
+    // 262, 16381 155 / 193 and 321 / 333, 20011 114 / 132 and 240 / 227, 24001 118 / 151 and
+    // 254 / 255, 50021 149 / 153 and 309 / 256), from 64 MiB on where M is that much
+    // shorter (17011 1.90: 90 / 86 at 96 MiB, 35023 1.83: 112 / 87, 40009 1.60: 114 /
+    // 97); FP64 beyond 512 MiB (20011 x 80 82 / 99, 40009 x 40 87 / 100).
+    auto tiles_from = [&](double ratio) {  // points of all lines
+        if (prec == F64) return 32LL << 20;
+        if (ratio >= 1.75 || (m >= (1 << 17) && ratio >= 1.5)) return 8LL << 20;
+        return ratio >= 1.25 && m != (1 << 16) ? 18LL << 20 : 28LL << 20;
+    };
     bool tileblue = false;
-    // (small batches as above: FP32 20011 x 1 15 / 27 us, x 80 48 / 51, 40009 x 40 55 /
-    // 48; FP64 20011 x 20 34 / 47, x 80 82 / 99, 40009 x 40 87 / 100)
-    if (!mixblue && m > line_max(prec) && n < (1 << 17) && (lines == 0 || lines * m > (prec == F32 ? 8LL << 20 : 32LL << 20))) {
+    if (!mixblue && m > line_max(prec) && n < (1 << 17) && (lines == 0 || lines * m > tiles_from(2.0))) {
         TileFits small{prec, 16 * kTileThreads, kTileThreads, {}};
         tiles = std::make_shared<TilePlan>();
         const TileStatus st = tile_plan(small, n, true, tiles.get());
         if (st == TILE_FAILED) return false;
-        const long long mt = (long long)tiles->n1 * tiles->n2;
+        const double ratio = st == TILE_OK ? (double)m / ((double)tiles->n1 * tiles->n2) : 0.0;
         const double least = prec == F64 ? 1.6 : m <= (1 << 15) ? 1.0 : 1.2;
-        tileblue = st == TILE_OK && m >= least * mt;
+        tileblue = st == TILE_OK && ratio >= least && (lines == 0 || lines * m > tiles_from(ratio));
         if (!tileblue) tiles.reset();
     }
     if (tileblue) {

@@ -127,3 +127,18 @@ def test_small_realdft_leading_axes(pkg, dev, prec, dims, batch):
     assert ol.rel_l2(run_plan(pkg, dev, "realdft", dims, x, batch, prec), y) < tol
     y = rounded(y, prec)
     assert ol.rel_l2(run_plan(pkg, dev, "invrealdft", dims, y, batch, prec), pocket("invrealdft", dims, y, batch)) < tol
+
+
+@pytest.mark.parametrize("n,batch,tiles", [(16381, 896, False), (16381, 897, True), (12007, 576, False),
+                                           (12007, 577, True), (24001, 448, False), (24001, 449, True),
+                                           (17011, 128, False), (17011, 129, True), (40009, 65, True)])
+def test_small_bluestein_tiles_begin(pkg, dev, n, batch, tiles):
+    """FP32 batches on either side of the size where tiles replace the power
+    of two's three passes."""
+    plan = pkg.Plan("dft", "f32", [n], batch)
+    desc = plan.describe()
+    plan.close()
+    assert ("in tiles" in desc) == tiles, desc
+    x = rounded(ol.uniform(47, 2 * n * batch), "f32")
+    err = ol.rel_l2(run_plan(pkg, dev, "dft", [n], x, batch, "f32"), pocket("dft", [n], x, batch))
+    assert err < 2 * 4 * EPS["f32"] * math.sqrt(math.log2(n)), (desc, err)
