@@ -1581,10 +1581,23 @@ static double axis_inv_scale(int norm, int n)
     return is_pow2(n) ? 1.0 : 1.0 / n;  // reference behaviour
 }
 
+// A few long columns keep fewer CUs busy than the row pass between two
+// transposes (us, transposes / strided): type 4 of 4096 points, two halves of
+// 2048 per tile (FP32 8 columns 16.9 / 20.4, 32 21.7 / 25.0, 96 25.0 / 26.3, FP64 4 17.1 /
+// 19.1, 32 25.6 / 27.6), and columns that are an array's only ones or nearly so, so
+// that a tile covers several arrays (4096 x 2 x 16: DCT-2 FP32 16.5 / 24.6, DCT-4 15.5 /
+// 26.5; DCT-4 2048 x 2 x 16 FP32 14.6 / 16.8, FP64 16.3 / 18.2).
+static bool trig_few(int prec, int t4, int n, long long cols, long long B)
+{
+    if (t4 && n == 4096 && cols <= (prec == F32 ? 96 : 40)) return true;
+    if (B > 4 || cols * (B / 2) > 32 || cols < 2) return false;
+    return t4 ? B == 2 && n == 2048 : prec == F32 && n == 4096;
+}
+
 // The strided form of a trig axis of n points over rows of B reals in `outer`
 // arrays: every length that has a column kernel (up to 4096 points).  Longer
-// axes and arrays beyond 32-bit offsets are transposed (dist stays 0).  False
-// if a table cannot be made.
+// axes, arrays beyond 32-bit offsets and a few long columns are transposed
+// (dist stays 0).  False if a table cannot be made.
 static bool trig_col(TrigColArgs &c, int prec, int t4, int n, long long outer, long long B)
 {
     TrigColArgs a{};
@@ -1592,6 +1605,7 @@ static bool trig_col(TrigColArgs &c, int prec, int t4, int n, long long outer, l
     a.total = outer * a.ncols;
     a.dist = (long long)n * a.ncols;
     a.scale = a.w0 = 1.0;
+    if (trig_few(prec, t4, n, a.total, B)) return true;
     if ((prec == F32 ? tcol_impl<float>(n, 0, a, nullptr, true) : tcol_impl<double>(n, 0, a, nullptr, true)) != hipSuccess)
         return true;
     a.tw = stage_table(prec, t4 ? n / 2 : n);

@@ -45,3 +45,22 @@ def test_strided_trig_adjoint(pkg, dev, dims, op):
     v = run_plan(pkg, dev, op, dims, g, 1, "f64", vjp=True)
     scale = np.linalg.norm(g) * np.linalg.norm(fx)
     assert abs(np.dot(v, x) - np.dot(g, fx)) < 64 * EPS["f64"] * scale
+
+
+@pytest.mark.parametrize("prec,kind,dims,batch,few", [
+    ("f32", "t4", [4096, 64], 3, True), ("f32", "t4", [4096, 256], 1, False), ("f64", "t4", [4096, 64], 1, True),
+    ("f64", "t4", [4096, 128], 1, False), ("f32", "t4", [2048, 2], 32, True), ("f64", "t4", [2048, 2], 33, False),
+    ("f32", "t2t3", [4096, 2], 32, True), ("f32", "t2t3", [4096, 2], 33, False), ("f32", "t2t3", [4096, 4], 8, True),
+    ("f32", "t2t3", [4096, 4], 9, False), ("f64", "t2t3", [4096, 2], 3, False)])
+def test_few_long_columns(pkg, dev, prec, kind, dims, batch, few):
+    """A few long columns are transposed (through the plan's workspace), one
+    more is not."""
+    plan = pkg.Plan(kind, prec, dims, batch)
+    transposed = plan.workspace_bytes > 0
+    plan.close()
+    assert transposed == few
+    p = int(np.prod(dims))
+    x = rounded(ol.uniform(64, p * batch), prec)
+    for op in ("dct4", "dst4") if kind == "t4" else ("dct2", "dst3"):
+        err = ol.rel_l2(run_plan(pkg, dev, op, dims, x, batch, prec), ol.run_oracle(op, dims, x, batch))
+        assert err < 8 * EPS[prec] * math.sqrt(math.log2(p)), (op, err)
