@@ -128,15 +128,17 @@ double cost_of(const MixPlan &p, int prec, double conflict)
 
 // Time of one workgroup that has its CU to itself, in issue slots: the rounds
 // of its busiest SIMD, and per stage a trip through LDS, a table load and a
-// barrier.
-double latency_of(const MixPlan &p, int prec)
+// barrier.  The same in both precisions, whose instructions issue at one rate
+// (weighing FP64's half as much again took smaller radices: mean over 24
+// lengths from 480 to 196608 points, up to 40 lines, 4 % longer).
+double latency_of(const MixPlan &p)
 {
     double c = 0;
     for (int s = 0; s < p.steps; s++) {
         const int total = p.G * p.st[s].nb, R = p.st[s].radix, reps = (total + p.nth - 1) / p.nth;
         const int waves = (std::min(p.nth, total) + 63) / 64;
         const bool mid = p.blue && s == p.stages - 1;
-        c += reps * ((waves + 3) / 4) * (R * (dft_ops(R) * (mid ? 2 : 1) + 16) * (prec == 0 ? 1.0 : 1.5) + 50) + 350;
+        c += reps * ((waves + 3) / 4) * (R * (dft_ops(R) * (mid ? 2 : 1) + 16) + 50) + 350;
     }
     return c;
 }
@@ -175,7 +177,7 @@ struct Search {
                 if (!ok) continue;
                 if (nth > shape.nth_min && nth - 64 >= most) break;  // only idle waves beyond
                 p.nth = nth;
-                const double c = shape.few ? latency_of(p, prec) : cost_of(p, prec, conflict);
+                const double c = shape.few ? latency_of(p) : cost_of(p, prec, conflict);
                 if (c < best) {
                     best = c;
                     plan = p;
@@ -360,9 +362,10 @@ const TileFit &TileFits::get(int L, MixLanes lanes, bool blue)
         TileFit f;
         f.ok = mix_fit(prec, L, blue, sh, &f.plan, &f.cost);
         // a point read and written takes half an issue slot of its CU's share
-        // of the memory bandwidth, more where a tile covers part of a segment
-        if (f.ok && !few)
-            f.cost += 0.5 * (prec == F32 ? 1 : 2) * L *
+        // of the memory bandwidth (few workgroups: a whole tile's in FP64), more
+        // where a tile covers part of a segment
+        if (f.ok && !(few && prec == F32))
+            f.cost += 0.5 * (prec == F32 ? 1 : 2) * L * (few ? f.plan.G : 1) *
                       (lanes == MIX_LANES_POINTS ? 1.0 : std::max(1.0, (double)seg() / f.plan.G));
         if (f.ok && (!best.ok || f.cost < best.cost)) best = f;
         return f.ok;

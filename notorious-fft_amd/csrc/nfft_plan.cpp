@@ -734,16 +734,23 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode, long long l
         // (NFFT_SMOOTH=2: tiles before lines from 2048 / 1024 points on), else
         // two phases of tiles; lengths with no split for them use Bluestein.
         const bool line = mix_plan(prec, n, lines, &mx);
-        // small batches: two or four times the tiles (us, two / four: FP64 N = 20000 x 5
-        // 15.0 / 14.1, 30000 x 8 15.6 / 17.0, FP32 50000 x 5 13.5 / 14.8), also where a line
-        // would fill its workgroup ( FP32 N = 15000 x 17 11.8 against 14.1, 50000 x 5 14.7 / 17.4,
-        // 30000 x 30 26.5 / 18.7; FP64 15000 x 40 28.9 / 21.4)
-        const bool few = lines > 0 && lines * n <= 5 << 16;
+        // Small batches: tiles of a half or a quarter of the points, and of the
+        // schedule that ends first, also where a line would fill its workgroup (us,
+        // full / half / quarter: FP64 N = 24000 x 5 18.5 / 14.0 / 13.9, x 17 21.2 / 17.0 /
+        // 17.2, x 21 22.4 / 17.6 / 26.7, 100000 x 5 21.9 / 25.1; FP32 30000 x 7 15.6 / 13.3 /
+        // 13.0, x 23 17.9 / 17.7 / 17.5, x 50 24.3 / 28.9; line / half / quarter: FP32 20480 x
+        // 3 22.6 / 11.6 / 11.1, x 34 26.1 / 14.5 / 14.9, 15000 x 33 14.0 / 13.8 / 13.7, x 47 14.3 /
+        // 15.3; FP64 10240 x 6 16.6 / 12.9 / 12.6, 10000 x 6 12.6 / 13.2 / 12.8).
+        const long long points = lines * n;
+        const bool few = lines > 0 && points <= (prec == F64   ? (n > 65536 ? 13 << 15 : 1 << 19)
+                                                 : n > 15000 ? 3 << 18
+                                                             : 1 << 19);
         if (few) {
-            fits.points /= n > 24000 ? 2 : 4;
+            fits.points /= points <= 5 << 16 && (prec == F64 || n <= 24000) ? 4 : 2;
             fits.few = true;
         }
-        const bool tiles_first = !line || (few && n > 12000) || (smooth_env == 2 && n > (prec == F32 ? 2048 : 1024));
+        const bool tiles_first = !line || (few && n > (prec == F64 ? 10000 : 12000)) ||
+                                 (smooth_env == 2 && n > (prec == F32 ? 2048 : 1024));
         int use = smooth_mode == 1 ? 1 : tuned_choice(prec, n);
         if (use < 0 && env_int("NFFT_TUNE", 0)) use = tune_smooth(n, prec);
         if (use != 0 && tiles_first) {

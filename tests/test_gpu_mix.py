@@ -142,3 +142,20 @@ def test_small_bluestein_tiles_begin(pkg, dev, n, batch, tiles):
     x = rounded(ol.uniform(47, 2 * n * batch), "f32")
     err = ol.rel_l2(run_plan(pkg, dev, "dft", [n], x, batch, "f32"), pocket("dft", [n], x, batch))
     assert err < 2 * 4 * EPS["f32"] * math.sqrt(math.log2(n)), (desc, err)
+
+
+@pytest.mark.parametrize("prec,n,batch,tiles", [
+    ("f64", 10240, 51, True), ("f64", 10240, 52, False), ("f64", 10000, 3, False), ("f64", 24000, 13, True),
+    ("f64", 24000, 22, True), ("f64", 100000, 5, True), ("f32", 20480, 38, True), ("f32", 20480, 39, False),
+    ("f32", 15000, 34, True), ("f32", 15000, 35, False), ("f32", 30000, 26, True), ("f32", 30000, 27, True)])
+def test_small_batches_of_tiles(pkg, dev, prec, n, batch, tiles):
+    """Tiles of a quarter, a half and all of the points, and lines, on either
+    side of the batches where they change."""
+    plan = pkg.Plan("dft", prec, [n], batch)
+    desc = plan.describe()
+    plan.close()
+    assert desc.startswith("mixed-radix four-step") == tiles, desc
+    x = rounded(ol.uniform(48, 2 * n * batch), prec)
+    for op in ("dft", "invdft"):
+        err = ol.rel_l2(run_plan(pkg, dev, op, [n], x, batch, prec), pocket(op, [n], x, batch))
+        assert err < 4 * EPS[prec] * math.sqrt(math.log2(n)), (op, err, desc)
