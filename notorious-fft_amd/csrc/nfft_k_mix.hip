@@ -320,10 +320,17 @@ template <typename T, bool BLUE, class TW> static hipError_t mix_go(const MixArg
     // lines of a workgroup are addressed by 32-bit byte offsets
     const long long far = std::max(a.in_dist, a.out_dist);
     if ((far * (a.pl.G - 1) + a.pl.L) * (long long)sizeof(Cx<T>) >= (1LL << 32)) a.pl.G = 1;
+    a.flat = !BLUE && a.pl.steps == 1 && a.in_dist == a.pl.L && a.out_dist == a.pl.L;
+    if (a.flat && a.nlines * a.pl.L >= 1 << 21) {
+        // 2048 points on 256 threads where that makes 1024 workgroups (2^24 points in us,
+        // 1024 / 2048 / 4096: FP64 N = 3 115 / 98 / 103, 30 151 / 97 / 104, FP32 7 46 / 42 / 44)
+        a.pl.G = 2048 / a.pl.L;
+        a.pl.nth = 256;
+    }
     const long long grid = (a.nlines + a.pl.G - 1) / a.pl.G;
-    const size_t lds = (size_t)a.pl.G * a.pl.lp * sizeof(Cx<T>);
+    const size_t lds = (size_t)a.pl.G * (a.flat ? a.pl.L | 1 : a.pl.lp) * sizeof(Cx<T>);
     if (grid > 0x7fffffffLL || lds > kMixLds || a.pl.nth < 64 || a.pl.nth > mix_threads<T>()) return hipErrorInvalidValue;
-    for (int i = 0; i < a.pl.steps; i++)  // every butterfly has its place in a thread
+    for (int i = 0; i < a.pl.steps && !a.flat; i++)  // every butterfly has its place in a thread
         if (a.pl.G * a.pl.st[i].nb > a.pl.nth * mix_reps(a.pl.st[i].radix)) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_mix_line<T, BLUE, TW>), dim3((unsigned)grid), dim3(a.pl.nth), lds, s, a);
     return hipGetLastError();

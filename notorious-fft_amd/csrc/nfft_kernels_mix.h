@@ -284,7 +284,43 @@ struct MixArgs {
     double scale;
     int n;                    // Bluestein: transform length
     const void *chirp, *H;    // Bluestein: n chirp entries, L filter entries (scaled 1 / L)
+    int flat = 0;             // mix_flat
 };
+
+// Lines of one butterfly, next to each other on both sides: copied through LDS
+// in their order in memory, a line per thread in between.  Loaded straight, the
+// lanes' lines lie R points apart (2^24 points, straight / copied in us: FP32 N = 7
+// 71.5 / 42, 30 100 / 44, FP64 3 150 / 98, 30 153 / 98).
+template <int R> __host__ __device__ constexpr int mix_flat_pitch() { return R % 2 ? R : R + 1; }
+template <typename T, int R>
+__device__ __forceinline__ void mix_flat(__amdgpu_buffer_rsrc_t in, __amdgpu_buffer_rsrc_t out, int cnt, T sg, T sc, Cx<T> *lds)
+{
+    using C = Cx<T>;
+    constexpr int P = mix_flat_pitch<R>();
+    const int total = cnt * R;
+    auto at = [](int i) { return i / R * (P - R) + i; };
+    for (int i0 = threadIdx.x; i0 < total; i0 += 8 * blockDim.x) {
+        C x[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) x[k] = buf_ld<C>(in, (uint32_t)(i0 + k * blockDim.x) * (uint32_t)sizeof(C), 0);
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            if (i0 + k * (int)blockDim.x < total) lds[at(i0 + k * blockDim.x)] = x[k];
+    }
+    __syncthreads();
+    for (int g = threadIdx.x; g < cnt; g += blockDim.x) {
+        C v[R];
+#pragma unroll
+        for (int t = 0; t < R; t++) v[t] = lds[g * P + t];
+#pragma unroll
+        for (int t = 0; t < R; t++) v[t].y *= sg;
+        dft_any<R, -1>(v);
+#pragma unroll
+        for (int t = 0; t < R; t++) lds[g * P + t] = cmk<C>(v[t].x * sc, v[t].y * (sc * sg));
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < total; i += blockDim.x) buf_st<C>(out, (uint32_t)i * (uint32_t)sizeof(C), 0, lds[at(i)]);
+}
 
 // Bound: one read and one write of the lines where a CU keeps two workgroups
 // (up to 10240 FP32 / 5120 FP64 points by LDS, 16 waves at 128 VGPRs); beyond,
@@ -311,6 +347,16 @@ template <typename T, bool BLUE, class TW> __global__ void __launch_bounds__(mix
                                          a.n,
                                          a.inverse ? (T)-1 : (T)1,
                                          (T)a.scale};
+    if constexpr (!BLUE) {
+        if (a.flat) {
+            switch (a.pl.L) {
+#define NFFT_MIX_CASE(R) case R: mix_flat<T, R>(io.in, io.out, cnt, io.sg, io.sc, (C *)smem); break;
+                NFFT_MIX_RADICES(NFFT_MIX_CASE)
+#undef NFFT_MIX_CASE
+            }
+            return;
+        }
+    }
     mix_lines<T, BLUE>(a.pl, (C *)smem, a.tw, io);
 }
 

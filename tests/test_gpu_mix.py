@@ -159,3 +159,15 @@ def test_small_batches_of_tiles(pkg, dev, prec, n, batch, tiles):
     for op in ("dft", "invdft"):
         err = ol.rel_l2(run_plan(pkg, dev, op, [n], x, batch, prec), pocket(op, [n], x, batch))
         assert err < 4 * EPS[prec] * math.sqrt(math.log2(n)), (op, err, desc)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("n", [3, 5, 7, 9, 12, 15, 21, 28, 30])
+def test_small_lines_of_one_butterfly(pkg, dev, prec, n):
+    """Copied through LDS: one line, a partial last group, and the batch from
+    which the groups are larger; in place and both directions."""
+    for batch in (1, 300, (1 << 21) // n + 1):
+        x = rounded(ol.uniform(49, 2 * n * batch), prec)
+        for op, inplace in (("dft", True), ("invdft", False)):
+            err = ol.rel_l2(run_plan(pkg, dev, op, [n], x, batch, prec, inplace=inplace), pocket(op, [n], x, batch))
+            assert err < 4 * EPS[prec] * math.sqrt(math.log2(n)), (batch, op, err)
