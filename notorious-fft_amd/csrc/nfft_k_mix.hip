@@ -264,10 +264,19 @@ bool mix_plan(int prec, long long n, long long lines, MixPlan *p)
     MixShape sh = line_shape((int)n);
     // Small batches end with their longest workgroup: few lines in each, radices
     // around 10 (us, large batches' schedule / this / two LDS buffers: FP32 N = 1200
-    // x 40 9.6 / 6.2 / 8.7, 10^4 x 20 13 / 11 / 16; FP64 720 x 40 10.2 / 6.2 / 6.5,
-    // 2000 x 60 11.2 / 7.1 / 12.5).
-    if (lines > 0 && lines * n <= (n > 512 ? 1 << 19 : 1 << 20)) {  // (FP64 1000 x 1000 11.2 / 14.3)
-        sh.g_min = sh.g_max = (int)std::min<long long>(sh.g_max, (lines + 1023) / 1024);
+    // x 40 9.6 / 6.2 / 8.7, 10^4 x 20 13 / 11 / 16; FP64 720 x 40 10.2 / 6.2 / 6.5, 2000 x
+    // 60 11.2 / 7.1 / 12.5, 720 x 729 11.2 / 8.0 / 9.1, 1000 x 1049 10.9 / 12.4 / 12.7, 480 x
+    // 3277 12.6 / 11.3 / 18.3).  The kernels' registers leave room for four
+    // workgroups a CU in FP32, two in FP64.  FP64 lines of up to 128 points gain
+    // from it in larger batches, in groups of about 4096 points (100 x 31458 26.5 /
+    // 22.5 / 24.7, x 83887 58.2 / 49.2 / 55.3; 360 x 11651 26.7 / 28.8 / 39.4).
+    const long long points = lines * n, most = prec == F32 ? (n > 512 ? 1 << 19 : 1 << 20) : (n > 512 ? 9 << 16 : 5 << 19);
+    const int groups = prec == F32 ? 1024 : 512;
+    if (lines > 0 && points <= most) {
+        sh.g_min = sh.g_max = (int)std::min<long long>(sh.g_max, (lines + groups - 1) / groups);
+        sh.few = true;
+    } else if (lines > 0 && prec == F64 && n > 32 && n <= 128 && points <= 9 << 20) {
+        sh.g_min = sh.g_max = (int)(4096 / n);
         sh.few = true;
     }
     if (n < 2 || !mix_fit(prec, n, false, sh, p)) return false;

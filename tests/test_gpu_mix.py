@@ -171,3 +171,14 @@ def test_small_lines_of_one_butterfly(pkg, dev, prec, n):
         for op, inplace in (("dft", True), ("invdft", False)):
             err = ol.rel_l2(run_plan(pkg, dev, op, [n], x, batch, prec, inplace=inplace), pocket(op, [n], x, batch))
             assert err < 4 * EPS[prec] * math.sqrt(math.log2(n)), (batch, op, err)
+
+
+@pytest.mark.parametrize("prec,n,batch", [("f64", 720, 819), ("f64", 720, 820), ("f64", 480, 5461), ("f64", 480, 5462),
+                                          ("f64", 100, 26215), ("f64", 100, 94371), ("f64", 100, 94372),
+                                          ("f32", 480, 2185)])
+def test_small_middling_batches(pkg, dev, prec, n, batch):
+    """On either side of the sizes where the schedules of small batches end."""
+    x = rounded(ol.uniform(50, 2 * n * batch), prec)
+    for op in ("dft", "invdft"):
+        err = ol.rel_l2(run_plan(pkg, dev, op, [n], x, batch, prec), pocket(op, [n], x, batch))
+        assert err < 4 * EPS[prec] * math.sqrt(math.log2(n)), (op, err)
