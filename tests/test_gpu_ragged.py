@@ -165,3 +165,16 @@ def test_ragged_rejects_oversize(pkg):
     assert lib.nfft_ragged_create(ctypes.byref(h), 0, 2, arr, 0) == pkg.E_UNSUPPORTED
     arr = (ctypes.c_int * 1)(0)
     assert lib.nfft_ragged_create(ctypes.byref(h), 0, 1, arr, 0) == pkg.E_SIZE
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("extra", [0, 1])
+def test_ragged_small_batch(pkg, dev, prec, extra):
+    """2^19 points, the largest batch whose short transforms take a small
+    batch's schedules, and one more."""
+    sizes = [2, 3, 7, 16, 30, 97, 100, 360, 509, 1000, 1021, 2048, 4093, 4096, 6000, 8192] * 18
+    rest = (1 << 19) + extra - sum(sizes)
+    assert rest > 0
+    sizes += [min(64, rest - at) for at in range(0, rest, 64)]
+    assert sum(sizes) == (1 << 19) + extra
+    check_vs_pocketfft(pkg, dev, prec, sizes)
