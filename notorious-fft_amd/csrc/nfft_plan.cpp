@@ -279,9 +279,17 @@ static int env_int(const char *name, int dflt)
 // ---------------------------------------------------------------------------
 // mixed radix vs Bluestein for 7-smooth lengths
 // ---------------------------------------------------------------------------
+// Record "c2c-smooth p<prec> n<N> <0|1> mix l<lines>": the choice between
+// Bluestein and the one-pass lines and tiles, for a small batch of so many
+// lines or for large ones (l0).  Lines of another form are not read: those
+// without the two fields chose against an engine that is gone.
 static std::string smooth_key(int prec, long long n)
 {
     return "c2c-smooth p" + std::to_string(prec) + " n" + std::to_string(n);
+}
+static std::string smooth_tag(long long n, long long lines)
+{
+    return "mix l" + std::to_string(lines > 0 && lines * n <= 1 << 20 ? lines : 0);
 }
 
 // Tuning results of this process, by record key (value: the text after the
@@ -307,38 +315,44 @@ static void tune_mem_put(const std::string &key, const std::string &val)
 
 // Choice recorded in the NFFT_TUNE_CACHE file (the last record wins), else
 // measured earlier in this process (-1: none).
-static int tuned_choice(int prec, long long n)
+static int tuned_choice(int prec, long long n, long long lines)
 {
-    const std::string key = smooth_key(prec, n);
+    const std::string key = smooth_key(prec, n), tag = smooth_tag(n, lines);
     int found = -1;
     const char *path = getenv("NFFT_TUNE_CACHE");
     if (path && *path) {
         if (FILE *f = fopen(path, "r")) {
             char line[256];
             while (fgets(line, sizeof line, f)) {
-                if (strncmp(line, key.c_str(), key.size()) == 0 && line[key.size()] == ' ')
-                    found = atoi(line + key.size() + 1);
+                if (strncmp(line, key.c_str(), key.size()) != 0 || line[key.size()] != ' ') continue;
+                const char *val = line + key.size() + 1;
+                const size_t len = strcspn(val, "\r\n");
+                if ((val[0] == '0' || val[0] == '1') && std::string(val + 1, len - 1) == " " + tag) found = val[0] - '0';
             }
             fclose(f);
         }
     }
     std::string mem;
-    if (found < 0 && tune_mem_get(key, &mem)) found = atoi(mem.c_str());
+    if (found < 0 && tune_mem_get(key + " " + tag, &mem)) found = atoi(mem.c_str());
     return found;
 }
 
 // Project-written autotuner: times the mixed-radix plan and the Bluestein
-// plan of length n on a synthetic batch of about 2^22 points and records the
-// faster one (1: mixed radix, 0: Bluestein) in NFFT_TUNE_CACHE.
-static int tune_smooth(int n, int prec)
+// plan of length n on synthetic data, a small batch as it is and a large one
+// of about 2^22 points, and records the faster one (1: mixed radix, 0:
+// Bluestein) in NFFT_TUNE_CACHE.
+static int tune_smooth(int n, int prec, long long batch)
 {
+    const std::string tag = smooth_tag(n, batch);
+    const bool large = tag == smooth_tag(n, 0);
+    if (large) batch = 0;
     C2C cand[2];
-    if (!cand[0].init(n, prec, 0) || !cand[1].init(n, prec, 1)) {
+    if (!cand[0].init(n, prec, 0, 2, batch) || !cand[1].init(n, prec, 1, 2, batch)) {
         cand[0].release();
         cand[1].release();
         return -1;
     }
-    const long long lines = std::max(1LL, (1LL << 22) / n);
+    const long long lines = large ? std::max(1LL, (1LL << 22) / n) : batch;
     const size_t cb = cx_bytes(prec);
     hipStream_t st = setup_stream();
     void *x = nullptr, *y = nullptr, *scr = nullptr;
@@ -367,11 +381,11 @@ static int tune_smooth(int n, int prec)
         return -1;
     }
     const int pick = ms[1] < ms[0] ? 1 : 0;
-    tune_mem_put(smooth_key(prec, n), std::to_string(pick));
+    tune_mem_put(smooth_key(prec, n) + " " + tag, std::to_string(pick));
     const char *path = getenv("NFFT_TUNE_CACHE");
     if (path && *path) {
         if (FILE *f = fopen(path, "a")) {
-            fprintf(f, "%s %d\n", smooth_key(prec, n).c_str(), pick);
+            fprintf(f, "%s %d %s\n", smooth_key(prec, n).c_str(), pick, tag.c_str());
             fclose(f);
         }
     }
@@ -751,8 +765,8 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode, long long l
         }
         const bool tiles_first = !line || (few && n > (prec == F64 ? 10000 : 12000)) ||
                                  (smooth_env == 2 && n > (prec == F32 ? 2048 : 1024));
-        int use = smooth_mode == 1 ? 1 : tuned_choice(prec, n);
-        if (use < 0 && env_int("NFFT_TUNE", 0)) use = tune_smooth(n, prec);
+        int use = smooth_mode == 1 ? 1 : tuned_choice(prec, n, lines);
+        if (use < 0 && env_int("NFFT_TUNE", 0)) use = tune_smooth(n, prec, lines);
         if (use != 0 && tiles_first) {
             tiles = std::make_shared<TilePlan>();
             const TileStatus st = tile_plan(fits, n, false, tiles.get());

@@ -469,6 +469,33 @@ def test_smooth_autotuner(pkg, dev, tmp_path, monkeypatch):
     assert len(cache.read_text().splitlines()) == len(lines)  # no second measurement
 
 
+def test_smooth_records(pkg, dev, tmp_path, monkeypatch):
+    """Records of the choice between mixed radix and Bluestein hold for one
+    batch class each; those of an earlier form are not read."""
+    cache = tmp_path / "tune.txt"
+    monkeypatch.setenv("NFFT_TUNE_CACHE", str(cache))
+
+    def mixed(n, batch):
+        p = pkg.Plan("dft", "f32", [n], batch)
+        desc = p.describe()
+        p.close()
+        return desc.startswith("mixed-radix")
+
+    cache.write_text("c2c-smooth p0 n3000 0\n")
+    assert mixed(3000, 4) and mixed(3000, 5000)
+    cache.write_text("c2c-smooth p0 n3000 0 mix l4\n")
+    assert not mixed(3000, 4) and mixed(3000, 5) and mixed(3000, 5000)
+    cache.write_text("c2c-smooth p0 n3000 1 mix l4\nc2c-smooth p0 n3000 0 mix l0\n")
+    assert mixed(3000, 4) and not mixed(3000, 5000)
+    # measured for each class, once
+    cache.write_text("")
+    monkeypatch.setenv("NFFT_TUNE", "1")
+    for batch in (6, 6, 5000, 7000):
+        mixed(3024, batch)
+    lines = [l.split() for l in cache.read_text().splitlines()]
+    assert [l[:3] + l[4:] for l in lines] == [["c2c-smooth", "p0", "n3024", "mix", c] for c in ("l6", "l0")], lines
+
+
 ROWT_PF_CASES = ([("f32", 16, n2, 26) for n2 in (256, 512, 1024, 2048)] +
                  [("f32", lg, 0, 26) for lg in range(15, 23)] +
                  [("f32", 20, n2, 26) for n2 in (512, 2048)] +
