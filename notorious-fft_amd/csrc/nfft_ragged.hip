@@ -190,13 +190,17 @@ static void ragged_free(nfft_ragged *r)
     delete r;
 }
 
-// Tuning records are keyed by precision and size list.
+// Tuning records are keyed by precision and size list: "ragged p<prec>
+// c<count> h2:<hash> <form>", 1 for a workgroup per tile, 2 to 4 for a resident
+// grid of so many workgroups per CU, and "ragged-gl ... <points per thread of a
+// tile x 100 + quarters of the scratch budget>".  Those of the persistent
+// kernel, whose numbers meant other things, have h and not h2: in their keys.
 static std::string tune_key(int prec, const std::vector<int> &sizes)
 {
     unsigned long long h = 1469598103934665603ULL;
     for (int v : sizes) h = (h ^ (unsigned long long)v) * 1099511628211ULL;
     char b[96];
-    snprintf(b, sizeof b, "ragged p%d c%zu h%016llx", prec, sizes.size(), h);
+    snprintf(b, sizeof b, "ragged p%d c%zu h2:%016llx", prec, sizes.size(), h);
     return b;
 }
 
@@ -515,11 +519,11 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
     const std::string key = tune_key(prec, std::vector<int>(sizes, sizes + count));
-    // a record or the autotuner makes the tile launches resident grids of so
-    // many workgroups per CU; otherwise one workgroup per tile
-    int per_cu = tune_lookup(key);
-    const bool recorded = per_cu > 0;
-    r->tile_grid = recorded ? ncu * per_cu : 0;
+    // a workgroup per tile, or, by a record or the autotuner, a resident grid
+    const auto grid_of = [&](int form) { return form > 1 ? ncu * form : 0; };
+    const int record = tune_lookup(key);
+    const bool recorded = record > 0;
+    r->tile_grid = grid_of(record);
     const bool ok = dev_malloc(&r->d_items, items.size() * sizeof(RagItem)) == hipSuccess &&
                     dev_malloc(&r->d_offs, goffs.size() * sizeof(long long)) == hipSuccess &&
                     dev_malloc(&r->d_phases, phases.size() * sizeof(MixPhase)) == hipSuccess &&
@@ -538,10 +542,10 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
             (void)hipEventCreate(&e0);
             (void)hipEventCreate(&e1);
             float best = 1e30f;
-            per_cu = 1;
+            int form = 1;
             // at most what the kernel's register budget keeps resident
-            for (int pc = 1; pc <= (prec == F32 ? 4 : 2); pc++) {
-                r->tile_grid = ncu * pc;
+            for (int pc = 2; pc <= (prec == F32 ? 4 : 2); pc++) {
+                r->tile_grid = grid_of(pc);
                 (void)launch_ragged(r, 0, tin, tout, r->cap);
                 (void)hipEventRecord(e0, r->cap);
                 for (int k = 0; k < 3; k++) (void)launch_ragged(r, 0, tin, tout, r->cap);
@@ -549,12 +553,12 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
                 (void)hipEventSynchronize(e1);
                 float ms = 0;
                 (void)hipEventElapsedTime(&ms, e0, e1);
-                if (ms < best) { best = ms; per_cu = pc; }
+                if (ms < best) { best = ms; form = pc; }
             }
             (void)hipEventDestroy(e0);
             (void)hipEventDestroy(e1);
-            r->tile_grid = ncu * per_cu;
-            tune_store(key, per_cu);
+            r->tile_grid = grid_of(form);
+            tune_store(key, form);
         }
         if (tin) (void)hipFree(tin);
         if (tout) (void)hipFree(tout);

@@ -178,3 +178,19 @@ def test_ragged_small_batch(pkg, dev, prec, extra):
     sizes += [min(64, rest - at) for at in range(0, rest, 64)]
     assert sum(sizes) == (1 << 19) + extra
     check_vs_pocketfft(pkg, dev, prec, sizes)
+
+
+def test_ragged_records_of_the_persistent_kernel(pkg, dev, tmp_path, monkeypatch):
+    """Records of the earlier form (same names and numbers, other meanings) are
+    not read: the batch is measured again."""
+    cache = tmp_path / "tune.txt"
+    monkeypatch.setenv("NFFT_TUNE_CACHE", str(cache))
+    sizes = ragged_sizes(40, seed=6) + [40000]
+    check_vs_pocketfft(pkg, dev, "f32", sizes, flags=1)
+    new = cache.read_text()
+    cache.write_text("".join(" ".join(f[:3] + ["h" + f[3].split(":")[-1].lstrip("h"), "804" if f[0] == "ragged-gl" else "1"]) + "\n"
+                             for f in (l.split() for l in new.splitlines())))
+    old = cache.read_text()
+    check_vs_pocketfft(pkg, dev, "f32", sizes, flags=1)
+    added = cache.read_text()[len(old):]
+    assert [l.split()[:4] for l in added.splitlines()] == [l.split()[:4] for l in new.splitlines()], (old, added)
