@@ -533,33 +533,34 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
                     hipMemcpy(r->d_phases, phases.data(), phases.size() * sizeof(MixPhase), hipMemcpyHostToDevice) == hipSuccess;
     if (!ok) return fail("ragged setup: device allocation or copy failed");
     if ((flags & 1) && !recorded) {
-        // project-written autotuner: time the batch with a few resident grids
-        // on scratch data and keep the fastest
+        // project-written autotuner: time the batch as it is and with a few
+        // resident grids, at most what the kernel's registers keep resident, on
+        // scratch data and keep the fastest (the batch as it is where anything fails)
         void *tin = nullptr, *tout = nullptr;
-        if (dev_malloc(&tin, (size_t)r->total * cb) == hipSuccess && dev_malloc(&tout, (size_t)r->total * cb) == hipSuccess) {
-            (void)launch_fill_uniform(tin, 2 * r->total, 7, 0, prec, r->cap);
-            hipEvent_t e0, e1;
-            (void)hipEventCreate(&e0);
-            (void)hipEventCreate(&e1);
-            float best = 1e30f;
-            int form = 1;
-            // at most what the kernel's register budget keeps resident
-            for (int pc = 2; pc <= (prec == F32 ? 4 : 2); pc++) {
-                r->tile_grid = grid_of(pc);
-                (void)launch_ragged(r, 0, tin, tout, r->cap);
-                (void)hipEventRecord(e0, r->cap);
-                for (int k = 0; k < 3; k++) (void)launch_ragged(r, 0, tin, tout, r->cap);
-                (void)hipEventRecord(e1, r->cap);
-                (void)hipEventSynchronize(e1);
-                float ms = 0;
-                (void)hipEventElapsedTime(&ms, e0, e1);
-                if (ms < best) { best = ms; form = pc; }
+        hipEvent_t e0 = nullptr, e1 = nullptr;
+        bool timed = dev_malloc(&tin, (size_t)r->total * cb) == hipSuccess &&
+                     dev_malloc(&tout, (size_t)r->total * cb) == hipSuccess && hipEventCreate(&e0) == hipSuccess &&
+                     hipEventCreate(&e1) == hipSuccess &&
+                     launch_fill_uniform(tin, 2 * r->total, 7, 0, prec, r->cap) == hipSuccess;
+        float best = 1e30f;
+        int form = 1;
+        for (int f = 1; f <= (prec == F32 ? 4 : 2) && timed; f++) {
+            r->tile_grid = grid_of(f);
+            float ms = 0;
+            timed = launch_ragged(r, 0, tin, tout, r->cap) == NFFT_OK && hipEventRecord(e0, r->cap) == hipSuccess;
+            for (int k = 0; k < 3 && timed; k++) timed = launch_ragged(r, 0, tin, tout, r->cap) == NFFT_OK;
+            timed = timed && hipEventRecord(e1, r->cap) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
+                    hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
+            if (timed && ms < best) {
+                best = ms;
+                form = f;
             }
-            (void)hipEventDestroy(e0);
-            (void)hipEventDestroy(e1);
-            r->tile_grid = grid_of(form);
-            tune_store(key, form);
         }
+        r->tile_grid = grid_of(timed ? form : 1);
+        if (timed) tune_store(key, form);
+        else (void)hipGetLastError();
+        if (e0) (void)hipEventDestroy(e0);
+        if (e1) (void)hipEventDestroy(e1);
         if (tin) (void)hipFree(tin);
         if (tout) (void)hipFree(tout);
     }

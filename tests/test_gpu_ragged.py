@@ -194,3 +194,23 @@ def test_ragged_records_of_the_persistent_kernel(pkg, dev, tmp_path, monkeypatch
     check_vs_pocketfft(pkg, dev, "f32", sizes, flags=1)
     added = cache.read_text()[len(old):]
     assert [l.split()[:4] for l in added.splitlines()] == [l.split()[:4] for l in new.splitlines()], (old, added)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_ragged_recorded_forms(pkg, dev, prec, tmp_path, monkeypatch):
+    """Every form a record can ask for: a workgroup per tile, and resident grids
+    of fewer workgroups than tiles."""
+    cache = tmp_path / "tune.txt"
+    monkeypatch.setenv("NFFT_TUNE_CACHE", str(cache))
+    sizes = [65536, 65521, 40000, 30030, 50000, 60001] * 30
+    check_vs_pocketfft(pkg, dev, prec, sizes[:6], flags=1)  # the records' form
+    cache.write_text("")
+    make_and_destroy(pkg, prec, sizes, 1)
+    rec = [l.split() for l in cache.read_text().splitlines()]
+    for form in range(1, 5 if prec == "f32" else 3):
+        cache.write_text("".join(" ".join(f[:4] + [str(form) if f[0] == "ragged" else f[4]]) + "\n" for f in rec))
+        check_vs_pocketfft(pkg, dev, prec, sizes)
+
+
+def make_and_destroy(pkg, prec, sizes, flags):
+    pkg.core().nfft_ragged_destroy(make(pkg, prec, sizes, flags))
