@@ -1588,11 +1588,13 @@ static long long chunk_lines(long long nlines, long long per_line_elems, size_t 
 }
 
 // Scratch elements a complex engine needs for `lines` transforms: the
-// persistent four-step only ever uses its rotating slots.
+// persistent four-step and the teams only ever use their slots.
 static long long engine_elems(const C2C &e, long long lines, size_t cb)
 {
     if (e.pctr) return std::min(lines, e.pslots) * e.scratch_per_line;
-    return chunk_lines(lines, e.scratch_per_line, cb) * e.scratch_per_line;
+    long long chunk = chunk_lines(lines, e.scratch_per_line, cb);
+    if (e.tctr && lines >= e.tmin) chunk = std::min(chunk, (long long)e.xnq * e.tslots);
+    return chunk * e.scratch_per_line;
 }
 
 static double axis_inv_scale(int norm, int n)

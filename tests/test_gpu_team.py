@@ -94,3 +94,43 @@ def test_team_small_scratch(pkg, dev, monkeypatch):
         plan.check()
         plan.close()
     assert torch.equal(out[0], out[1])
+
+
+def _families(pkg, plan, x, y):
+    """Kernels of one execute, by the library's timer."""
+    import torch
+    pkg.prof_enable(True)
+    plan.execute("dft", x.data_ptr(), y.data_ptr())
+    torch.cuda.synchronize()
+    names = " ".join(pkg.prof_read())
+    pkg.prof_enable(False)
+    return names
+
+
+@pytest.mark.parametrize("n,batch,mb,team", [(1 << 15, 128, 0, True), (1 << 15, 127, 0, False), (1 << 15, 130, 4, False),
+                                             (1 << 17, 32, 0, True), (1 << 17, 31, 0, False), (1 << 17, 40, 8, False)])
+def test_team_path_taken(pkg, dev, n, batch, mb, team, monkeypatch):
+    """The team kernel runs from its smallest batch on and with scratch for its
+    slots (budgets of `mb` MiB), and not otherwise."""
+    import torch
+    if mb:
+        monkeypatch.setenv("NFFT_PERSIST_MB" if n == 1 << 15 else "NFFT_CHUNK_MB", str(mb))
+    plan = _plan(pkg, n, batch, True, monkeypatch)
+    x = torch.empty(2 * n * batch, dtype=torch.float64, device=dev)
+    pkg.fill_uniform(x.data_ptr(), x.numel(), 13, 0, "f64")
+    y = torch.empty_like(x)
+    names = _families(pkg, plan, x, y)
+    plan.check()
+    plan.close()
+    assert ("k_four_team" in names) == team, names
+    ref = ol.run_oracle("dft", [n], x[-2 * n:].cpu().numpy())
+    assert ol.rel_l2(y[-2 * n:].cpu().numpy(), ref) < tol_for("f64", n)
+
+
+def test_team_scratch(pkg, dev, monkeypatch):
+    """A large batch has scratch for the teams' slots (two transforms an XCD),
+    not for the whole batch."""
+    n, batch = 1 << 17, 300
+    plan = _plan(pkg, n, batch, True, monkeypatch)
+    assert plan.workspace_bytes <= 2 * 16 * 16 * n, plan.workspace_bytes
+    plan.close()
