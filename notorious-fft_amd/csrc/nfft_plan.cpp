@@ -594,11 +594,11 @@ static int xcd_setup(C2C &c)
 
 // The team four-step (k_four_team) of the lengths that have a shape for it,
 // beside the length's other path, which runs smaller batches than tmin and
-// the ones with less scratch than its slots.  NFFT_TEAM=0 turns it off.
-// Returns false on an error (error set).
-static bool team_setup(C2C &c)
+// the ones with less scratch than its slots.  NFFT_TEAM=0 turns it off; single
+// transforms (lines 1) never take it.  Returns false on an error (error set).
+static bool team_setup(C2C &c, long long lines)
 {
-    if (env_int("NFFT_TEAM", 1) == 0 || !team_find(c.prec, c.n, &c.tcfg)) return true;
+    if (lines == 1 || env_int("NFFT_TEAM", 1) == 0 || !team_find(c.prec, c.n, &c.tcfg)) return true;
     int dev = 0, ncu = 0, khz = 0;
     if (!hip_ok(hipGetDevice(&dev), "hipGetDevice") ||
         !hip_ok(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "device attribute") ||
@@ -734,7 +734,7 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode, long long l
         // where no other split or path is asked for
         const bool asked = t_four_force.lg2 >= 0 || tuned_four(prec, n).lg2 >= 0 || env_int("NFFT_TUNE", 0) ||
                            getenv("NFFT_FOUR_N2") || getenv("NFFT_PERSIST") || getenv("NFFT_XCD");
-        return persist_mode == 0 || asked || xctr || team_setup(*this);
+        return persist_mode == 0 || asked || xctr || team_setup(*this, lines);
     }
     // 7-smooth lengths: mixed radix (the reference uses Bluestein for every
     // non-power-of-two length; results agree to rounding) where it is the
@@ -878,7 +878,7 @@ bool C2C::init(int n_, int prec_, int smooth_mode, int persist_mode, long long l
     }
     // filter spectrum H = FFT_m(h) / m, computed in FP64 by this engine
     C2C h64;
-    if (!h64.init(m, F64, smooth_m ? 1 : 2)) return false;
+    if (!(smooth_m ? h64.init(m, F64, 1) : h64.init(m, F64, 2, 2, 1))) return false;
     hipStream_t st = setup_stream();
     void *hbuf = nullptr, *Hbuf = nullptr, *sbuf = nullptr;
     bool ok = hip_ok(dev_malloc(&hbuf, (size_t)m * 16), "hipMalloc") &&
