@@ -1,4 +1,4 @@
-"""Ragged batches (one persistent launch replayed from a HIP graph): every
+"""Ragged batches (one HIP graph of a few launches over the whole list): every
 transform against pocketfft (numpy.fft, FP64), the replays against eager
 per-size plans, with the program's own work between replays."""
 import ctypes
@@ -214,3 +214,43 @@ def test_ragged_recorded_forms(pkg, dev, prec, tmp_path, monkeypatch):
 
 def make_and_destroy(pkg, prec, sizes, flags):
     pkg.core().nfft_ragged_destroy(make(pkg, prec, sizes, flags))
+
+
+@pytest.mark.parametrize("prec,sizes", [
+    # 7-smooth lines and tiles, one-pass Bluestein and tiles, a power of two as M and a 7-smooth one
+    ("f32", [20412, 20480, 20736, 10169, 10177, 10193, 2047, 2048, 2053, 4096, 8192]),
+    ("f64", [10206, 10240, 10290, 5101, 5107, 5113, 2039, 2047, 2053, 4096, 8192])])
+def test_ragged_group_limits(pkg, dev, prec, sizes):
+    """The longest lengths that run in one workgroup and the first ones in tiles."""
+    check_vs_pocketfft(pkg, dev, prec, sizes * 3)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_ragged_sequences_in_place(pkg, dev, prec, monkeypatch):
+    """Long transforms in several sequences over one scratch (a budget of 2 MiB
+    under intermediates of more than 8) beside short ones, input overwritten,
+    replayed with other contents."""
+    import torch
+    monkeypatch.setenv("NFFT_RAGGED_MB", "2")
+    sizes = [65521, 16, 40000, 65536, 97, 32771, 30030, 65536, 12289, 1000, 50000] * 4
+    tiles = sum(n for n in sizes if n > 20480)
+    assert tiles * (8 if prec == "f32" else 16) > 4 * (2 << 20)
+    lib = pkg.core()
+    h = make(pkg, prec, sizes)
+    total = sum(sizes)
+    buf = torch.empty(2 * total, dtype=torch.float32 if prec == "f32" else torch.float64, device=dev)
+    for inverse, seed in ((0, 52), (1, 53), (0, 54)):
+        x = rounded(ol.uniform(seed, 2 * total), prec)
+        buf.copy_(torch.from_numpy(x))
+        torch.cuda.synchronize()
+        pkg.check(lib.nfft_ragged_execute(h, inverse, buf.data_ptr(), buf.data_ptr(), None), "ragged_execute")
+        pkg.check(lib.nfft_ragged_check(h, None), "ragged_check")
+        y = buf.cpu().numpy().astype(np.float64)
+        off = 0
+        for n in sizes:
+            z = x[2 * off:2 * (off + n):2] + 1j * x[2 * off + 1:2 * (off + n):2]
+            want = np.fft.ifft(z) * (n if (n & (n - 1)) == 0 else 1) if inverse else np.fft.fft(z)
+            err = ol.rel_l2(y[2 * off:2 * (off + n):2] + 1j * y[2 * off + 1:2 * (off + n):2], want)
+            assert err < tol_for(prec, n), (inverse, n, err)
+            off += n
+    lib.nfft_ragged_destroy(h)
