@@ -342,7 +342,8 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
     // Short transforms of small batches take the schedules that end first, a line or
     // a few to a workgroup (us, persistent kernel before / large batches' schedules /
     // these: FP32 sizes below 1000 x 30 24.5 / 28.7 / 22.5, x 200 26.0 / 30.2 / 23.7, x 400 27.1 /
-    // 30.9 / 23.3, x 2000, 10^6 points in all, 37.0 / 31.5 / 25.2; x 20000 100.7 / 73.5).
+    // 30.9 / 23.3, x 2000, 10^6 points in all, 37.0 / 31.5 / 25.2; x 20000 100.7 / 73.5), but not
+    // Bluestein lines of more than 4096 points (10007 x 1 143 / 37 / 44).
     const bool few = env_int_rg("NFFT_FEW", 1) != 0 && r->total <= 1 << 19;
     std::vector<MixPhase> phases;
     long long h_elems = 0;
@@ -372,11 +373,10 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
             MixShape sh;
             sh.nth_min = sh.nth_max = gc.nth;
             sh.lds_max = gc.lds;
-            sh.few = few;
+            sh.few = few && !(blue && m2 > 4096);
             const int points = 16 * gc.nth;
             sh.g_max = blue ? points : std::max(1, std::min(256, points / n));
             if (few && !blue) sh.g_min = sh.g_max = std::min(sh.g_max, (count + 1023) / 1024);
-            if (few && blue) sh.g_max = std::min(sh.g_max, 4096);
             if (blue && m2 <= 4096) {
                 sh.g_max = std::max(1, points / m2);
                 one = mix_fit(prec, m2, true, sh, &ph.pl);
