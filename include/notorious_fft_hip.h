@@ -140,9 +140,10 @@ int nfft_plan_check(nfft_plan *plan, void *stream);
  * follow the reference's normalisation (1/N for non-power-of-two N only).
  * flags bit 0: autotune on a scratch batch -- first the tile size (points per
  * thread of a tile) and the scratch budget of the long transforms over five
- * candidates, then a resident grid for their tiles (workgroups per CU); the
- * choices are appended to the file named by NFFT_TUNE_CACHE, if set, and read
- * back (not measured again) by later creates with the same size list. */
+ * candidates, then a workgroup per tile against resident grids for the tile
+ * launches; the choices are appended to the file named by NFFT_TUNE_CACHE, if
+ * set, and read back (not measured again) by later creates with the same size
+ * list. */
 int nfft_ragged_create(nfft_ragged **r, int prec, int count, const int *sizes, int flags);
 int nfft_ragged_execute(nfft_ragged *r, int inverse, const void *in, void *out, void *stream);
 int nfft_ragged_destroy(nfft_ragged *r);

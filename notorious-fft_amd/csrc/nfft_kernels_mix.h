@@ -326,9 +326,11 @@ __device__ __forceinline__ void mix_flat(__amdgpu_buffer_rsrc_t in, __amdgpu_buf
 // (up to 10240 FP32 / 5120 FP64 points by LDS, 16 waves at 128 VGPRs); beyond,
 // one workgroup alternates loading, stages and storing.  2^26 points, before
 // (mixed-radix lines with two LDS buffers up to 2048 points, Bluestein or a
-// two-pass four-step) and now: FP32 N = 100 346 -> 213 us (5.0 TB/s), N =
-// 1000 489 -> 261, N = 10^4 800 -> 230 (4.7 TB/s), N = 20000 982 -> 410; FP64
-// N = 100 598 -> 435 us, N = 1000 709 -> 516, N = 10^4 1365 -> 527.
+// two-pass four-step) and now: FP32 N = 100 346 -> 212 us (5.1 TB/s), N =
+// 1000 489 -> 253, N = 10^4 800 -> 222 (4.8 TB/s), N = 20000 982 -> 357; FP64
+// N = 100 598 -> 435 us, N = 1000 709 -> 516, N = 10^4 1365 -> 527.  Counters
+// of FP32 N = 10^4, and of Bluestein lines of 10007 points (15 waves a CU, 54 %
+// vector issue, 69 % of their time waiting): profiles/mixed_radix_pmc.md.
 template <typename T, bool BLUE, class TW> __global__ void __launch_bounds__(mix_threads<T>()) k_mix_line(MixArgs a)
 {
     using C = Cx<T>;
@@ -498,7 +500,8 @@ __device__ __forceinline__ void mix_tile(const PH &ph, const Cx<T> *src, Cx<T> *
 
 // Item of workgroup b: kTileRun neighbouring items go to one XCD (workgroup b
 // runs on XCD b mod 8), since tiles whose edges share 128-byte lines then
-// share an L2 (the ragged batch of nfft_ragged.hip: 1.54 -> 1.42 ms).
+// share an L2 (the ragged batch of nfft_ragged.hip: 1.54 -> 1.42 ms, with
+// its groups after the tiles and FP32 twiddles).
 constexpr int kTileRun = 16;
 __device__ __forceinline__ long long mix_item(long long b, long long nitems)
 {
@@ -519,8 +522,8 @@ struct MixTileArgs {
 // Bound: memory, as the ragged tiles (four workgroups of 4096 points per CU in
 // FP32, two in FP64).  2^26 points, before (two LDS buffers per tile, radices
 // up to 10; Bluestein over the next power of two) and now: FP32 N = 20736 1134
-// -> 472 us, 196608 1225 -> 480, 10^6 1589 (Bluestein) -> 667, 33333 2496 ->
-// 1584; FP64 20736 1810 -> 839, 196608 1969 -> 923, 33331 4441 -> 3697.
+// -> 444 us, 196608 1225 -> 441, 10^6 1589 (Bluestein) -> 676, 33333 2496 ->
+// 1580; FP64 20736 1810 -> 839, 196608 1969 -> 923, 33331 4441 -> 3697.
 template <typename T, bool ONCE> __global__ void __launch_bounds__(mix_threads<T>()) k_mix_tile(MixTileArgs a)
 {
     using C = Cx<T>;

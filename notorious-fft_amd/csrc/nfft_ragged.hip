@@ -7,26 +7,29 @@
 // (nfft_kernels_mix.h) and the whole batch is a handful of launches:
 //   - short transforms, in groups of one size: lines of any 7-smooth length
 //     (powers of two among them) up to 20480 points (FP32) / 10240 (FP64),
-//     and Bluestein lines whose 7-smooth M >= 2N - 1 is as short; one launch
-//     per workgroup size and form;
+//     and Bluestein lines whose M >= 2N - 1 is as short, the power of two up
+//     to 4096 points and 7-smooth beyond; one launch per workgroup size and
+//     form;
 //   - long transforms, in tiles: 7-smooth N = N1 x N2 in two phases (columns,
 //     rows), Bluestein over M = M1 x M2 in three (columns, rows, columns); one
 //     launch per phase over the tiles of all of them, the intermediate of each
 //     in a scratch region of its own.
 // The phases follow each other by the order of the stream: no tile waits for
 // another inside a kernel; the short transforms run beside them on a second
-// branch of the graph (1.42 -> 1.36 ms on the batch below).  Batches whose intermediates exceed the scratch
-// budget (NFFT_RAGGED_MB) run in several such sequences.
+// branch of the graph (1.42 -> 1.36 ms on the batch below, with FP32 twiddles).
+// Batches whose intermediates exceed the scratch budget (NFFT_RAGGED_MB) run in
+// several such sequences.
 //
 // One persistent launch with queued tiles and dependency waits, over the
 // power-of-two lines and two-buffer mixed-radix tiles, took 2.43 ms (FP32) for
 // 10,000 sizes log-uniform in [16, 65536], 40 % of them primes (80.5 M
-// points); this form takes 1.36 ms (FP64 5.0 -> 2.8 ms).  What changed with it: M is 7-smooth instead of
-// the next power of two (2.1 N instead of 2.9 N on average), transforms of up
-// to 20480 points cross memory once, and a tile's stages run in registers.
-// The tile launches are bound by memory (3.9 TB/s over 128-byte segments; with
-// the butterflies left out they take as long), 16 waves per CU: with half of
-// them 1.80 ms, with three quarters 1.46.
+// points); this form takes 1.41 ms (1.35 with FP32 twiddles; FP64 5.0 -> 3.0
+// ms).  What changed with it: M beyond 4096 points is 7-smooth instead of the
+// next power of two, transforms of up to 20480 points cross memory once, and a
+// tile's stages run in registers.
+// The tile launches wait for memory: 16 waves a CU, 70 to 72 % of their time
+// waiting, 3.3 to 3.7 TB/s over 128-byte segments, vector issue 29 to 40 %
+// (profiles/mixed_radix_pmc.md).
 // Inverse transforms follow the reference's normalisation: unnormalised for
 // powers of two, 1/N for other lengths (src/05_algorithms.h:315-333).
 #include <hip/hip_runtime.h>
