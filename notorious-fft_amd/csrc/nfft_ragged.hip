@@ -345,9 +345,10 @@ static int ragged_create_impl(nfft_ragged **out, int prec, int count, const int 
     // Short transforms of small batches take the schedules that end first, a line or
     // a few to a workgroup (us, persistent kernel before / large batches' schedules /
     // these: FP32 sizes below 1000 x 30 24.5 / 28.7 / 22.5, x 200 26.0 / 30.2 / 23.7, x 400 27.1 /
-    // 30.9 / 23.3, x 2000, 10^6 points in all, 37.0 / 31.5 / 25.2; x 20000 100.7 / 73.5), but not
-    // Bluestein lines of more than 4096 points (10007 x 1 143 / 37 / 44).
-    const bool few = env_int_rg("NFFT_FEW", 1) != 0 && r->total <= 1 << 19;
+    // 30.9 / 23.3, x 2000, 0.5 M points in all, 37.0 / 31.5 / 25.2; FP64 x 800, 0.2 M points,
+    // 34.5 / 26.5 by the last two, but x 2000 36.3 / 38.1), but not Bluestein lines of
+    // more than 4096 points (10007 x 1 143 / 37 / 44).
+    const bool few = env_int_rg("NFFT_FEW", 1) != 0 && r->total <= (prec == F32 ? 1 << 19 : 1 << 18);
     std::vector<MixPhase> phases;
     long long h_elems = 0;
     for (auto &kv : by_size) {

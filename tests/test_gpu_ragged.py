@@ -170,13 +170,14 @@ def test_ragged_rejects_oversize(pkg):
 @pytest.mark.parametrize("prec", ["f32", "f64"])
 @pytest.mark.parametrize("extra", [0, 1])
 def test_ragged_small_batch(pkg, dev, prec, extra):
-    """2^19 points, the largest batch whose short transforms take a small
-    batch's schedules, and one more."""
-    sizes = [2, 3, 7, 16, 30, 97, 100, 360, 509, 1000, 1021, 2048, 4093, 4096, 6000, 8192] * 18
-    rest = (1 << 19) + extra - sum(sizes)
+    """2^19 points (FP64 2^18), the largest batch whose short transforms take a
+    small batch's schedules, and one more."""
+    limit, times = (1 << 19, 18) if prec == "f32" else (1 << 18, 8)
+    sizes = [2, 3, 7, 16, 30, 97, 100, 360, 509, 1000, 1021, 2048, 4093, 4096, 6000, 8192] * times
+    rest = limit + extra - sum(sizes)
     assert rest > 0
     sizes += [min(64, rest - at) for at in range(0, rest, 64)]
-    assert sum(sizes) == (1 << 19) + extra
+    assert sum(sizes) == limit + extra
     check_vs_pocketfft(pkg, dev, prec, sizes)
 
 
